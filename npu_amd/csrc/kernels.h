@@ -20,8 +20,18 @@ int gm_launch_dequant_k(int qtype, const void* raw, int64_t n_blocks, float* out
 int gm_launch_transcode_i8(int qtype, const void* raw, int64_t n_blocks, void* out, hipStream_t s);
 int gm_launch_matvec(int qtype, const void* w, int M, int K, const float* x, int n_tok, float* y,
                      hipStream_t s);
-// Dense bf16 matvec (K % 256 == 0, K <= 16384, 16-byte aligned w and x).
+// Dense bf16 product, any number of tokens (K % 32 == 0, K <= 16384, 16-byte
+// aligned w and x).
 int gm_launch_mv_bf16(const uint16_t* w, int M, int K, const float* x, int n_tok, float* y, hipStream_t s);
+// Two or more tokens, with the extras of gm_launch_gemm_bf16.
+int gm_launch_dense(const uint16_t* w, int M, const uint16_t* w2, int M2, int K, const float* x, int T,
+                    const float* add, float* y, float* y2, hipStream_t s);
+// Many tokens (gemm_bf16.hip): y = x W^T (+ add, [T][M]) and, when w2 is given,
+// y2 = x W2^T in the same launch.  K % 32 == 0; w, w2 and x 16-byte aligned.
+// gm_gemm_bf16_takes: whether a call is large enough for it.
+bool gm_gemm_bf16_takes(int rows, int T);
+int gm_launch_gemm_bf16(const uint16_t* w, int M, const uint16_t* w2, int M2, int K, const float* x, int T,
+                        const float* add, float* y, float* y2, hipStream_t s);
 int gm_launch_gateup(int qtype, const void* wg, const void* wu, int FF, int D, const float* x, int n_tok,
                      float* h, hipStream_t s);
 // One token, y = add + W x (add may be NULL); with nx (a MoE block's router,

@@ -22,7 +22,7 @@
 // per A operand add exact bf16 x bf16 products in fp32 and x loses nothing.
 // A block holds 16 RT rows; its WPB waves split K, each issuing NC k-steps'
 // loads at a time, and their tiles are summed in LDS in wave order.
-#include "common.h"
+#include "bf16_split.h"
 #include "kernels.h"
 #include "moe_decode.h"
 
@@ -254,31 +254,10 @@ __global__ void __launch_bounds__(64 * NW) k_mv_bf16(const uint16_t* __restrict_
   }
 }
 
-typedef __bf16 gm_bf16x8 __attribute__((ext_vector_type(8)));
-
-// x = h + m + l over 8 fp32 values -> three bf16x8 planes (exact split, see above).
-__device__ __forceinline__ void split3(const gm_f32x4& xa, const gm_f32x4& xb, gm_u32x4 (&pl)[3]) {
-  const float v[8] = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
-  uint32_t hb[8], mb[8], lb[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    hb[i] = __float_as_uint(v[i]) & 0xffff0000u;
-    const float r = v[i] - __uint_as_float(hb[i]);
-    mb[i] = __float_as_uint(r) & 0xffff0000u;
-    lb[i] = __float_as_uint(r - __uint_as_float(mb[i]));     // low 16 bits are zero
-  }
-#pragma unroll
-  for (int d = 0; d < 4; ++d) {
-    pl[0][d] = __builtin_amdgcn_perm(hb[2 * d + 1], hb[2 * d], 0x07060302u);
-    pl[1][d] = __builtin_amdgcn_perm(mb[2 * d + 1], mb[2 * d], 0x07060302u);
-    pl[2][d] = __builtin_amdgcn_perm(lb[2 * d + 1], lb[2 * d], 0x07060302u);
-  }
-}
-
 template <int RT, int WPB, int NC>
 __global__ void __launch_bounds__(64 * WPB) k_mv_bf16_mfma(const uint16_t* __restrict__ w, int M, int K,
                                                         const float* __restrict__ x, int n_tok,
-                                                        float* __restrict__ y) {
+                                                        const float* __restrict__ add, float* __restrict__ y) {
   __shared__ gm_f32x4 red[WPB > 1 ? WPB - 1 : 1][RT][64];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l16 = lane & 15, q = lane >> 4;
   const int row0 = blockIdx.x * 16 * RT;
@@ -336,16 +315,17 @@ __global__ void __launch_bounds__(64 * WPB) k_mv_bf16_mfma(const uint16_t* __res
     const int row = row0 + rt * 16 + 4 * q;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      if (row + i < M) out[row + i] = acc[rt][i];
+      if (row + i < M) out[row + i] = add ? add[(int64_t)tok * M + row + i] + acc[rt][i] : acc[rt][i];
   }
 }
 
 template <int RT, int WPB>
-int launch_mfma_w(const uint16_t* w, int M, int K, const float* x, int n_tok, float* y, hipStream_t s) {
+int launch_mfma_w(const uint16_t* w, int M, int K, const float* x, int n_tok, const float* add, float* y,
+                  hipStream_t s) {
   const dim3 grid((unsigned)((M + 16 * RT - 1) / (16 * RT)), (unsigned)((n_tok + 15) / 16));
   const int steps = K / (32 * WPB);                              // k-steps per wave (exact: WPB divides K / 32)
 #define GM_MV_GO(NC)                                                                               \
-  hipLaunchKernelGGL((k_mv_bf16_mfma<RT, WPB, NC>), grid, dim3(64 * WPB), 0, s, w, M, K, x, n_tok, y); \
+  hipLaunchKernelGGL((k_mv_bf16_mfma<RT, WPB, NC>), grid, dim3(64 * WPB), 0, s, w, M, K, x, n_tok, add, y); \
   break;
   switch (steps % 8 == 0 ? 8 : steps % 4 == 0 ? 4 : steps % 2 == 0 ? 2 : 1) {
     case 8: GM_MV_GO(8)
@@ -362,17 +342,18 @@ int launch_mfma_w(const uint16_t* w, int M, int K, const float* x, int n_tok, fl
 // the grid holds about 1024 waves, each wave taking an equal number of 32-wide
 // k-steps: the largest of 8 (4 for grids of >= 256 blocks), 4, 2, 1 that divides
 // K / 32 (K = 576: 2 waves of 9 steps).
-int launch_mfma(const uint16_t* w, int M, int K, const float* x, int n_tok, float* y, hipStream_t s) {
+int launch_mfma(const uint16_t* w, int M, int K, const float* x, int n_tok, const float* add, float* y,
+                hipStream_t s) {
   const int rt = M >= 8192 ? 2 : 1;
   const int blocks = (M + 16 * rt - 1) / (16 * rt);
   int wpb = blocks < 256 ? 8 : 4;
   while ((K / 32) % wpb) wpb >>= 1;
 #define GM_MV_W(R)                                              \
   switch (wpb) {                                                \
-    case 8: return launch_mfma_w<R, 8>(w, M, K, x, n_tok, y, s); \
-    case 4: return launch_mfma_w<R, 4>(w, M, K, x, n_tok, y, s); \
-    case 2: return launch_mfma_w<R, 2>(w, M, K, x, n_tok, y, s); \
-    default: return launch_mfma_w<R, 1>(w, M, K, x, n_tok, y, s); \
+    case 8: return launch_mfma_w<R, 8>(w, M, K, x, n_tok, add, y, s); \
+    case 4: return launch_mfma_w<R, 4>(w, M, K, x, n_tok, add, y, s); \
+    case 2: return launch_mfma_w<R, 2>(w, M, K, x, n_tok, add, y, s); \
+    default: return launch_mfma_w<R, 1>(w, M, K, x, n_tok, add, y, s); \
   }
   if (rt == 2) GM_MV_W(2)
   GM_MV_W(1)
@@ -425,11 +406,19 @@ int launch_mv1(const uint16_t* w, int M, int K, const float* x, float* y, const 
 }  // namespace
 
 // K a multiple of 32 and <= 16384, w and x 16-byte aligned (checked by the
-// caller).  One token: the streaming FMA kernel; more: the MFMA kernel, 16
-// tokens per column tile.
+// caller).  One token: the streaming FMA kernel; more: gm_launch_dense.
 int gm_launch_mv_bf16(const uint16_t* w, int M, int K, const float* x, int n_tok, float* y, hipStream_t s) {
   if (n_tok == 1) return launch_mv1(w, M, K, x, y, nullptr, s);
-  return launch_mfma(w, M, K, x, n_tok, y, s);
+  return gm_launch_dense(w, M, nullptr, 0, K, x, n_tok, nullptr, y, nullptr, s);
+}
+
+// Two or more tokens: the tiled GEMM (gemm_bf16.hip) where the call fills the
+// chip, else the MFMA kernel above, 16 tokens per column tile.
+int gm_launch_dense(const uint16_t* w, int M, const uint16_t* w2, int M2, int K, const float* x, int T,
+                    const float* add, float* y, float* y2, hipStream_t s) {
+  if (gm_gemm_bf16_takes(M + (w2 ? M2 : 0), T)) return gm_launch_gemm_bf16(w, M, w2, M2, K, x, T, add, y, y2, s);
+  if (int rc = launch_mfma(w, M, K, x, T, add, y, s)) return rc;
+  return w2 ? launch_mfma(w2, M2, K, x, T, nullptr, y2, s) : GM_OK;
 }
 
 // One token, y = add + W x (the residual of the core layers' output projections);
