@@ -315,6 +315,21 @@ int gm_ssm_decode(const gm_ssm_layer* L, const float* x, float* y, float* conv_s
                   void* ws, size_t ws_bytes, void* stream);
 
 /*
+ * A prompt of T tokens through a core layer in one call: as T calls of
+ * gm_attn_decode at positions pos .. pos + T - 1 / of gm_ssm_decode (the same
+ * sums in another order), every launch over all tokens (1024 at a time).  x and
+ * y are [T][D]; T = 0 does nothing; the caches must be 16-byte aligned.  Replace
+ * qwen/forward.py:attn_forward (133-239) / ssm_forward (292-431) at T > 1.
+ */
+size_t gm_attn_prefill_workspace_bytes(const gm_attn_layer* L, int T, int max_pos);
+int gm_attn_prefill(const gm_attn_layer* L, const float* x, float* y, int T, float* k_cache, float* v_cache, int pos,
+                    int max_pos, const float* rope_cos, const float* rope_sin, int flags, void* ws, size_t ws_bytes,
+                    void* stream);
+size_t gm_ssm_prefill_workspace_bytes(const gm_ssm_layer* L, int T);
+int gm_ssm_prefill(const gm_ssm_layer* L, const float* x, float* y, int T, float* conv_state, float* rec_state,
+                   int flags, void* ws, size_t ws_bytes, void* stream);
+
+/*
  * A core layer linked to the MoE block that follows it in the decoder layer
  * (qwen/forward.py:880-884 runs x = x + moe_forward(rms_norm(x, post_norm)) on
  * the core layer's output): as gm_attn_decode / gm_ssm_decode, and the layer's

@@ -108,6 +108,11 @@ SIGNATURES = {
     "gm_ssm_decode": (_i32, [ctypes.POINTER(GmSsmLayer), _vp, _vp, _vp, _vp, _i32, _vp, _sz, _vp]),
     "gm_ssm_decode_moe": (_i32, [ctypes.POINTER(GmSsmLayer), _vp, _vp, _vp, _vp, _i32, _vp, _sz,
                                  ctypes.POINTER(GmMoeLayer), _vp, _sz, _vp]),
+    "gm_attn_prefill_workspace_bytes": (_sz, [ctypes.POINTER(GmAttnLayer), _i32, _i32]),
+    "gm_attn_prefill": (_i32, [ctypes.POINTER(GmAttnLayer), _vp, _vp, _i32, _vp, _vp, _i32, _i32, _vp, _vp, _i32,
+                               _vp, _sz, _vp]),
+    "gm_ssm_prefill_workspace_bytes": (_sz, [ctypes.POINTER(GmSsmLayer), _i32]),
+    "gm_ssm_prefill": (_i32, [ctypes.POINTER(GmSsmLayer), _vp, _vp, _i32, _vp, _vp, _i32, _vp, _sz, _vp]),
     "gm_moe_forward_acc": (_i32, [ctypes.POINTER(GmMoeLayer), _vp, _vp, _i32, _vp, _sz, _vp]),
     "gm_rms_norm": (_i32, [_vp, _vp, _i32, _i32, _f32, _vp, _vp]),
 }

@@ -444,6 +444,53 @@ int gm_ssm_decode(const gm_ssm_layer* L, const float* x, float* y, float* conv_s
   return gm_ssm_run(L, x, y, conv_state, rec_state, flags, static_cast<uint8_t*>(ws), as_stream(stream));
 }
 
+// ---- prompts through the core layers
+size_t gm_attn_prefill_workspace_bytes(const gm_attn_layer* L, int T, int max_pos) {
+  if (T < 1 || max_pos < 1 || check_attn(L) != GM_OK) return 0;
+  return gm_attn_prefill_ws(L, T, max_pos);
+}
+
+int gm_attn_prefill(const gm_attn_layer* L, const float* x, float* y, int T, float* k_cache, float* v_cache, int pos,
+                    int max_pos, const float* rope_cos, const float* rope_sin, int flags, void* ws, size_t ws_bytes,
+                    void* stream) {
+  if (int rc = check_attn(L)) return rc;
+  if (T < 0) return gm_fail_arg("gm_attn_prefill: negative T");
+  if (T == 0) return GM_OK;
+  if (int rc = check_io("gm_attn_prefill", x, y)) return rc;
+  if (max_pos < 1 || pos < 0 || pos > max_pos - T)
+    return gm_fail_arg("gm_attn_prefill: positions %d .. + %d must be in [0, max_pos=%d)", pos, T, max_pos);
+  if (!k_cache || !v_cache || !ws || (L->rope_dim > 0 && (!rope_cos || !rope_sin)))
+    return gm_fail_arg("gm_attn_prefill: NULL cache, rope table or workspace");
+  if (reinterpret_cast<uintptr_t>(k_cache) % 16 || reinterpret_cast<uintptr_t>(v_cache) % 16)
+    return gm_fail_arg("gm_attn_prefill: the caches must be 16-byte aligned");
+  const size_t need = gm_attn_prefill_ws(L, T, max_pos);
+  if (ws_bytes < need)
+    return gm_fail_arg("gm_attn_prefill: workspace %zu bytes < %zu needed", ws_bytes, need), GM_EWORKSPACE;
+  if (reinterpret_cast<uintptr_t>(ws) % 256) return gm_fail_arg("gm_attn_prefill: workspace must be 256-byte aligned");
+  return gm_attn_prefill_run(L, x, y, k_cache, v_cache, T, pos, rope_cos, rope_sin, flags, static_cast<uint8_t*>(ws),
+                             as_stream(stream));
+}
+
+size_t gm_ssm_prefill_workspace_bytes(const gm_ssm_layer* L, int T) {
+  if (T < 1 || check_ssm(L) != GM_OK) return 0;
+  return gm_ssm_prefill_ws(L, T);
+}
+
+int gm_ssm_prefill(const gm_ssm_layer* L, const float* x, float* y, int T, float* conv_state, float* rec_state,
+                   int flags, void* ws, size_t ws_bytes, void* stream) {
+  if (int rc = check_ssm(L)) return rc;
+  if (T < 0) return gm_fail_arg("gm_ssm_prefill: negative T");
+  if (T == 0) return GM_OK;
+  if (int rc = check_io("gm_ssm_prefill", x, y)) return rc;
+  if (!rec_state || !ws || (L->conv_k > 1 && !conv_state))
+    return gm_fail_arg("gm_ssm_prefill: NULL state or workspace");
+  const size_t need = gm_ssm_prefill_ws(L, T);
+  if (ws_bytes < need)
+    return gm_fail_arg("gm_ssm_prefill: workspace %zu bytes < %zu needed", ws_bytes, need), GM_EWORKSPACE;
+  if (reinterpret_cast<uintptr_t>(ws) % 256) return gm_fail_arg("gm_ssm_prefill: workspace must be 256-byte aligned");
+  return gm_ssm_prefill_run(L, x, y, conv_state, rec_state, T, flags, static_cast<uint8_t*>(ws), as_stream(stream));
+}
+
 // The MoE block that follows a core layer, for the linked entry points: it must
 // run on the T = 1 accumulator kernels (gm_moe_chain_fused(&moe, 1, 1) == 1),
 // share the core layer's D and carry router_t; its workspace holds the

@@ -17,23 +17,21 @@
 //    loads (1.2 us a step when alone on a CU) two or three others fill.
 // One token tile per wave (CT = 1) against two at the same row count: 136
 // against 163 us there, 57 against 73 at T = 300 (more blocks, three to a CU).
+// A step's 64 k are summed by themselves, the lower planes first, two row tiles'
+// chains of MFMAs in turn, and then added to the running sum: error against 64
+// bits 1.2e-7 (one chain through all steps: 5e-7 at K = 2048, 7e-7 at 4096; the
+// few-token kernel: 2.5e-7), at the same speed as adding every 256 k (1.8e-7).
 // Measured before (k_mv_bf16_mfma, every weight read per 16 tokens) and now, us:
-//   M = 9216 K = 2048:  T = 24 26 -> 18, 57 41 -> 23, 120 76 -> 35, 300 199 -> 57, 1021 651 -> 135
-//   M = 2048 K = 4096:  T = 100 44 -> 40, 300 114 -> 44, 1000 364 -> 73
-//   M = 248320 K = 2048: T = 20 508 -> 236-259, 57 1051 -> 269
-// (T = 1021: 855 TFLOP/s on the matrix cores; a large library product: 1120.)
+//   M = 9216 K = 2048:  T = 24 26 -> 19, 57 41 -> 23, 120 76 -> 37, 300 199 -> 58, 1021 651 -> 141
+//   M = 2048 K = 4096:  T = 100 44 -> 40, 300 114 -> 45, 1000 364 -> 77
+//   M = 248320 K = 2048: T = 20 508 -> 274, 57 1051 -> 296
+// (T = 1021: 819 TFLOP/s on the matrix cores; a large library product: 1120.)
 #include "bf16_split.h"
 #include "kernels.h"
 
 namespace {
 
 constexpr int kBK = 64;                       // k values per step (two 32-wide MFMA k-steps)
-// Steps between two additions into the running total: the chain of fp32
-// additions stays as short as the K parts of the few-token kernel (error against
-// 64 bits at K = 2048 / 4096 without it 5e-7 / 7e-7, with it 2e-7, the few-token
-// kernel 3e-7).
-constexpr int kFold = 4;
-
 struct GemmArgs {
   const uint16_t* w;     // [M][K]
   const uint16_t* w2;    // [M2][K] rows that follow w's (M2 = 0: none)
@@ -103,13 +101,11 @@ __global__ void __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) k_gemm_bf16(GemmArg
     }
   };
 
-  // acc: the sums of up to kFold steps, then added into tot (a chain of 8 kFold
-  // additions at most, as short as the K parts of the few-token kernel)
-  gm_f32x4 acc[RT][CT], tot[RT][CT];
+  gm_f32x4 acc[RT][CT];
 #pragma unroll
   for (int r = 0; r < RT; ++r)
 #pragma unroll
-    for (int c = 0; c < CT; ++c) { acc[r][c] = gm_f32x4{0.f, 0.f, 0.f, 0.f}; tot[r][c] = acc[r][c]; }
+    for (int c = 0; c < CT; ++c) acc[r][c] = gm_f32x4{0.f, 0.f, 0.f, 0.f};
 
   load(min(s0, nstep - 1));
   stage(0);
@@ -127,37 +123,54 @@ __global__ void __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) k_gemm_bf16(GemmArg
     if (more) load(min(s + 1, nstep - 1));
     if (s < s1) {
       const uint8_t* A = abuf + (i & 1) * ABUF;
+      gm_u32x4 pl[CT][2][3];
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        if (s * kBK + 32 * h >= K) break;                       // K % 64 == 32: half a last step
-        gm_u32x4 pl[CT][3];
+      for (int c = 0; c < CT; ++c)
 #pragma unroll
-        for (int c = 0; c < CT; ++c) split3(xc[c][h][0], xc[c][h][1], pl[c]);
+        for (int h = 0; h < 2; ++h) split3(xc[c][h][0], xc[c][h][1], pl[c][h]);
+      const bool half = s * kBK + 32 >= K;                      // K % 64 == 32: half a last step
+      constexpr int RG = 2;                                     // row tiles at a time: two independent chains
 #pragma unroll
-        for (int r = 0; r < RT; ++r) {
-          const int ra = 16 * r + l16;
-          const gm_bf16x8 a = *reinterpret_cast<const gm_bf16x8*>(A + ra * (2 * kBK) + 16 * ((4 * h + q) ^ ((ra >> 1) & 7)));
+      for (int r0 = 0; r0 < RT; r0 += RG) {
+        gm_bf16x8 a[RG][2];
+        gm_f32x4 d[RG][CT];
 #pragma unroll
-          for (int c = 0; c < CT; ++c)
+        for (int r = 0; r < RG; ++r) {
+          const int ra = 16 * (r0 + r) + l16;
 #pragma unroll
-            for (int p = 0; p < 3; ++p)
-              acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(gm_bf16x8, pl[c][p]), acc[r][c], 0, 0, 0);
+          for (int h = 0; h < 2; ++h)
+            a[r][h] = *reinterpret_cast<const gm_bf16x8*>(A + ra * (2 * kBK) + 16 * ((4 * h + q) ^ ((ra >> 1) & 7)));
+#pragma unroll
+          for (int c = 0; c < CT; ++c) d[r][c] = gm_f32x4{0.f, 0.f, 0.f, 0.f};
         }
+        auto mul = [&](int h, int p) {
+#pragma unroll
+          for (int r = 0; r < RG; ++r)
+#pragma unroll
+            for (int c = 0; c < CT; ++c)
+              d[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[r][h], __builtin_bit_cast(gm_bf16x8, pl[c][h][p]),
+                                                                d[r][c], 0, 0, 0);
+        };
+        if (!half) {
+          mul(1, 2);
+          mul(0, 2);
+          mul(1, 1);
+          mul(0, 1);
+          mul(1, 0);
+        } else {
+          mul(0, 2);
+          mul(0, 1);
+        }
+        mul(0, 0);
+#pragma unroll
+        for (int r = 0; r < RG; ++r)
+#pragma unroll
+          for (int c = 0; c < CT; ++c) acc[r0 + r][c] += d[r][c];
       }
-    }
-    if (i % kFold == kFold - 1) {
-#pragma unroll
-      for (int r = 0; r < RT; ++r)
-#pragma unroll
-        for (int c = 0; c < CT; ++c) { tot[r][c] += acc[r][c]; acc[r][c] = gm_f32x4{0.f, 0.f, 0.f, 0.f}; }
     }
     if (more) stage((i + 1) & 1);
     __syncthreads();
   }
-#pragma unroll
-  for (int r = 0; r < RT; ++r)
-#pragma unroll
-    for (int c = 0; c < CT; ++c) acc[r][c] += tot[r][c];
   if constexpr (KS > 1) {                                       // K parts added in part order
     gm_f32x4* red = reinterpret_cast<gm_f32x4*>(smem);
     if (grp > 0) {

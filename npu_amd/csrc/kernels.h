@@ -23,7 +23,8 @@ int gm_launch_matvec(int qtype, const void* w, int M, int K, const float* x, int
 // Dense bf16 product, any number of tokens (K % 32 == 0, K <= 16384, 16-byte
 // aligned w and x).
 int gm_launch_mv_bf16(const uint16_t* w, int M, int K, const float* x, int n_tok, float* y, hipStream_t s);
-// Two or more tokens, with the extras of gm_launch_gemm_bf16.
+// The core layers' prompts: any number of tokens, with the extras of
+// gm_launch_gemm_bf16.
 int gm_launch_dense(const uint16_t* w, int M, const uint16_t* w2, int M2, int K, const float* x, int T,
                     const float* add, float* y, float* y2, hipStream_t s);
 // Many tokens (gemm_bf16.hip): y = x W^T (+ add, [T][M]) and, when w2 is given,
@@ -65,6 +66,14 @@ struct GmSsmWs {
 GmSsmWs gm_ssm_ws_layout(const gm_ssm_layer* L);
 int gm_ssm_run(const gm_ssm_layer* L, const float* x, float* y, float* conv_state, float* rec_state, int flags,
                uint8_t* ws, hipStream_t s, const GmNextRouter* moe = nullptr);
+
+// A prompt of T >= 2 tokens through a core layer (core_prefill.hip).
+size_t gm_attn_prefill_ws(const gm_attn_layer* L, int T, int max_pos);
+int gm_attn_prefill_run(const gm_attn_layer* L, const float* x, float* y, float* kc, float* vc, int T, int pos0,
+                        const float* cosr, const float* sinr, int flags, uint8_t* ws, hipStream_t s);
+size_t gm_ssm_prefill_ws(const gm_ssm_layer* L, int T);
+int gm_ssm_prefill_run(const gm_ssm_layer* L, const float* x, float* y, float* conv_state, float* rec_state, int T,
+                       int flags, uint8_t* ws, hipStream_t s);
 
 // MoE workspace layout for T tokens (offsets in bytes, 256-byte aligned).
 struct GmMoeWs {

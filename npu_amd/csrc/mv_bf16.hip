@@ -254,7 +254,11 @@ __global__ void __launch_bounds__(64 * NW) k_mv_bf16(const uint16_t* __restrict_
   }
 }
 
-template <int RT, int WPB, int NC>
+// STEPS: two k-steps' products are summed by themselves, the lower planes first,
+// and then added to the running sum (as in gemm_bf16.hip): error against 64 bits
+// 2.4e-7 -> 0.9e-7, 3-6% slower at T <= 16; the core layers' prompts take it, so
+// that they are no less exact than their one-token path.
+template <int RT, int WPB, int NC, bool STEPS>
 __global__ void __launch_bounds__(64 * WPB) k_mv_bf16_mfma(const uint16_t* __restrict__ w, int M, int K,
                                                         const float* __restrict__ x, int n_tok,
                                                         const float* __restrict__ add, float* __restrict__ y) {
@@ -286,16 +290,25 @@ __global__ void __launch_bounds__(64 * WPB) k_mv_bf16_mfma(const uint16_t* __res
       xb[c] = xr[(c0 + 32 * c) / 4 + 1];
     }
     __builtin_amdgcn_sched_barrier(0);                          // every load of the chunk before the first use
+    constexpr int NS = STEPS && NC > 1 ? 2 : 1;
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      gm_u32x4 pl[3];
-      split3(xa[c], xb[c], pl);
+    for (int c = 0; c < NC; c += NS) {
+      gm_u32x4 pl[NS][3];
+      gm_f32x4 d[RT];
 #pragma unroll
-      for (int rt = 0; rt < RT; ++rt)
+      for (int u = 0; u < NS; ++u) split3(xa[c + u], xb[c + u], pl[u]);
 #pragma unroll
-        for (int p = 0; p < 3; ++p)
-          acc[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gm_bf16x8, a[rt][c]),
-                                                            __builtin_bit_cast(gm_bf16x8, pl[p]), acc[rt], 0, 0, 0);
+      for (int rt = 0; rt < RT; ++rt) d[rt] = STEPS ? gm_f32x4{0.f, 0.f, 0.f, 0.f} : acc[rt];
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int u = 0; u < NS; ++u)
+#pragma unroll
+          for (int rt = 0; rt < RT; ++rt)
+            d[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gm_bf16x8, a[rt][c + u]),
+                                                            __builtin_bit_cast(gm_bf16x8, pl[u][STEPS ? 2 - i : i]), d[rt], 0, 0, 0);
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) acc[rt] = STEPS ? acc[rt] + d[rt] : d[rt];
     }
   }
   if (wave > 0) {
@@ -319,13 +332,13 @@ __global__ void __launch_bounds__(64 * WPB) k_mv_bf16_mfma(const uint16_t* __res
   }
 }
 
-template <int RT, int WPB>
+template <int RT, int WPB, bool STEPS>
 int launch_mfma_w(const uint16_t* w, int M, int K, const float* x, int n_tok, const float* add, float* y,
                   hipStream_t s) {
   const dim3 grid((unsigned)((M + 16 * RT - 1) / (16 * RT)), (unsigned)((n_tok + 15) / 16));
   const int steps = K / (32 * WPB);                              // k-steps per wave (exact: WPB divides K / 32)
 #define GM_MV_GO(NC)                                                                               \
-  hipLaunchKernelGGL((k_mv_bf16_mfma<RT, WPB, NC>), grid, dim3(64 * WPB), 0, s, w, M, K, x, n_tok, add, y); \
+  hipLaunchKernelGGL((k_mv_bf16_mfma<RT, WPB, NC, STEPS>), grid, dim3(64 * WPB), 0, s, w, M, K, x, n_tok, add, y); \
   break;
   switch (steps % 8 == 0 ? 8 : steps % 4 == 0 ? 4 : steps % 2 == 0 ? 2 : 1) {
     case 8: GM_MV_GO(8)
@@ -342,6 +355,7 @@ int launch_mfma_w(const uint16_t* w, int M, int K, const float* x, int n_tok, co
 // the grid holds about 1024 waves, each wave taking an equal number of 32-wide
 // k-steps: the largest of 8 (4 for grids of >= 256 blocks), 4, 2, 1 that divides
 // K / 32 (K = 576: 2 waves of 9 steps).
+template <bool STEPS>
 int launch_mfma(const uint16_t* w, int M, int K, const float* x, int n_tok, const float* add, float* y,
                 hipStream_t s) {
   const int rt = M >= 8192 ? 2 : 1;
@@ -350,10 +364,10 @@ int launch_mfma(const uint16_t* w, int M, int K, const float* x, int n_tok, cons
   while ((K / 32) % wpb) wpb >>= 1;
 #define GM_MV_W(R)                                              \
   switch (wpb) {                                                \
-    case 8: return launch_mfma_w<R, 8>(w, M, K, x, n_tok, add, y, s); \
-    case 4: return launch_mfma_w<R, 4>(w, M, K, x, n_tok, add, y, s); \
-    case 2: return launch_mfma_w<R, 2>(w, M, K, x, n_tok, add, y, s); \
-    default: return launch_mfma_w<R, 1>(w, M, K, x, n_tok, add, y, s); \
+    case 8: return launch_mfma_w<R, 8, STEPS>(w, M, K, x, n_tok, add, y, s); \
+    case 4: return launch_mfma_w<R, 4, STEPS>(w, M, K, x, n_tok, add, y, s); \
+    case 2: return launch_mfma_w<R, 2, STEPS>(w, M, K, x, n_tok, add, y, s); \
+    default: return launch_mfma_w<R, 1, STEPS>(w, M, K, x, n_tok, add, y, s); \
   }
   if (rt == 2) GM_MV_W(2)
   GM_MV_W(1)
@@ -406,19 +420,20 @@ int launch_mv1(const uint16_t* w, int M, int K, const float* x, float* y, const 
 }  // namespace
 
 // K a multiple of 32 and <= 16384, w and x 16-byte aligned (checked by the
-// caller).  One token: the streaming FMA kernel; more: gm_launch_dense.
+// caller).  One token: the streaming FMA kernel; more: the tiled GEMM
+// (gemm_bf16.hip) where the call fills the chip, else the MFMA kernel above, 16
+// tokens per column tile.
 int gm_launch_mv_bf16(const uint16_t* w, int M, int K, const float* x, int n_tok, float* y, hipStream_t s) {
   if (n_tok == 1) return launch_mv1(w, M, K, x, y, nullptr, s);
-  return gm_launch_dense(w, M, nullptr, 0, K, x, n_tok, nullptr, y, nullptr, s);
+  if (gm_gemm_bf16_takes(M, n_tok)) return gm_launch_gemm_bf16(w, M, nullptr, 0, K, x, n_tok, nullptr, y, nullptr, s);
+  return launch_mfma<false>(w, M, K, x, n_tok, nullptr, y, s);
 }
 
-// Two or more tokens: the tiled GEMM (gemm_bf16.hip) where the call fills the
-// chip, else the MFMA kernel above, 16 tokens per column tile.
 int gm_launch_dense(const uint16_t* w, int M, const uint16_t* w2, int M2, int K, const float* x, int T,
                     const float* add, float* y, float* y2, hipStream_t s) {
   if (gm_gemm_bf16_takes(M + (w2 ? M2 : 0), T)) return gm_launch_gemm_bf16(w, M, w2, M2, K, x, T, add, y, y2, s);
-  if (int rc = launch_mfma(w, M, K, x, T, add, y, s)) return rc;
-  return w2 ? launch_mfma(w2, M2, K, x, T, nullptr, y2, s) : GM_OK;
+  if (int rc = launch_mfma<true>(w, M, K, x, T, add, y, s)) return rc;
+  return w2 ? launch_mfma<true>(w2, M2, K, x, T, nullptr, y2, s) : GM_OK;
 }
 
 // One token, y = add + W x (the residual of the core layers' output projections);

@@ -11,17 +11,17 @@ Same names and call signatures as the reference:
   ssm_states, n_layer, skip_moe)`` (:834-893), returning ``(logits [T, vocab],
   kv_caches, ssm_states)``.
 
-Each core layer runs as one C-ABI call per token (``gm_attn_decode`` /
+Each core layer runs one token as one C-ABI call (``gm_attn_decode`` /
 ``gm_ssm_decode``): its large projections are bf16 weights resident in HBM (as the
 reference's NPU operators stage them, :813-831), its small ones and all state fp32.
 The KV cache is preallocated as ``[max_pos][n_head_kv][head_dim]`` per layer (the
 reference concatenates a ``[B, T, n_head, head_dim]`` cache per step, repeating each kv
 head over its q heads); the Gated DeltaNet state is ``(conv_state [1, C, k - 1],
 S [1, Hv, Sk, Sv])``, the reference's tuple, as device tensors updated in place.
-Several tokens (prefill) run the core layers one token at a time, which is the
-causal attention of the reference's masked prefill and the token loop of its
-recurrence; the MoE block then takes the layer's T tokens at once.  There is no CPU
-path: without the built library every call raises.
+Several tokens (a prompt) are one call per core layer too (``gm_attn_prefill`` /
+``gm_ssm_prefill``), every launch over all tokens; the MoE block then takes the
+layer's T tokens at once.  There is no CPU path: without the built library every
+call raises.
 """
 from __future__ import annotations
 
@@ -158,6 +158,20 @@ class GpuAttn:
                                         L.stream_ptr())
         L.check(rc, "gm_attn_decode_moe")
 
+    def prompt(self, x: torch.Tensor, cache: "KVCache", pos: int, cos: torch.Tensor, sin: torch.Tensor,
+               residual: bool, out: torch.Tensor) -> None:
+        """x [T, D], positions pos .. pos + T - 1, in one call (gm_attn_prefill).  The
+        workspace (61 KB a token, at most 1024 tokens' worth) is the call's own."""
+        T = x.shape[0]
+        n = L.lib().gm_attn_prefill_workspace_bytes(ctypes.byref(self.struct), T, cache.max_pos)
+        if n == 0:
+            raise ValueError(f"gm_attn_prefill_workspace_bytes: {L.last_error()}")
+        ws = torch.empty(n, dtype=torch.uint8, device=x.device)
+        rc = L.lib().gm_attn_prefill(ctypes.byref(self.struct), L.ptr(x), L.ptr(out), T, L.ptr(cache.k),
+                                     L.ptr(cache.v), pos, cache.max_pos, L.ptr(cos), L.ptr(sin),
+                                     L.GM_MOE_RESIDUAL if residual else 0, L.ptr(ws), n, L.stream_ptr())
+        L.check(rc, "gm_attn_prefill")
+
 
 class KVCache:
     """One attention layer's cache, ``[max_pos][n_head_kv][head_dim]`` fp32 for k and v,
@@ -204,9 +218,13 @@ def attn_forward(x: torch.Tensor, layer: AttnLayer, cfg: Config, cos: torch.Tens
     cd, sd = _rope_on_device(cos, sin)
     y = torch.empty_like(xd)
     with profile("attn.decode"):
-        for t in range(T):
-            layer.gpu.step(xd[t], kv_cache, start_pos + t, cd, sd, residual, y[t], moe_link)
-            kv_cache.length += 1
+        if T > 1 and kv_cache.k.data_ptr() % 16 == 0 and kv_cache.v.data_ptr() % 16 == 0:
+            layer.gpu.prompt(xd, kv_cache, start_pos, cd, sd, residual, y)
+            kv_cache.length += T
+        else:
+            for t in range(T):
+                layer.gpu.step(xd[t], kv_cache, start_pos + t, cd, sd, residual, y[t], moe_link)
+                kv_cache.length += 1
     y = y.view(1, T, D)
     return (y.cpu() if on_host else y), kv_cache
 
@@ -289,6 +307,19 @@ class GpuSsm:
                                        mws.numel(), L.stream_ptr())
         L.check(rc, "gm_ssm_decode_moe")
 
+    def prompt(self, x: torch.Tensor, state, residual: bool, out: torch.Tensor) -> None:
+        """x [T, D] in one call (gm_ssm_prefill).  The workspace (108 KB a token, at most
+        1024 tokens' worth) is the call's own."""
+        conv, S = state
+        T = x.shape[0]
+        n = L.lib().gm_ssm_prefill_workspace_bytes(ctypes.byref(self.struct), T)
+        if n == 0:
+            raise ValueError(f"gm_ssm_prefill_workspace_bytes: {L.last_error()}")
+        ws = torch.empty(n, dtype=torch.uint8, device=x.device)
+        rc = L.lib().gm_ssm_prefill(ctypes.byref(self.struct), L.ptr(x), L.ptr(out), T, L.ptr(conv), L.ptr(S),
+                                    L.GM_MOE_RESIDUAL if residual else 0, L.ptr(ws), n, L.stream_ptr())
+        L.check(rc, "gm_ssm_prefill")
+
 
 def ssm_forward(x: torch.Tensor, layer: SSMLayer, cfg: Config, ssm_state, *, residual: bool = False,
                 moe_link=None):
@@ -311,8 +342,10 @@ def ssm_forward(x: torch.Tensor, layer: SSMLayer, cfg: Config, ssm_state, *, res
     xd = x.reshape(T, D).to(device(), torch.float32).contiguous()
     y = torch.empty_like(xd)
     with profile("ssm.decode"):
-        for t in range(T):
-            layer.gpu.step(xd[t], state, residual, y[t], moe_link)
+        if T > 1:
+            layer.gpu.prompt(xd, state, residual, y)
+        elif T == 1:
+            layer.gpu.step(xd[0], state, residual, y[0], moe_link)
     y = y.view(1, T, D)
     return (y.cpu() if on_host else y), state
 

@@ -28,3 +28,101 @@ def test_gemm_bf16_tiles(gpu, M, K, T):
     bound = (2 * 24 + K / 256 + 4) * 2.0 ** -24 * (x.abs().double() @ w.abs().double().T)
     assert bool(((y - ref).abs() <= bound).all())
     assert float((y - ref).norm() / ref.norm()) <= 1e-6
+
+
+# ---- prompts through the core layers (gm_attn_prefill / gm_ssm_prefill)
+def _cfgs(**kw):
+    from npu_amd import qwen_core as QN
+    from oracle import qwen_core as QC
+    kw = dict(dict(d_model=512, n_head=4, n_head_kv=2, head_dim=128, rope_dim=32, rope_theta=1e6,
+                   ssm_d_inner=256, ssm_d_state=64, ssm_n_k_heads=2, ssm_n_v_heads=4), **kw)
+    return QC.CoreCfg(**kw), QN.Config(**kw)
+
+
+def _rel(a, b):
+    return float((a.double().cpu() - b.double()).abs().max() / b.double().abs().max())
+
+
+def _attn(ocfg, seed):
+    g = torch.Generator().manual_seed(seed)
+    D, Hq, Hkv, Dh = ocfg.d_model, ocfg.n_head, ocfg.n_head_kv, ocfg.head_dim
+    bf = lambda *s: (torch.randn(*s, generator=g) * 0.03).to(torch.bfloat16).float()
+    nw = lambda n: 1 + 0.1 * torch.randn(n, generator=g)
+    return dict(attn_norm=nw(D), post_norm=nw(D), wq=bf(2 * Hq * Dh, D), wk=bf(Hkv * Dh, D), wv=bf(Hkv * Dh, D),
+                wo=bf(D, Hq * Dh), q_norm=2 * nw(Dh), k_norm=2 * nw(Dh))
+
+
+# one query block with its keys in 5 parts, blocks that end inside a position's heads (G = 3),
+# every head_dim, a rotation over the whole head, one token past a block and past the part of
+# 1024, no rotation
+@pytest.mark.parametrize("kw,parts", [
+    (dict(), (2, 700, 2, 17)),
+    (dict(n_head=6, n_head_kv=2, head_dim=64, rope_dim=64), (5, 43, 1, 22)),
+    (dict(n_head=16, n_head_kv=2, head_dim=256, rope_dim=96), (9, 8, 130)),
+    (dict(n_head=2, n_head_kv=2, head_dim=512, rope_dim=0), (3, 65)),
+    (dict(n_head=4, n_head_kv=1, head_dim=64, rope_dim=16), (1025, 2)),
+])
+def test_attention_prompts(gpu, kw, parts):
+    """A sequence fed in parts of several tokens, each on the cache of the parts before, against
+    the oracle fed the same way: fp32 sums in another order, bar 1e-4 as for single steps."""
+    from npu_amd import qwen_core as QN
+    from oracle import qwen_core as QC
+    print(f"attention prompt case {kw} {parts}", flush=True)
+    ocfg, ncfg = _cfgs(**kw)
+    W = _attn(ocfg, 31)
+    OL, NL = QC.AttnW(**W), QN.AttnLayer(i=0, **W)
+    cos, sin = QC.build_partial_rope_cache(ocfg.rope_dim, sum(parts) + 3, ocfg.rope_theta)
+    x = torch.randn(1, sum(parts), ocfg.d_model, generator=torch.Generator().manual_seed(32))
+    oc = nc = None
+    pos = 0
+    for i, n in enumerate(parts):
+        xp = x[:, pos:pos + n]
+        yo, oc = QC.attn_forward(xp, OL, ocfg, cos, sin, oc, pos)
+        yn, nc = QN.attn_forward(xp.to(gpu), NL, ncfg, cos, sin, nc, pos, residual=i == 1)
+        pos += n
+        assert nc.length == pos
+        assert _rel(yn - xp.to(gpu) if i == 1 else yn, yo) <= 1e-4, f"part {i}"
+    rep = ocfg.n_head // ocfg.n_head_kv
+    assert _rel(nc.k[:pos], oc[0][0, :, ::rep]) <= 1e-5 and _rel(nc.v[:pos], oc[1][0, :, ::rep]) <= 1e-5
+    assert not nc.k[pos:].any()                            # nothing past the filled positions
+
+
+# d_state 64 / 128 / 256, prompts around the 16 staged tokens (8 at 256) and past the part of
+# 1024, conv kernels of 1, 2 and 8 taps, and a prompt shorter than the conv state
+@pytest.mark.parametrize("kw,parts", [
+    (dict(), (2, 16, 1, 33)),
+    (dict(ssm_d_inner=512, ssm_d_state=128, ssm_d_conv=8), (3, 2, 31)),
+    (dict(ssm_d_inner=1024, ssm_d_state=256, ssm_d_conv=2, ssm_n_k_heads=1), (9, 8)),
+    (dict(ssm_d_conv=1, ssm_n_k_heads=4), (5, 18)),
+    (dict(ssm_d_inner=128, ssm_n_k_heads=1, ssm_n_v_heads=2), (1026, 3)),
+])
+def test_ssm_prompts(gpu, kw, parts):
+    from npu_amd import qwen_core as QN
+    from oracle import qwen_core as QC
+    print(f"ssm prompt case {kw} {parts}", flush=True)
+    ocfg, ncfg = _cfgs(**kw)
+    g = torch.Generator().manual_seed(41)
+    D, Hv, Hk, S = ocfg.d_model, ocfg.ssm_n_v_heads, ocfg.ssm_n_k_heads, ocfg.ssm_d_state
+    C = 2 * Hk * S + Hv * S
+    bf = lambda *s: (torch.randn(*s, generator=g) * 0.03).to(torch.bfloat16).float()
+    r = lambda *s, sc=1.0: torch.randn(*s, generator=g) * sc
+    W = dict(attn_norm=1 + r(D, sc=0.1), post_norm=1 + r(D, sc=0.1), w_in=bf(C, D), w_gate=bf(Hv * S, D),
+             conv1d=r(C, ocfg.ssm_d_conv, sc=0.5), a=-torch.rand(Hv, generator=g), alpha=r(Hv, D, sc=0.05),
+             beta=r(Hv, D, sc=0.05), dt_bias=r(Hv, sc=0.5), ssm_norm=1 + r(S, sc=0.1), w_out=bf(D, Hv * S))
+    OL, NL = QC.SSMW(**W), QN.SSMLayer(i=0, **W)
+    x = torch.randn(1, sum(parts), D, generator=torch.Generator().manual_seed(42))
+    ck = ocfg.ssm_d_conv
+    os_ = (torch.zeros(1, C, ck - 1), torch.zeros(1, Hv, S, S))
+    ns = None
+    pos = 0
+    for i, n in enumerate(parts):
+        xp = x[:, pos:pos + n]
+        # the oracle's new conv state is cin[..., -(ck - 1):], which for one tap is everything
+        yo, os_ = QC.ssm_forward(xp, OL, ocfg, os_)
+        os_ = (os_[0][..., :ck - 1] if ck == 1 else os_[0], os_[1])
+        yn, ns = QN.ssm_forward(xp.to(gpu), NL, ncfg, ns, residual=i == 1)
+        pos += n
+        assert _rel(yn - xp.to(gpu) if i == 1 else yn, yo) <= 1e-4, f"part {i}"
+        assert _rel(ns[1], os_[1]) <= 1e-4, f"part {i}: recurrent state"
+        if ck > 1:
+            assert _rel(ns[0], os_[0]) <= 1e-5, f"part {i}: conv state"
