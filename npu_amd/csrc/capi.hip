@@ -53,8 +53,11 @@ GmMoeWs gm_moe_ws_layout(const gm_moe_layer* L, int T) {
   w.yp = o; o = align256(o + (Td * k + Td) * (size_t)L->D * 4);
   w.pre = o; o = align256(o + gm_prefill_scratch_bytes(L, T));     // every T: gm_moe_prefill takes any T
   w.acc = o; o = align256(o + 2 * gm_acc_bytes(L->E));
+  const size_t b8 = T > GM_DECODE_MAX_T && gm_pf8_ok(L) ? align256(gm_pf8_scratch_bytes(L, T)) : 0;
+  w.pre8 = o; o += b8;
   w.tl = o; o = align256(o + GM_TL_BYTES);                   // last: the timeline tool reads the end
   w.total = o;
+  w.total_min = o - b8;
   return w;
 }
 
@@ -288,7 +291,7 @@ int gm_moe_chain(const gm_moe_layer* layers, int n_layers, const float* x, float
     if (L->D != layers[0].D) return gm_fail_arg("gm_moe_chain: layer %d has D=%d, layer 0 D=%d", l, L->D, layers[0].D);
     if (!ws[l]) return gm_fail_arg("gm_moe_chain: workspace %d is NULL", l);
     if (reinterpret_cast<uintptr_t>(ws[l]) % 256) return gm_fail_arg("gm_moe_chain: workspace %d not 256-byte aligned", l);
-    const size_t need = gm_moe_ws_layout(L, T).total;
+    const size_t need = gm_moe_ws_layout(L, T).total_min;
     if (ws_bytes[l] < need)
       return gm_fail_arg("gm_moe_chain: workspace %d has %zu bytes < %zu needed", l, ws_bytes[l], need), GM_EWORKSPACE;
     fused = fused && chain_layer_fused(layers, l, T);
@@ -605,7 +608,7 @@ extern "C" int gm_moe_forward_noalloc(const gm_moe_layer* L, const float* x, flo
                                       void* stream) {
   if (int rc = check_layer(L)) return rc;
   if (T < 0) return gm_fail_arg("gm_moe_forward_noalloc: negative T");
-  const size_t need = gm_moe_ws_layout(L, T).total;
+  const size_t need = gm_moe_ws_layout(L, T).total_min;
   if (need > GM_NOALLOC_SCRATCH_BYTES)
     return gm_fail_arg("gm_moe_forward_noalloc: T=%d needs %zu workspace bytes, more than the %zu of the static "
                        "scratch (use gm_moe_forward with a workspace)", T, need, (size_t)GM_NOALLOC_SCRATCH_BYTES),
@@ -638,17 +641,18 @@ static int moe_forward_impl(const gm_moe_layer* L, const float* x, float* y, int
   if (reinterpret_cast<uintptr_t>(x) % 16 || reinterpret_cast<uintptr_t>(y) % 16)
     return gm_fail_arg("gm_moe_forward: x and y must be 16-byte aligned");
   const GmMoeWs lay = gm_moe_ws_layout(L, T);
-  if (ws_bytes < lay.total)
-    return gm_fail_arg("gm_moe_forward: workspace %zu bytes < %zu needed", ws_bytes, lay.total), GM_EWORKSPACE;
+  if (ws_bytes < lay.total_min)
+    return gm_fail_arg("gm_moe_forward: workspace %zu bytes < %zu needed", ws_bytes, lay.total_min), GM_EWORKSPACE;
   if (reinterpret_cast<uintptr_t>(ws) % 256) return gm_fail_arg("gm_moe_forward: workspace must be 256-byte aligned");
   uint8_t* w = static_cast<uint8_t*>(ws);
   hipStream_t s = as_stream(stream);
   const bool decode = path == kPathDecode || (path == kPathAuto && T <= GM_DECODE_MAX_T && T * L->k <= GM_GRP_MAXU);
   if (decode) return gm_dec_run(L, x, y, T, flags, w, lay, s, stage);
   if (stage != 0) return gm_fail_arg("gm_moe_forward_stage: stages are only defined for the decode path (T <= 8)");
+  if (T > GM_DECODE_MAX_T && gm_pf8_ok(L) && ws_bytes >= lay.total) return gm_pf8_run(L, x, y, T, flags, w, lay, s);
   if (!is_quant(L->q_gate) || !is_quant(L->q_down)) {
-    // Routed experts held as bf16 or I8 rows (K-quant expert tensors): the
-    // prefill GEMMs decode IQ4_XS / IQ3_XXS only, so the tokens run as decode
+    // Routed experts that neither set of prefill GEMMs takes (bf16 rows, I8 rows
+    // beside IQ ones, I8 layers in a smaller workspace): the tokens run as decode
     // chunks of at most 8 (every token's MoE output is independent of the
     // others).  Each chunk writes its logits / ids / weights / shared gate into
     // its rows of the full-T arrays.  (A shared expert in other formats than IQ

@@ -87,8 +87,10 @@ struct GmMoeWs {
   size_t yp;       // f32 [T * k + T][D]  per-pair / shared partial outputs (decode, T > 1)
   size_t pre;      // prefill scratch (see prefill.hip)
   size_t acc;      // T = 1 router accumulators, two buffers of gm_acc_bytes(E) (moe_decode.h)
+  size_t pre8;     // prefill scratch of layers with I8 routed experts (T > GM_DECODE_MAX_T, else empty)
   size_t tl;       // per-block timestamps (profiling build only, else empty); last region
   size_t total;
+  size_t total_min;  // without pre8: I8 layers then run T > GM_DECODE_MAX_T as decode chunks
 };
 
 // T = 1 router accumulators (layout in moe_decode.h): GM_ACC_COPIES copies of
@@ -145,6 +147,22 @@ int gm_dec_run(const gm_moe_layer* L, const float* x, float* y, int T, int flags
                   const GmMoeWs& lay, hipStream_t s, int stage = 0, const GmChainStep* cs = nullptr);
 int gm_pf_run(const gm_moe_layer* L, const float* x, float* y, int T, int flags, uint8_t* ws,
                    const GmMoeWs& lay, hipStream_t s);
+// I8 routed experts: whether gm_pf8_run takes the layer, its scratch (in ws.pre8,
+// beside ws.pre) and the run itself.
+bool gm_pf8_ok(const gm_moe_layer* L);
+size_t gm_pf8_scratch_bytes(const gm_moe_layer* L, int T);
+int gm_pf8_run(const gm_moe_layer* L, const float* x, float* y, int T, int flags, uint8_t* ws, const GmMoeWs& lay,
+               hipStream_t s);
+// Their GEMMs (prefill_i8.hip) on activation rows split into two f16 planes.
+struct GmPf8Rows {
+  uint16_t* hi;
+  uint16_t* lo;
+  float* scale;    // per row: 2^-s of the rows held times 2^s
+  float* sums;     // per 32 values of a row
+};
+int gm_pf8_split(const float* src, int rows, int K, const GmPf8Rows& a, hipStream_t s);
+int gm_pf8_gemm(const gm_moe_layer* L, bool down, const GmPf8Rows& a, const int32_t* segs, int nseg,
+                const int32_t* offsets, const int32_t* sorted, int T, float* out, hipStream_t s);
 int gm_launch_dispatch(const int32_t* ids, int T, int k, int E, int32_t* counts, int32_t* offsets,
                        int32_t* sorted_pairs, hipStream_t s);
 // Dispatch plus (inv != NULL) the inverse permutation and (segs != NULL) the

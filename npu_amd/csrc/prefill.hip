@@ -1257,23 +1257,15 @@ __global__ void __launch_bounds__(256) k_pfs_down_i8(const uint8_t* __restrict__
 
 constexpr size_t kGemmSmem = 2 * (size_t)kTileG + 256 * 4 + 128 * 16 + 2 * kSegTok * 4;
 
-template <int QTG, int QTD>
-int prefill_t(const gm_moe_layer* L, const float* x, float* y, int T, int flags, uint8_t* ws, const GmMoeWs& lay,
-              hipStream_t s) {
-  const int D = L->D, FF = L->FF, E = L->E, k = L->k;
+// Steps 1-3: prep and router (xn32: also the fp32 rows xn, or NULL), top-k and
+// dispatch (shared_T: tokens of the shared expert's own segments, or 0).
+int pf_route(const gm_moe_layer* L, const float* x, int T, uint8_t* ws, const GmMoeWs& lay, const PfWs& w,
+             float* xn32, int shared_T, hipStream_t s) {
+  const int D = L->D, E = L->E, k = L->k;
   float* logits = reinterpret_cast<float*>(ws + lay.logits);
   float* shg = reinterpret_cast<float*>(ws + lay.shg);
   int32_t* ids = reinterpret_cast<int32_t*>(ws + lay.ids);
   float* wts = reinterpret_cast<float*>(ws + lay.wts);
-  PfWs w = pf_layout(L, T, ws + lay.pre, nullptr);
-  const bool has_sh = L->gate_sh != nullptr;
-  const bool sh_apart = pf_shared_apart(L);
-  const bool sh_gemm = has_sh && !sh_apart;          // the shared expert as the GEMMs' ninth unit
-  // a shared expert in I8 rows: its own f16 MFMA GEMMs; other formats (bf16): the fp32 pass
-  const bool sh_i8 = sh_apart && L->q_gate_sh == GM_QTYPE_I8 && L->q_up_sh == GM_QTYPE_I8 &&
-                     L->q_down_sh == GM_QTYPE_I8;
-  const bool sh_f32 = sh_apart && !sh_i8;
-  const size_t P = (size_t)T * k;
   const int nrows = E + (L->sh_gate_inp ? 1 : 0);
   const int ldp = router_ld(L);
   const int nsplit = router_split(D);
@@ -1281,7 +1273,6 @@ int prefill_t(const gm_moe_layer* L, const float* x, float* y, int T, int flags,
     const int nrb = (nrows + 63) / 64, ntb = (T + 15) / 16, n_rt = nrb * ntb * nsplit;
     const dim3 g((unsigned)(n_rt + T));
     const bool f32 = L->q_router == GM_QTYPE_F32;
-    float* xn32 = sh_f32 ? w.xn : nullptr;
 #define GM_PR(NK, F32)                                                                                       \
   hipLaunchKernelGGL((k_pf_prep_router<NK, F32>), g, dim3(256), 0, s, L->router, L->sh_gate_inp, x, L->norm_w, \
                      L->norm_eps, T, D, E, ldp, w.part, nrb, ntb, n_rt, w.xh, w.xsc, xn32, w.rmsv)
@@ -1312,9 +1303,25 @@ int prefill_t(const gm_moe_layer* L, const float* x, float* y, int T, int flags,
                          w.rmsv, logits, shg, ids, wts);
   }
   GM_TRY(hipGetLastError());
-  if (int rc = gm_launch_dispatch_seg(ids, T, k, E, w.counts, w.offsets, w.sorted, w.inv, w.segs, kSegTok,
-                                     sh_gemm ? T : 0, s))
-    return rc;
+  return gm_launch_dispatch_seg(ids, T, k, E, w.counts, w.offsets, w.sorted, w.inv, w.segs, kSegTok, shared_T, s);
+}
+
+template <int QTG, int QTD>
+int prefill_t(const gm_moe_layer* L, const float* x, float* y, int T, int flags, uint8_t* ws, const GmMoeWs& lay,
+              hipStream_t s) {
+  const int D = L->D, FF = L->FF, E = L->E, k = L->k;
+  float* shg = reinterpret_cast<float*>(ws + lay.shg);
+  float* wts = reinterpret_cast<float*>(ws + lay.wts);
+  PfWs w = pf_layout(L, T, ws + lay.pre, nullptr);
+  const bool has_sh = L->gate_sh != nullptr;
+  const bool sh_apart = pf_shared_apart(L);
+  const bool sh_gemm = has_sh && !sh_apart;          // the shared expert as the GEMMs' ninth unit
+  // a shared expert in I8 rows: its own f16 MFMA GEMMs; other formats (bf16): the fp32 pass
+  const bool sh_i8 = sh_apart && L->q_gate_sh == GM_QTYPE_I8 && L->q_up_sh == GM_QTYPE_I8 &&
+                     L->q_down_sh == GM_QTYPE_I8;
+  const bool sh_f32 = sh_apart && !sh_i8;
+  const size_t P = (size_t)T * k;
+  if (int rc = pf_route(L, x, T, ws, lay, w, sh_f32 ? w.xn : nullptr, sh_gemm ? T : 0, s)) return rc;
   if (sh_f32) {                                      // shared expert rows yp[P + t], fp32
     if (int rc = gm_launch_gateup(L->q_gate_sh, L->gate_sh, L->up_sh, FF, D, w.xn, T, w.hsh, s)) return rc;
     if (int rc = gm_launch_matvec(L->q_down_sh, L->down_sh, D, FF, w.hsh, T, w.yp + P * D, s)) return rc;
@@ -1383,6 +1390,58 @@ size_t gm_prefill_scratch_bytes(const gm_moe_layer* L, int T) {
   size_t total = 0;
   pf_layout(L, T, nullptr, &total);
   return total;
+}
+
+// Layers whose routed experts (and shared expert, if any) are I8 rows, on the
+// GEMMs of prefill_i8.hip: fp32-exact activations, as their decode kernels have.
+bool gm_pf8_ok(const gm_moe_layer* L) {
+  const bool sh = !L->gate_sh || (L->q_gate_sh == GM_QTYPE_I8 && L->q_down_sh == GM_QTYPE_I8);
+  return L->q_gate == GM_QTYPE_I8 && L->q_down == GM_QTYPE_I8 && sh && L->D % kChunk == 0 && L->FF % kChunk == 0 &&
+         router_split(L->D) <= kRouterSplit;
+}
+
+struct Pf8Ws {
+  float* xn;           // [T][D] fp32 rows
+  float* h;            // [P + T][FF] fp32 SwiGLU rows
+  GmPf8Rows xr, hr;    // their planes (hi of both and lo of h in PfWs's f16 rows)
+};
+
+static Pf8Ws pf8_layout(const gm_moe_layer* L, int T, const PfWs& w, uint8_t* base, size_t* total) {
+  const size_t P = (size_t)T * L->k, D = L->D, FF = L->FF;
+  size_t o = 0;
+  auto take = [&](size_t bytes) { uint8_t* p = base ? base + o : nullptr; o = align256(o + bytes); return p; };
+  Pf8Ws v{};
+  v.xn = reinterpret_cast<float*>(take(T * D * 4));
+  v.xr = GmPf8Rows{w.xh, reinterpret_cast<uint16_t*>(take(T * D * 2)), w.xsc,
+                   reinterpret_cast<float*>(take(T * (D / 32) * 4))};
+  v.h = reinterpret_cast<float*>(take((P + T) * FF * 4));
+  v.hr = GmPf8Rows{w.hh, w.hb, w.hsc, reinterpret_cast<float*>(take((P + T) * (FF / 32) * 4))};
+  if (total) *total = o;
+  return v;
+}
+
+size_t gm_pf8_scratch_bytes(const gm_moe_layer* L, int T) {
+  size_t total = 0;
+  pf8_layout(L, T, PfWs{}, nullptr, &total);
+  return total;
+}
+
+int gm_pf8_run(const gm_moe_layer* L, const float* x, float* y, int T, int flags, uint8_t* ws, const GmMoeWs& lay,
+               hipStream_t s) {
+  const int D = L->D, FF = L->FF, k = L->k;
+  const PfWs w = pf_layout(L, T, ws + lay.pre, nullptr);
+  const Pf8Ws v = pf8_layout(L, T, w, ws + lay.pre8, nullptr);
+  const bool has_sh = L->gate_sh != nullptr;
+  const int nseg = max_segments(T, k, L->E);
+  if (int rc = pf_route(L, x, T, ws, lay, w, v.xn, has_sh ? T : 0, s)) return rc;
+  if (int rc = gm_pf8_split(v.xn, T, D, v.xr, s)) return rc;
+  if (int rc = gm_pf8_gemm(L, false, v.xr, w.segs, nseg, w.offsets, w.sorted, T, v.h, s)) return rc;
+  if (int rc = gm_pf8_split(v.h, T * k + (has_sh ? T : 0), FF, v.hr, s)) return rc;
+  if (int rc = gm_pf8_gemm(L, true, v.hr, w.segs, nseg, w.offsets, w.sorted, T, w.yp, s)) return rc;
+  hipLaunchKernelGGL(k_pf_combine, dim3(T), dim3(256), 0, s, x, w.yp, w.inv, reinterpret_cast<float*>(ws + lay.wts),
+                     reinterpret_cast<float*>(ws + lay.shg), T, k, D, has_sh ? 1 : 0, flags, y);
+  GM_TRY(hipGetLastError());
+  return GM_OK;
 }
 
 int gm_pf_run(const gm_moe_layer* L, const float* x, float* y, int T, int flags, uint8_t* ws, const GmMoeWs& lay,

@@ -126,3 +126,60 @@ def test_ssm_prompts(gpu, kw, parts):
         assert _rel(ns[1], os_[1]) <= 1e-4, f"part {i}: recurrent state"
         if ck > 1:
             assert _rel(ns[0], os_[0]) <= 1e-5, f"part {i}: conv state"
+
+
+# ---- MoE blocks with I8 routed experts over more than 8 tokens (prefill_i8.hip)
+def _i8_block(gpu, D, FF, E, k, q_gate, q_down, shared, seed):
+    from npu_amd import synth
+    from npu_amd.moe import GpuMoeBlock
+    h = synth.host_moe_layer(seed, D=D, FF=FF, E=E, k=k, q_gate=q_gate, q_down=q_down, shared=shared, norm=True)
+    return GpuMoeBlock.from_host(h, device=gpu)
+
+
+# the first T past the decode kernels (mostly one token an expert), segments of exactly 32, of
+# 33 and of 1 token (few experts), one row tile, odd counts of 128-wide steps, no shared expert
+@pytest.mark.parametrize("D,FF,E,k,T,q_gate,q_down,shared", [
+    (512, 256, 64, 8, 9, QT.Q6_K, QT.Q5_K, True),
+    (256, 256, 2, 2, 33, QT.Q8_0, QT.Q6_K, True),
+    (256, 512, 4, 1, 128, QT.Q5_K, QT.Q4_K, False),
+    (768, 256, 16, 4, 130, QT.Q4_K, QT.Q8_0, True),
+    (2048, 512, 256, 8, 41, QT.Q6_K, QT.Q6_K, True),
+])
+def test_moe_i8_prompts(gpu, D, FF, E, k, T, q_gate, q_down, shared):
+    """Against the same tokens through the decode kernels, eight at a time.  Both keep the
+    weights exact and the activations to 2^-23 with fp32 sums (each within 1e-6 of 64 bits),
+    so their difference is held to 3e-6 of the outputs; ids and weights come from the same
+    logits to fp32 rounding."""
+    print(f"i8 prompt case D={D} FF={FF} E={E} k={k} T={T} {q_gate} {q_down} {shared}", flush=True)
+    blk = _i8_block(gpu, D, FF, E, k, q_gate, q_down, shared, 300 + T)
+    g = torch.Generator().manual_seed(T)
+    x = (torch.randn(T, D, generator=g) * torch.exp(torch.randn(T, 1, generator=g))).to(gpu)
+    y = blk(x, residual=True)
+    ids = blk.stages(T)["topk_ids"].clone()
+    parts, pids = [], []
+    for t in range(0, T, 8):
+        parts.append(blk(x[t:t + 8], residual=True))
+        pids.append(blk.stages(len(x[t:t + 8]))["topk_ids"].clone())
+    assert torch.equal(ids, torch.cat(pids))
+    ref = torch.cat(parts).double()
+    err = (y.double() - ref).norm(dim=1) / ref.norm(dim=1)
+    assert float(err.max()) <= 3e-6, float(err.max())
+    assert torch.equal(y, blk(x, residual=True))           # fixed order: the same bits again
+
+
+def test_moe_i8_prompt_in_a_small_workspace(gpu):
+    """A workspace too small for the planes of the I8 GEMMs still runs the tokens (as decode
+    chunks): the static scratch of gm_moe_forward_noalloc, at a T that fits an IQ layer."""
+    import ctypes
+    from npu_amd import _lib as L, synth
+    from npu_amd.moe import GpuMoeBlock
+    blk = _i8_block(gpu, 2048, 512, 16, 8, QT.Q6_K, QT.Q6_K, True, 350)
+    iq = GpuMoeBlock.from_host(synth.host_moe_layer(351, D=2048, FF=512, E=16, k=8, norm=True), device=gpu)
+    limit = 16 << 20
+    T = max(t for t in range(9, 400) if ops.moe_workspace_bytes(iq.struct, t) <= limit)
+    assert ops.moe_workspace_bytes(blk.struct, T) > limit
+    x = torch.randn(T, 2048, generator=torch.Generator().manual_seed(1)).to(gpu)
+    y = torch.empty_like(x)
+    L.check(L.lib().gm_moe_forward_noalloc(ctypes.byref(blk.struct), L.ptr(x), L.ptr(y), T, 0, L.stream_ptr()), "noalloc")
+    ref = blk(x).double()
+    assert float((y.double() - ref).norm() / ref.norm()) <= 3e-6
