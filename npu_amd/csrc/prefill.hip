@@ -112,7 +112,11 @@ int router_split(int D) { return D / router_krange(D); }
 // Row stride of the router partials: E rows + the shared gate row, padded to 4.
 int router_ld(const gm_moe_layer* L) { return (L->E + 1 + 3) & ~3; }
 
-int max_segments(int T, int k, int E) { return (T * k) / kSegTok + E + (T + kSegTok - 1) / kSegTok + 1; }
+int max_segments(int T, int k, int E, int seg = kSegTok) { return (T * k) / seg + E + (T + seg - 1) / seg + 1; }
+
+// Tokens per segment of the I8 GEMMs: 16 while the experts have about that many
+// (one MFMA tile, two blocks to a CU), else 32.
+int pf8_seg(const gm_moe_layer* L, int T) { return T * L->k <= 24 * L->E ? 16 : 32; }
 
 PfWs pf_layout(const gm_moe_layer* L, int T, uint8_t* base, size_t* total) {
   const size_t P = (size_t)T * L->k, E = L->E;
@@ -1258,9 +1262,9 @@ __global__ void __launch_bounds__(256) k_pfs_down_i8(const uint8_t* __restrict__
 constexpr size_t kGemmSmem = 2 * (size_t)kTileG + 256 * 4 + 128 * 16 + 2 * kSegTok * 4;
 
 // Steps 1-3: prep and router (xn32: also the fp32 rows xn, or NULL), top-k and
-// dispatch (shared_T: tokens of the shared expert's own segments, or 0).
+// dispatch into segs (shared_T: tokens of the shared expert's own segments, or 0).
 int pf_route(const gm_moe_layer* L, const float* x, int T, uint8_t* ws, const GmMoeWs& lay, const PfWs& w,
-             float* xn32, int shared_T, hipStream_t s) {
+             float* xn32, int shared_T, int32_t* segs, int seg_tok, hipStream_t s) {
   const int D = L->D, E = L->E, k = L->k;
   float* logits = reinterpret_cast<float*>(ws + lay.logits);
   float* shg = reinterpret_cast<float*>(ws + lay.shg);
@@ -1303,7 +1307,7 @@ int pf_route(const gm_moe_layer* L, const float* x, int T, uint8_t* ws, const Gm
                          w.rmsv, logits, shg, ids, wts);
   }
   GM_TRY(hipGetLastError());
-  return gm_launch_dispatch_seg(ids, T, k, E, w.counts, w.offsets, w.sorted, w.inv, w.segs, kSegTok, shared_T, s);
+  return gm_launch_dispatch_seg(ids, T, k, E, w.counts, w.offsets, w.sorted, w.inv, segs, seg_tok, shared_T, s);
 }
 
 template <int QTG, int QTD>
@@ -1321,7 +1325,7 @@ int prefill_t(const gm_moe_layer* L, const float* x, float* y, int T, int flags,
                      L->q_down_sh == GM_QTYPE_I8;
   const bool sh_f32 = sh_apart && !sh_i8;
   const size_t P = (size_t)T * k;
-  if (int rc = pf_route(L, x, T, ws, lay, w, sh_f32 ? w.xn : nullptr, sh_gemm ? T : 0, s)) return rc;
+  if (int rc = pf_route(L, x, T, ws, lay, w, sh_f32 ? w.xn : nullptr, sh_gemm ? T : 0, w.segs, kSegTok, s)) return rc;
   if (sh_f32) {                                      // shared expert rows yp[P + t], fp32
     if (int rc = gm_launch_gateup(L->q_gate_sh, L->gate_sh, L->up_sh, FF, D, w.xn, T, w.hsh, s)) return rc;
     if (int rc = gm_launch_matvec(L->q_down_sh, L->down_sh, D, FF, w.hsh, T, w.yp + P * D, s)) return rc;
@@ -1401,6 +1405,7 @@ bool gm_pf8_ok(const gm_moe_layer* L) {
 }
 
 struct Pf8Ws {
+  int32_t* segs;       // the segment list (more segments than PfWs's where they are of 16)
   float* xn;           // [T][D] fp32 rows
   float* h;            // [P + T][FF] fp32 SwiGLU rows
   GmPf8Rows xr, hr;    // their planes (hi of both and lo of h in PfWs's f16 rows)
@@ -1411,6 +1416,7 @@ static Pf8Ws pf8_layout(const gm_moe_layer* L, int T, const PfWs& w, uint8_t* ba
   size_t o = 0;
   auto take = [&](size_t bytes) { uint8_t* p = base ? base + o : nullptr; o = align256(o + bytes); return p; };
   Pf8Ws v{};
+  v.segs = reinterpret_cast<int32_t*>(take((1 + 4 * (size_t)max_segments(T, L->k, L->E, pf8_seg(L, T))) * 4));
   v.xn = reinterpret_cast<float*>(take(T * D * 4));
   v.xr = GmPf8Rows{w.xh, reinterpret_cast<uint16_t*>(take(T * D * 2)), w.xsc,
                    reinterpret_cast<float*>(take(T * (D / 32) * 4))};
@@ -1432,12 +1438,12 @@ int gm_pf8_run(const gm_moe_layer* L, const float* x, float* y, int T, int flags
   const PfWs w = pf_layout(L, T, ws + lay.pre, nullptr);
   const Pf8Ws v = pf8_layout(L, T, w, ws + lay.pre8, nullptr);
   const bool has_sh = L->gate_sh != nullptr;
-  const int nseg = max_segments(T, k, L->E);
-  if (int rc = pf_route(L, x, T, ws, lay, w, v.xn, has_sh ? T : 0, s)) return rc;
+  const int seg = pf8_seg(L, T), nseg = max_segments(T, k, L->E, seg);
+  if (int rc = pf_route(L, x, T, ws, lay, w, v.xn, has_sh ? T : 0, v.segs, seg, s)) return rc;
   if (int rc = gm_pf8_split(v.xn, T, D, v.xr, s)) return rc;
-  if (int rc = gm_pf8_gemm(L, false, v.xr, w.segs, nseg, w.offsets, w.sorted, T, v.h, s)) return rc;
+  if (int rc = gm_pf8_gemm(L, false, v.xr, v.segs, nseg, w.offsets, w.sorted, T, seg, v.h, s)) return rc;
   if (int rc = gm_pf8_split(v.h, T * k + (has_sh ? T : 0), FF, v.hr, s)) return rc;
-  if (int rc = gm_pf8_gemm(L, true, v.hr, w.segs, nseg, w.offsets, w.sorted, T, w.yp, s)) return rc;
+  if (int rc = gm_pf8_gemm(L, true, v.hr, v.segs, nseg, w.offsets, w.sorted, T, seg, w.yp, s)) return rc;
   hipLaunchKernelGGL(k_pf_combine, dim3(T), dim3(256), 0, s, x, w.yp, w.inv, reinterpret_cast<float*>(ws + lay.wts),
                      reinterpret_cast<float*>(ws + lay.shg), T, k, D, has_sh ? 1 : 0, flags, y);
   GM_TRY(hipGetLastError());

@@ -1,6 +1,6 @@
 // Grouped GEMMs over routed experts held as I8 rows (Q8_0 / Q4_K / Q5_K / Q6_K
-// tensors, transcoded), for the MoE prefill (prefill.hip): the same segments of
-// at most 32 tokens per expert, with fp32-exact activations as the decode
+// tensors, transcoded), for the MoE prefill (prefill.hip): segments of at
+// most 16 or 32 tokens per expert, with fp32-exact activations as the decode
 // kernels of these layers have them.
 //
 // Activations: each row times a power of two (its largest magnitude in [2^14,
@@ -20,14 +20,8 @@ using namespace gm_moe;
 
 typedef _Float16 gm_f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 gm_f16x2 __attribute__((ext_vector_type(2)));
-typedef uint32_t gm_u32x3 __attribute__((ext_vector_type(3)));
 
 namespace {
-
-constexpr int kSeg = 32;             // tokens per segment, two MFMA tiles
-constexpr int kStep = 128;           // k per pipeline step: four sub-blocks
-constexpr int kRowB = 2 * kStep;     // bytes of one row of one plane in LDS
-constexpr int kPlane = kSeg * kRowB;
 
 // fp32 rows -> planes hi, lo, the row's scale 2^-s and the sums of 32 (of the
 // scaled values).  One wave per row; K % 256 == 0.
@@ -70,30 +64,25 @@ __global__ void __launch_bounds__(256) k_pf8_split(const float* __restrict__ src
   if (lane == 0) scale[r] = __builtin_ldexpf(1.0f, -sh);
 }
 
-// One pipeline step of a lane's weight row: octet q of four sub-blocks, and
-// their {s0, s1, off}.
-struct W8 {
-  uint2 q[4];
-  gm_u32x3 m[4];
-};
-
-__device__ __forceinline__ W8 w8_load(const uint8_t* __restrict__ row, int step, int q) {
-  W8 w;
-#pragma unroll
-  for (int s = 0; s < 4; ++s) {
-    const uint8_t* sb = row + (step * 4 + s) * 48;
-    w.q[s] = *reinterpret_cast<const uint2*>(sb + 8 * q);
-    w.m[s] = *reinterpret_cast<const gm_u32x3*>(sb + 32);
-  }
-  return w;
-}
-
 // Four int8 -> f16: 0x6400 | (b ^ 0x80) is 1024 + 128 + b, exactly.
 __device__ __forceinline__ void i8x4_f16(uint32_t b, uint32_t& o0, uint32_t& o1) {
   const uint32_t u = b ^ 0x80808080u;
   const gm_f16x2 c = {(_Float16)-1152.f, (_Float16)-1152.f};
   o0 = __builtin_bit_cast(uint32_t, __builtin_bit_cast(gm_f16x2, __builtin_amdgcn_perm(0x64646464u, u, 0x04010400u)) + c);
   o1 = __builtin_bit_cast(uint32_t, __builtin_bit_cast(gm_f16x2, __builtin_amdgcn_perm(0x64646464u, u, 0x04030402u)) + c);
+}
+
+// N bytes per lane from global memory to dst + N lane (dst: wave-uniform, in LDS).
+template <int N>
+__device__ __forceinline__ void to_lds(const void* src, uint8_t* dst) {
+  if constexpr (N == 16) __builtin_amdgcn_global_load_lds(src, dst, 16, 0, 0);
+  else __builtin_amdgcn_global_load_lds(src, dst, 4, 0, 0);
+}
+
+// A block barrier behind the wave's LDS accesses only (__syncthreads() and the
+// fences would also wait for the loads into LDS that are to stay in flight).
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
 struct Gemm8 {
@@ -110,126 +99,201 @@ struct Gemm8 {
   int T, k, E, M, K, nrt;
 };
 
-template <int NMAT, int NT>
-__device__ __forceinline__ void w8_step(const W8 (&w)[2], const uint8_t* __restrict__ act,
-                                        const float* __restrict__ sums, int q, int l16,
-                                        gm_f32x4 (&acc)[2][2]) {
-  const bool low = q < 2;                                       // the lane's octet is in the first half
-#pragma unroll
-  for (int s = 0; s < 4; ++s) {
-    gm_f16x8 ah[NT], al[NT];
-    gm_f32x4 xs[NT];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      const int o = (16 * t + l16) * kRowB + 16 * ((4 * s + q) ^ l16);
-      ah[t] = *reinterpret_cast<const gm_f16x8*>(act + o);
-      al[t] = *reinterpret_cast<const gm_f16x8*>(act + kPlane + o);
-      xs[t] = *reinterpret_cast<const gm_f32x4*>(sums + s * kSeg + 16 * t + 4 * q);
-    }
-#pragma unroll
-    for (int n = 0; n < NMAT; ++n) {
-      uint32_t b[4];
-      i8x4_f16(w[n].q[s].x, b[0], b[1]);
-      i8x4_f16(w[n].q[s].y, b[2], b[3]);
-      const gm_u32x4 b0 = {low ? b[0] : 0u, low ? b[1] : 0u, low ? b[2] : 0u, low ? b[3] : 0u};
-      const gm_u32x4 b1 = {low ? 0u : b[0], low ? 0u : b[1], low ? 0u : b[2], low ? 0u : b[3]};
-      const gm_f16x8 B0 = __builtin_bit_cast(gm_f16x8, b0), B1 = __builtin_bit_cast(gm_f16x8, b1);
-      const float s0 = __uint_as_float(w[n].m[s].x), s1 = __uint_as_float(w[n].m[s].y),
-                  off = __uint_as_float(w[n].m[s].z);
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const gm_f32x4 z = {0.f, 0.f, 0.f, 0.f};
-        gm_f32x4 d0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[t], B0, z, 0, 0, 0);
-        gm_f32x4 d1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[t], B1, z, 0, 0, 0);
-        d0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[t], B0, d0, 0, 0, 0);
-        d1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[t], B1, d1, 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[n][t][i] += fmaf(s0, d0[i], fmaf(s1, d1[i], off * xs[t][i]));
-      }
-    }
+// Waits until at most n (0 .. 5 steps' worth) of the wave's loads are outstanding.
+template <int L>
+__device__ __forceinline__ void wait_steps(int n) {
+#define GM_VM(v) __builtin_amdgcn_s_waitcnt(((v) & 15) | ((v) >> 4) << 14 | 0xf70)
+  switch (n) {                                                  // uniform
+    case 0: GM_VM(0); break;
+    case 1: GM_VM(L); break;
+    case 2: GM_VM(2 * L); break;
+    case 3: GM_VM(3 * L); break;
+    case 4: GM_VM(4 * L); break;
+    default: GM_VM(5 * L); break;
   }
+#undef GM_VM
 }
 
-// Block = (segment, 64 weight rows): wave w rows 16 w .. 16 w + 15 of NMAT
-// matrices, all of the segment's tokens.  NMAT = 2: out = silu(gate) up; 1: out =
-// down row times the activation row's scale.  The next step's weights (registers)
-// and activation planes (straight into the other LDS buffer) load while a step is
-// multiplied.
-template <int NMAT>
-__global__ void __launch_bounds__(256, 2) k_pf8_gemm(Gemm8 P) {
-  __shared__ __attribute__((aligned(16))) uint8_t act[2][2 * kPlane];
-  __shared__ __attribute__((aligned(16))) float sums[2][4 * kSeg];
-  __shared__ int32_t in_row[kSeg], out_row[kSeg];
+// Block = (segment of at most 16 NT tokens, RTB tiles of 64 weight rows): wave w rows
+// 16 w .. 16 w + 15 of a tile of NMAT matrices, all of the segment's tokens.
+// NMAT = 2: out = silu(gate) up; 1: out = down row times the activation row's scale.
+//
+// Bound by the weights' way from HBM.  A step is 128 k (four sub-blocks); its
+// weights (into the wave's own LDS), activation planes and sums (into the block's)
+// come straight from global memory, NST - 1 steps ahead.  A load instruction
+// covers 5 1/3 weight rows of 192 contiguous bytes; loaded to registers as the MFMA
+// wants them, 16 rows by an instruction, they came at 2.3 TB/s whatever was in
+// flight (a probe of the two patterns alone: 3.1 and 6.9 TB/s).  Two buffers and
+// two or three blocks to a CU: one block with four or seven buffers (NST = 4 / 7)
+// had as much in flight but one wave per SIMD.
+// D = 2048, FF = 512, 256 experts, 150 tokens (Q5_K / Q6_K, 1.2 GB of I8 rows), us:
+//   gate/up 348 (16 rows an instruction) -> 270 (through LDS) -> 217 (a step's LDS
+//   reads together, the next loads not waited for before them); down 177 -> 123
+//   -> 111; 256 k a step: 316; one block of four buffers: 275 (down, seven: 184)
+// Granule g (16 bytes) of row r's step sits at position (g + 2 (r >> 2)) % 12 of
+// its 12: the 16 rows' reads of 32 bytes fall evenly on the banks.
+template <int NMAT, int NT, int RTB, int NST>
+__global__ void __launch_bounds__(256) k_pf8_gemm(Gemm8 P) {
+  constexpr int kStep = 128, kRowB = 2 * kStep, kWRow = 192, NW = 4;
+  constexpr int SEG = 16 * NT, PLANE = SEG * kRowB, NA = 2 * PLANE / 1024 / NW;   // act loads per wave and step
+  constexpr int WB = NMAT * 16 * kWRow;                         // a wave's weight bytes per step
+  constexpr int STAGE = 2 * PLANE + NW * WB + 4 * SEG * 4;      // planes, weights, sums [4][SEG]
+  constexpr int NL = 3 * NMAT + NA + 1;                         // loads per wave and step
+  static_assert(NL * (NST - 2) < 64 && NST - 2 <= 5, "vmcnt");
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];   // [NST][STAGE], then
+  int32_t* in_row = reinterpret_cast<int32_t*>(smem + NST * STAGE);  // [SEG]
+  int32_t* out_row = in_row + SEG;
   const int slot = blockIdx.x >> 3;                             // as xcd_tile of prefill.hip
   const int seg = (slot / P.nrt) * 8 + (blockIdx.x & 7), rt = slot % P.nrt;
   if (seg >= P.segs[0]) return;
   const int e = P.segs[1 + 4 * seg], start = P.segs[2 + 4 * seg], n = P.segs[3 + 4 * seg];
   const bool shared = e == P.E;
-  if (threadIdx.x < kSeg) {
-    const int c = threadIdx.x < n ? threadIdx.x : 0;            // rows past n repeat the first
+  if (threadIdx.x < SEG) {
+    const int c = (int)threadIdx.x < n ? threadIdx.x : 0;       // rows past n repeat the first
     const int pos = shared ? P.T * P.k + start + c : P.offsets[e] + start + c;
     in_row[threadIdx.x] = !P.sorted ? pos : shared ? start + c : P.sorted[pos] / P.k;
     out_row[threadIdx.x] = pos;
   }
   __syncthreads();
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, q = lane >> 4, l16 = lane & 15;
-  const int K = P.K, row = rt * 64 + wave * 16 + l16, nt = (n + 15) >> 4;
+  const int K = P.K, ns = K / kStep, total = RTB * ns, row0 = (rt * RTB * NW + wave) * 16;
   const int64_t rb = (int64_t)(K / 32) * 48;
-  const uint8_t* wr[NMAT];
+  const uint8_t* wp[NMAT];                                      // the wave's first row
+#pragma unroll
+  for (int i = 0; i < NMAT; ++i) wp[i] = (shared ? P.wsh[i] : P.w[i] + (int64_t)e * P.M * rb) + row0 * rb;
+  auto turn = [](int r) { return 2 * (r >> 2); };
+  int wo[3];                                                    // the lane's granules of a 16-row step
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    const int id = 64 * j + lane, r = id / 12;
+    wo[j] = r * (int)rb + 16 * ((id % 12 + 12 - turn(r)) % 12);
+  }
+  int qo[4], mo[4];                                             // where row l16's octet q and scales are
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    qo[s] = l16 * kWRow + 16 * ((3 * s + (q >> 1) + turn(l16)) % 12) + 8 * (q & 1);
+    mo[s] = l16 * kWRow + 16 * ((3 * s + 2 + turn(l16)) % 12);
+  }
+  // each wave brings 4 SEG / NW of a step's sums, one per lane
+  const int si = wave * SEG + (lane % SEG);
+  const float* sp = P.sums + (int64_t)in_row[si % SEG] * (K / 32) + si / SEG;
+  int ar[NA];                                                   // the lane's activation rows: 4 rows an instruction
+#pragma unroll
+  for (int m = 0; m < NA; ++m) ar[m] = in_row[4 * ((NA * wave + m) % (SEG / 4)) + (lane >> 4)];
+  float ds[NT][4];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) ds[t][i] = P.scale[in_row[16 * t + 4 * q + i]];
+  auto load = [&](int it, int b) {
+    const int tile = it / ns, s = it - tile * ns;
+    uint8_t* st = smem + b * STAGE;
+#pragma unroll
+    for (int i = 0; i < NMAT; ++i)
+#pragma unroll
+      for (int j = 0; j < 3; ++j)
+        to_lds<16>(wp[i] + (int64_t)tile * 16 * NW * rb + s * kWRow + wo[j],
+                   st + 2 * PLANE + wave * WB + i * 16 * kWRow + j * 1024);
+#pragma unroll
+    for (int m = 0; m < NA; ++m) {
+      const int id = NA * wave + m, pl = id / (SEG / 4), r4 = id % (SEG / 4), r = 4 * r4 + (lane >> 4);
+      to_lds<16>((pl ? P.lo : P.hi) + (int64_t)ar[m] * K + s * kStep + 8 * (l16 ^ (r & 15)),
+                 st + pl * PLANE + r4 * 1024);
+    }
+    if (lane < SEG) to_lds<4>(sp + s * 4, st + 2 * PLANE + NW * WB + wave * SEG * 4);
+  };
+  gm_f32x4 acc[NMAT][NT];
 #pragma unroll
   for (int i = 0; i < NMAT; ++i)
-    wr[i] = (shared ? P.wsh[i] : P.w[i] + (int64_t)e * P.M * rb) + row * rb;
-  const int tt = threadIdx.x & 31, ts = (threadIdx.x >> 5) & 3;  // this thread's activation sum (first 128)
-  const float* sp = P.sums + (int64_t)in_row[tt] * (K / 32) + ts;
-  auto load_act = [&](int step, int buf) {                      // 1 KB: 4 rows of one plane
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      const int id = 4 * m + wave, pl = id >> 3, r4 = id & 7;
-      if (r4 * 4 >= 16 * nt) continue;                          // wave-uniform
-      const int r = 4 * r4 + (lane >> 4), g = l16 ^ (r & 15);
-      __builtin_amdgcn_global_load_lds((pl ? P.lo : P.hi) + (int64_t)in_row[r] * K + step * kStep + 8 * g,
-                                       act[buf] + pl * kPlane + r4 * 1024, 16, 0, 0);
+    for (int t = 0; t < NT; ++t) acc[i][t] = gm_f32x4{0.f, 0.f, 0.f, 0.f};
+  __builtin_amdgcn_s_waitcnt(0);                                // every other load is in: only steps count below
+  const int ahead = total < NST - 1 ? total : NST - 1;
+  for (int i = 0; i < ahead; ++i) load(i, i);
+  const bool low = q < 2;                                       // the lane's octet is in the first half
+  for (int it = 0, b = 0; it < total; ++it, b = b + 1 < NST ? b + 1 : 0) {
+    const int rest = total - 1 - it;                            // steps after this one, NST - 2 of them on their way
+    wait_steps<NL>(rest < NST - 2 ? rest : NST - 2);
+    lds_barrier();                                              // everyone's part of step it; step it - 1 is done with
+    if (it + NST - 1 < total) load(it + NST - 1, b == 0 ? NST - 1 : b - 1);
+    const uint8_t* st = smem + b * STAGE;
+    const uint8_t* wb = st + 2 * PLANE + wave * WB;
+    const float* sums = reinterpret_cast<const float*>(st + 2 * PLANE + NW * WB);
+    constexpr int GS = NT == 1 ? 4 : 2;                         // sub-blocks whose LDS reads go out together
+#pragma unroll
+    for (int s0 = 0; s0 < 4; s0 += GS) {
+      gm_f16x8 ah[GS][NT], al[GS][NT];
+      gm_f32x4 xs[GS][NT], sc[GS][NMAT];                        // sc: s0, s1, off
+      gm_u32x2 w[GS][NMAT];
+#pragma unroll
+      for (int u = 0; u < GS; ++u) {
+        const int s = s0 + u;
+#pragma unroll
+        for (int i = 0; i < NMAT; ++i) {
+          w[u][i] = *reinterpret_cast<const gm_u32x2*>(wb + i * 16 * kWRow + qo[s]);
+          sc[u][i] = *reinterpret_cast<const gm_f32x4*>(wb + i * 16 * kWRow + mo[s]);
+        }
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          const int o = (16 * t + l16) * kRowB + 16 * ((4 * s + q) ^ l16);
+          ah[u][t] = *reinterpret_cast<const gm_f16x8*>(st + o);
+          al[u][t] = *reinterpret_cast<const gm_f16x8*>(st + PLANE + o);
+          xs[u][t] = *reinterpret_cast<const gm_f32x4*>(sums + s * SEG + 16 * t + 4 * q);
+        }
+      }
+      issue_fence();
+#pragma unroll
+      for (int u = 0; u < GS; ++u)
+#pragma unroll
+        for (int i = 0; i < NMAT; ++i) {
+          uint32_t o[4];
+          i8x4_f16(w[u][i].x, o[0], o[1]);
+          i8x4_f16(w[u][i].y, o[2], o[3]);
+          const gm_u32x4 b0 = {low ? o[0] : 0u, low ? o[1] : 0u, low ? o[2] : 0u, low ? o[3] : 0u};
+          const gm_u32x4 b1 = {low ? 0u : o[0], low ? 0u : o[1], low ? 0u : o[2], low ? 0u : o[3]};
+          const gm_f16x8 B0 = __builtin_bit_cast(gm_f16x8, b0), B1 = __builtin_bit_cast(gm_f16x8, b1);
+#pragma unroll
+          for (int t = 0; t < NT; ++t) {
+            const gm_f32x4 z = {0.f, 0.f, 0.f, 0.f};
+            gm_f32x4 d0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[u][t], B0, z, 0, 0, 0);
+            gm_f32x4 d1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[u][t], B1, z, 0, 0, 0);
+            d0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[u][t], B0, d0, 0, 0, 0);
+            d1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[u][t], B1, d1, 0, 0, 0);
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+              acc[i][t][c] += fmaf(sc[u][i].x, d0[c], fmaf(sc[u][i].y, d1[c], sc[u][i].z * xs[u][t][c]));
+          }
+        }
     }
-  };
-  gm_f32x4 acc[2][2];
+    if ((it + 1) % ns == 0) {
+      // a row tile is done: lane l holds tokens 4 (l / 16) + i of a token tile, weight row l % 16
+      const int row = row0 + (it / ns) * 16 * NW + l16;
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+      for (int t = 0; t < NT; ++t)
 #pragma unroll
-    for (int t = 0; t < 2; ++t) acc[i][t] = gm_f32x4{0.f, 0.f, 0.f, 0.f};
-  W8 w[2], wn[2];
-  load_act(0, 0);
+        for (int i = 0; i < 4; ++i) {
+          const int c = 16 * t + 4 * q + i;
+          if (c < n) {
+            float v = acc[0][t][i] * ds[t][i];
+            if constexpr (NMAT == 2) v = gm_silu(v) * (acc[NMAT - 1][t][i] * ds[t][i]);
+            P.out[(int64_t)out_row[c] * P.M + row] = v;
+          }
 #pragma unroll
-  for (int i = 0; i < NMAT; ++i) w[i] = w8_load(wr[i], 0, q);
-  if (threadIdx.x < 128) sums[0][ts * kSeg + tt] = sp[0];
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-  const int ns = K / kStep;
-  for (int s = 0; s < ns; ++s) {
-    const int sn = s + 1 < ns ? s + 1 : s, b = s & 1;           // the last step re-reads itself, unused
-#pragma unroll
-    for (int i = 0; i < NMAT; ++i) wn[i] = w8_load(wr[i], sn, q);
-    const float su = sp[sn * 4];
-    if (s + 1 < ns) load_act(sn, b ^ 1);
-    if (nt == 1) w8_step<NMAT, 1>(w, act[b], sums[b], q, l16, acc);
-    else w8_step<NMAT, 2>(w, act[b], sums[b], q, l16, acc);
-    if (threadIdx.x < 128) sums[b ^ 1][ts * kSeg + tt] = su;
-#pragma unroll
-    for (int i = 0; i < NMAT; ++i) w[i] = wn[i];
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
+          for (int m = 0; m < NMAT; ++m) acc[m][t][i] = 0.f;
+        }
+    }
   }
-  // lane l holds tokens 4 (l / 16) + i of a tile, weight row l % 16
-#pragma unroll
-  for (int t = 0; t < 2; ++t)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int c = 16 * t + 4 * q + i;
-      if (c >= n) continue;
-      const float ds = P.scale[in_row[c]];
-      float v = acc[0][t][i] * ds;
-      if constexpr (NMAT == 2) v = gm_silu(v) * (acc[1][t][i] * ds);
-      P.out[(int64_t)out_row[c] * P.M + row] = v;
-    }
+}
+
+template <int NMAT, int NT, int RTB, int NST>
+int launch8(Gemm8 P, int nseg, hipStream_t s) {
+  constexpr size_t smem = NST * (2 * 16 * NT * 256 + 4 * NMAT * 16 * 192 + 4 * 16 * NT * 4) + 2 * 16 * NT * 4;
+  static_assert(smem <= 160 * 1024, "LDS of a CU");
+  P.nrt = P.M / (64 * RTB);
+  if (int rc = gm_set_smem(k_pf8_gemm<NMAT, NT, RTB, NST>, smem)) return rc;
+  hipLaunchKernelGGL((k_pf8_gemm<NMAT, NT, RTB, NST>), dim3((unsigned)((nseg + 7) / 8 * 8 * P.nrt)), dim3(256), smem, s, P);
+  GM_TRY(hipGetLastError());
+  return GM_OK;
 }
 
 }  // namespace
@@ -241,7 +305,7 @@ int gm_pf8_split(const float* src, int rows, int K, const GmPf8Rows& a, hipStrea
 }
 
 int gm_pf8_gemm(const gm_moe_layer* L, bool down, const GmPf8Rows& a, const int32_t* segs, int nseg,
-                const int32_t* offsets, const int32_t* sorted, int T, float* out, hipStream_t s) {
+                const int32_t* offsets, const int32_t* sorted, int T, int seg_tok, float* out, hipStream_t s) {
   const int M = down ? L->D : L->FF, K = down ? L->FF : L->D;
   auto u8 = [](const void* p) { return static_cast<const uint8_t*>(p); };
   Gemm8 P{};
@@ -251,10 +315,10 @@ int gm_pf8_gemm(const gm_moe_layer* L, bool down, const GmPf8Rows& a, const int3
   P.wsh[1] = u8(down ? nullptr : L->up_sh);
   P.hi = a.hi; P.lo = a.lo; P.scale = a.scale; P.sums = a.sums;
   P.out = out; P.segs = segs; P.offsets = offsets; P.sorted = down ? nullptr : sorted;
-  P.T = T; P.k = L->k; P.E = L->E; P.M = M; P.K = K; P.nrt = M / 64;
-  const dim3 g((unsigned)((nseg + 7) / 8 * 8 * P.nrt));
-  if (down) hipLaunchKernelGGL(k_pf8_gemm<1>, g, dim3(256), 0, s, P);
-  else hipLaunchKernelGGL(k_pf8_gemm<2>, g, dim3(256), 0, s, P);
-  GM_TRY(hipGetLastError());
-  return GM_OK;
+  P.T = T; P.k = L->k; P.E = L->E; P.M = M; P.K = K;
+  // M % 256 == 0: whole tiles.  As many steps in flight as the LDS holds.
+  if (seg_tok == 16 && down) return launch8<1, 1, 4, 2>(P, nseg, s);
+  if (seg_tok == 16) return launch8<2, 1, 1, 2>(P, nseg, s);
+  if (down) return launch8<1, 2, 4, 2>(P, nseg, s);
+  return launch8<2, 2, 1, 2>(P, nseg, s);
 }
