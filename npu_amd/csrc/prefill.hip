@@ -13,10 +13,11 @@
 //      then dispatch (dispatch.hip):
 //      histogram -> exclusive scan -> stable scatter of (token, slot) pairs by
 //      expert, the inverse permutation, and every expert's token list (and the
-//      shared expert's, which takes all T tokens) cut into segments of <= kSegTok
+//      shared expert's, which takes all T tokens) cut into segments of <= 32
+//      or 64 (pf_seg)
 //   4. k_pf_gateup:   per (segment, 64 weight rows): h = silu(G x) * (U x).  The raw
-//                     superblocks are fetched one superblock ahead into registers
-//                     and decoded to f16 integers (kvalue or grid magnitude times
+//                     superblocks come through LDS, one superblock ahead, and are
+//                     decoded to f16 integers (kvalue or grid magnitude times
 //                     the integer part of the sub-block scale) straight into
 //                     v_mfma_f32_16x16x32_f16 operands; the superblock's fp16 d
 //                     multiplies the fp32 partial sum of each superblock.  The
@@ -24,7 +25,7 @@
 //                     stored as bf16 in expert-sorted row order.
 //   5. k_pf_h16:      every h row scaled by a power of two into f16's range and
 //                     converted exactly (the scale is kept per row)
-//   6. k_pf_down:     per (segment, 2 x 128 weight rows): y_pair = Down_e h on
+//   6. k_pf_down:     per (segment, 2 x 128 or 2 x 256 weight rows): y_pair = Down_e h on
 //                     v_mfma_f32_16x16x32_f16 with f16 integer weight operands as in
 //                     4, fp32 out times the row's h scale; the segment's h tile is
 //                     staged in LDS once per block
@@ -48,16 +49,7 @@ typedef float gm_f32x8 __attribute__((ext_vector_type(8)));
 
 namespace {
 
-// Tokens per segment.  32 (two MFMA column tiles) leaves the GEMM kernels at
-// 168 VGPRs, three waves per SIMD: config 4 227 -> 219 us per block against 64
-// tokens (four tiles, 2 waves per SIMD), although the 512-token shared unit
-// then decodes its weights for 16 segments instead of 8.
-constexpr int kSegTok = 32;
-constexpr int kNT = kSegTok / 16;   // MFMA column tiles per segment
-constexpr int kChunk = 256;         // K elements per pipeline step (one superblock column)
-constexpr int kRowB = 2 * kChunk;          // bytes per gate/up LDS activation row (f16, swizzled)
-constexpr int kTileG = kSegTok * kRowB;    // one gate/up activation buffer
-constexpr int kGran = kSegTok * (2 * kChunk / 16) / 256;  // 16-byte granules per thread of one chunk
+constexpr int kChunk = 256;         // K elements of a superblock
 
 // f(integral_constant<int, n>) for the segment's tile count n = ntiles in
 // [1, NT], as a chain of uniform branches (one instantiation per count).
@@ -112,7 +104,19 @@ int router_split(int D) { return D / router_krange(D); }
 // Row stride of the router partials: E rows + the shared gate row, padded to 4.
 int router_ld(const gm_moe_layer* L) { return (L->E + 1 + 3) & ~3; }
 
-int max_segments(int T, int k, int E, int seg = kSegTok) { return (T * k) / seg + E + (T + seg - 1) / seg + 1; }
+int max_segments(int T, int k, int E, int seg) { return (T * k) / seg + E + (T + seg - 1) / seg + 1; }
+
+// Tokens per segment of the IQ GEMMs.  Their kernels are bound by the decoding of
+// weights to f16, once per segment, so an expert's tokens should fit one; but a
+// segment of 64 halves the waves that a CU holds.  Block times at D = 2048, FF =
+// 512, E = 256, k = 8 (32 / 64): T = 512 192 / 213 us, 768 231 / 235, 1024 268 /
+// 257, 2048 437 / 381, 3072 612 / 523; at D = 512, FF = 256, E = 16, k = 4, where
+// 64 leaves CUs without a block: T = 768 45 / 50, 1280 56 / 55, 2048 72 / 67.
+constexpr int kSegMin = 32;
+int pf_seg(const gm_moe_layer* L, int T) {
+  const int64_t pairs = (int64_t)T * L->k;
+  return L->FF <= 2 * kChunk && pairs >= 28 * (int64_t)L->E && pairs / 64 * (L->FF / 64) >= 512 ? 64 : kSegMin;
+}
 
 // Tokens per segment of the I8 GEMMs: 16 while the experts have about that many
 // (one MFMA tile, two blocks to a CU), else 32.
@@ -127,7 +131,7 @@ PfWs pf_layout(const gm_moe_layer* L, int T, uint8_t* base, size_t* total) {
   w.offsets = reinterpret_cast<int32_t*>(take((E + 1) * 4));
   w.sorted = reinterpret_cast<int32_t*>(take(P * 4));
   w.inv = reinterpret_cast<int32_t*>(take(P * 4));
-  w.segs = reinterpret_cast<int32_t*>(take((1 + 4 * (size_t)max_segments(T, L->k, L->E)) * 4));
+  w.segs = reinterpret_cast<int32_t*>(take((1 + 4 * (size_t)max_segments(T, L->k, L->E, kSegMin)) * 4));
   w.rmsv = reinterpret_cast<float*>(take((size_t)T * 4));
   w.xh = reinterpret_cast<uint16_t*>(take((size_t)T * L->D * 2));
   w.xsc = reinterpret_cast<float*>(take((size_t)T * 4));
@@ -517,39 +521,38 @@ __device__ __forceinline__ PfRaw<QT> pf_load(const uint8_t* __restrict__ sb, int
   else return pf_load_iq3(sb, q);
 }
 
-// Sub-block scales of the lane's two sub-blocks (2q, 2q+1): the full scale
-// (bf16 path) or, for the f16 path, only its integer factor, with the
-// superblock factor pf_dscale applied to the fp32 accumulator instead:
+// Sub-block scales of the lane's two sub-blocks (2q, 2q+1): f16 weights hold only
+// the integer factor, and the superblock factor pf_dscale is applied to the fp32
+// partial sums:
 //   IQ4_XS: d * (ls - 32)            -> integer ls - 32 in [-32, 31], factor d
 //   IQ3_XXS: d * (0.5 + s4) * 0.5    -> integer 2 s4 + 1 in [1, 31], factor d / 4
 // so every f16 weight is an integer product, exact up to 2048 in magnitude:
 // |(2 s4 + 1) g| <= 1922 is always exact, |kv (ls - 32)| <= 4064 is rounded
 // once to f16's 11 significant bits when odd and above 2048; f16's small
 // exponent range never meets a tiny d.
+// The lane's integer scales as an f16 pair {sub-block 2q, 2q + 1} (exact: 0x6400 |
+// n is the f16 1024 + n) and the addends that go with them (u8x4_to_f16).
 template <int QT>
-__device__ __forceinline__ gm_f32x2 pf_scales(const PfRaw<QT>& r, int q) {
-  if constexpr (QT == GM_QTYPE_IQ4_XS) {
-    const float d = gm_h2f(r.h0 & 0xffffu);
-    const uint32_t sh = r.h0 >> 16, sl = (r.h1 >> (8 * q)) & 0xffu;
-    const int ls0 = (int)((sl & 15u) | (((sh >> (4 * q)) & 3u) << 4));
-    const int ls1 = (int)((sl >> 4) | (((sh >> (4 * q + 2)) & 3u) << 4));
-    return gm_f32x2{d * (float)(ls0 - 32), d * (float)(ls1 - 32)};
-  } else {
-    const float d = gm_h2f(r.d);
-    return gm_f32x2{d * (0.5f + (float)(r.w0 >> 28)) * 0.5f, d * (0.5f + (float)(r.w1 >> 28)) * 0.5f};
-  }
-}
+struct PfF16Scale {
+  gm_f16x2 s, c;
+  __device__ __forceinline__ gm_f16x2 sh(int h) const { return gm_f16x2{s[h], s[h]}; }
+  __device__ __forceinline__ gm_f16x2 ch(int h) const { return gm_f16x2{c[h], c[h]}; }
+};
 
 template <int QT>
-__device__ __forceinline__ gm_f32x2 pf_int_scales(const PfRaw<QT>& r, int q) {
+__device__ __forceinline__ PfF16Scale<QT> pf_f16_scales(const PfRaw<QT>& r, int q) {
+  PfF16Scale<QT> o;
   if constexpr (QT == GM_QTYPE_IQ4_XS) {
-    const uint32_t sh = r.h0 >> 16, sl = (r.h1 >> (8 * q)) & 0xffu;
-    const int ls0 = (int)((sl & 15u) | (((sh >> (4 * q)) & 3u) << 4));
-    const int ls1 = (int)((sl >> 4) | (((sh >> (4 * q + 2)) & 3u) << 4));
-    return gm_f32x2{(float)(ls0 - 32), (float)(ls1 - 32)};
+    const uint32_t sl = (r.h1 >> (8 * q)) & 0xffu, hi = r.h0 >> (16 + 4 * q);
+    const uint32_t n = (sl & 0x0fu) | (sl & 0xf0u) << 12 | (hi & 3u) << 4 | (hi & 12u) << 18;
+    o.s = __builtin_bit_cast(gm_f16x2, n | 0x64006400u) - gm_f16x2{(_Float16)1056.f, (_Float16)1056.f};
+    o.c = o.s * gm_f16x2{(_Float16)-1152.f, (_Float16)-1152.f};
   } else {
-    return gm_f32x2{(float)(2 * (r.w0 >> 28) + 1), (float)(2 * (r.w1 >> 28) + 1)};
+    const uint32_t n = (r.w0 >> 28) << 1 | (r.w1 >> 28) << 17 | 0x00010001u;
+    o.s = __builtin_bit_cast(gm_f16x2, n | 0x64006400u) - gm_f16x2{(_Float16)1024.f, (_Float16)1024.f};
+    o.c = o.s * gm_f16x2{(_Float16)-1024.f, (_Float16)-1024.f};
   }
+  return o;
 }
 
 template <int QT>
@@ -568,9 +571,10 @@ static_assert(gm_iq4_xor::check(kKvU, kKvUx), "XOR lookup of kvalues + 128");
 
 __device__ __forceinline__ uint32_t lut_kvu(uint32_t nib) { return gm_lut16_xor(kKvUx, nib); }
 
-// Four unsigned bytes u -> two f16x2 holding (u - 128) * s, rounded once:
-// 0x6400 | u is the f16 1024 + u, and fma(1024 + u, s, c) with c = -1152 s
-// (exact in f16 for |s| <= 32: 9 s 2^7) is (u - 128) s in one rounding.
+// Four unsigned bytes u -> two f16x2 holding (u - b) * s, rounded once (b = 128
+// for IQ4_XS, 0 for IQ3_XXS's magnitudes): 0x6400 | u is the f16 1024 + u, and
+// fma(1024 + u, s, c) with c = -(1024 + b) s (exact in f16 for |s| <= 32) is
+// (u - b) s in one rounding.
 __device__ __forceinline__ void u8x4_to_f16(uint32_t u, gm_f16x2 s, gm_f16x2 c, uint32_t& o0, uint32_t& o1) {
   const gm_f16x2 a = __builtin_bit_cast(gm_f16x2, __builtin_amdgcn_perm(0x64646464u, u, 0x04010400u));
   const gm_f16x2 b = __builtin_bit_cast(gm_f16x2, __builtin_amdgcn_perm(0x64646464u, u, 0x04030402u));
@@ -578,19 +582,17 @@ __device__ __forceinline__ void u8x4_to_f16(uint32_t u, gm_f16x2 s, gm_f16x2 c, 
   o1 = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(b, s, c));
 }
 
-// IQ3_XXS sign table for k-step decode: entry i (7-bit ksigns index) holds
-// byte masks (0x00 / 0xff) for the 8 signs of ksigns(i) and the same masks
-// & 0x01 per byte: {signs 0-3, signs 4-7, low bits 0-3, low bits 4-7}.
-__device__ __forceinline__ void pf_stage_signs_u8(gm_u32x4* tab) {
+// IQ3_XXS sign table for k-step decode: entry i (7-bit ksigns index) holds the
+// signs of ksigns(i) such that entry << p has those of weights 2p and 2p + 1 at
+// bits 15 and 31, where the f16 pair p has its own (one dword: a fourth of the
+// LDS traffic of byte masks for both halves).
+__device__ __forceinline__ void pf_stage_signs(uint32_t* tab) {
   for (int i = threadIdx.x; i < 128; i += blockDim.x) {
     const uint32_t s = gm_ksigns((uint32_t)i);
-    uint32_t m0 = 0, m1 = 0;
+    uint32_t m = 0;
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      m0 |= ((s >> b) & 1u) ? 0xffu << (8 * b) : 0u;
-      m1 |= ((s >> (b + 4)) & 1u) ? 0xffu << (8 * b) : 0u;
-    }
-    tab[i] = gm_u32x4{m0, m1, m0 & 0x01010101u, m1 & 0x01010101u};
+    for (int p = 0; p < 4; ++p) m |= ((s >> (2 * p)) & 1u) << (15 - p) | ((s >> (2 * p + 1)) & 1u) << (31 - p);
+    tab[i] = m;
   }
 }
 
@@ -602,7 +604,7 @@ __device__ __forceinline__ void pf_stage_signs_u8(gm_u32x4* tab) {
 template <int QT>
 __device__ __forceinline__ gm_f16x8 a_f16(const PfRaw<QT>& r, int j, gm_f16x2 sc, gm_f16x2 cc,
                                           const uint32_t* __restrict__ grid,
-                                          const gm_u32x4* __restrict__ sgn) {
+                                          const uint32_t* __restrict__ sgn) {
   uint32_t o[4];
   if constexpr (QT == GM_QTYPE_IQ4_XS) {
     const int sl = j >> 2, c = j & 3, sh = 4 * (c >> 1);
@@ -614,49 +616,42 @@ __device__ __forceinline__ gm_f16x8 a_f16(const PfRaw<QT>& r, int j, gm_f16x2 sc
     const uint32_t qw = r.q[2 * sl + (g >> 1)] >> (16 * (g & 1));
     const uint32_t ga = grid[qw & 0xffu], gb = grid[(qw >> 8) & 0xffu];
     const uint32_t w = sl ? r.w1 : r.w0;
-    const gm_u32x4 m = sgn[(w >> (7 * g)) & 127u];
-    // signed magnitude + 128 per byte: |v| <= 62, so no byte carries into the next
-    const uint32_t ua = ((ga ^ m.x) + m.z) ^ 0x80808080u;
-    const uint32_t ub = ((gb ^ m.y) + m.w) ^ 0x80808080u;
-    u8x4_to_f16(ua, sc, cc, o[0], o[1]);
-    u8x4_to_f16(ub, sc, cc, o[2], o[3]);
+    const uint32_t m = sgn[(w >> (7 * g)) & 127u];
+    u8x4_to_f16(ga, sc, cc, o[0], o[1]);               // the magnitudes times the scale, then their signs
+    u8x4_to_f16(gb, sc, cc, o[2], o[3]);
+#pragma unroll
+    for (int p = 0; p < 4; ++p) o[p] ^= (m << p) & 0x80008000u;
   }
   return __builtin_bit_cast(gm_f16x8, gm_u32x4{o[0], o[1], o[2], o[3]});
 }
 
-// B operand of k-step j from an LDS activation row: the 8 activations of the
-// lane's k-slots are contiguous, so one 16-byte read.
-__device__ __forceinline__ gm_u32x4 b_lds(const uint8_t* __restrict__ row, int q, int j) {
-  return *reinterpret_cast<const gm_u32x4*>(row + 2 * (32 * (2 * q + (j >> 2)) + 8 * (j & 3)));
-}
-
-// The same from row r of a gate/up activation tile, whose granule g (8 values)
-// of row r sits at slot g ^ (r & 15): the 16 rows a wave reads at once then hit
-// 16 different 16-byte bank groups without padding the 512-byte rows.
-__device__ __forceinline__ gm_u32x4 b_lds_swz(const uint8_t* __restrict__ tile, int r, int q, int j) {
-  const int g = 4 * (2 * q + (j >> 2)) + (j & 3);
-  return *reinterpret_cast<const gm_u32x4*>(tile + r * kRowB + 16 * (g ^ (r & 15)));
+// Activation rows in LDS: every 16-byte granule (8 values) g of row r at slot
+// g ^ (r & 15) of its row, so that the 16 rows a wave reads at once hit 16
+// different bank groups without padding.  The B operand of k-step j, the 8
+// activations of the lane's k-slots, is granule 4 (2q + (j >> 2)) + (j & 3) of a
+// superblock; a gate/up row holds NH-th parts of superblocks (NH = 2: the
+// k-steps of one half, granules 4q + (j & 3)).
+template <int ROWB>
+__device__ __forceinline__ gm_f16x8 b_lds(const uint8_t* tile, int r, int g) {
+  return __builtin_bit_cast(gm_f16x8, *reinterpret_cast<const gm_u32x4*>(tile + r * ROWB + 16 * (g ^ (r & 15))));
 }
 
 // Half H (k-steps 4H .. 4H+3) of one superblock column of the gate and up
 // rows against NT token tiles: f16 integer operands into the superblock's
 // partial sums pg / pu.
-template <int QT, int NT, int H>
-__device__ __forceinline__ void gu_half(const PfRaw<QT>& wg, const PfRaw<QT>& wu, int q, int l16,
-                                        const uint8_t* __restrict__ xb, const uint32_t* __restrict__ grid,
-                                        const gm_u32x4* __restrict__ sgn, gm_f32x4 (&pg)[kNT], gm_f32x4 (&pu)[kNT]) {
-  const gm_f32x2 sg2 = pf_int_scales<QT>(wg, q), su2 = pf_int_scales<QT>(wu, q);
-  const float sgf = H ? sg2.y : sg2.x, suf = H ? su2.y : su2.x;
-  const gm_f16x2 sgh = {(_Float16)sgf, (_Float16)sgf}, suh = {(_Float16)suf, (_Float16)suf};
-  const gm_f16x2 cgh = {(_Float16)(-1152.f * sgf), (_Float16)(-1152.f * sgf)};
-  const gm_f16x2 cuh = {(_Float16)(-1152.f * suf), (_Float16)(-1152.f * suf)};
+template <int QT, int NT, int NH, int H>
+__device__ __forceinline__ void gu_half(const PfRaw<QT>& wg, const PfRaw<QT>& wu, const PfF16Scale<QT>& sg,
+                                        const PfF16Scale<QT>& su, int q, int l16, const uint8_t* __restrict__ xb,
+                                        const uint32_t* __restrict__ grid, const uint32_t* __restrict__ sgn,
+                                        gm_f32x4 (&pg)[NT], gm_f32x4 (&pu)[NT]) {
 #pragma unroll
   for (int j = 4 * H; j < 4 * H + 4; ++j) {
-    const gm_f16x8 A = a_f16<QT>(wg, j, sgh, cgh, grid, sgn);
-    const gm_f16x8 U = a_f16<QT>(wu, j, suh, cuh, grid, sgn);
+    const gm_f16x8 A = a_f16<QT>(wg, j, sg.sh(H), sg.ch(H), grid, sgn);
+    const gm_f16x8 U = a_f16<QT>(wu, j, su.sh(H), su.ch(H), grid, sgn);
+    const int g = NH == 1 ? 4 * (2 * q + H) + (j & 3) : 4 * q + (j & 3);
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      const gm_f16x8 B = __builtin_bit_cast(gm_f16x8, b_lds_swz(xb, t * 16 + l16, q, j));
+      const gm_f16x8 B = b_lds<512 / NH>(xb, t * 16 + l16, g);
       pg[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, B, pg[t], 0, 0, 0);
       pu[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(U, B, pu[t], 0, 0, 0);
     }
@@ -664,61 +659,44 @@ __device__ __forceinline__ void gu_half(const PfRaw<QT>& wg, const PfRaw<QT>& wu
   }
 }
 
-// The superblock's partial sums times the superblock factor of each
-// accumulator row (rows 4q + i, whose factors lanes 4q + i hold) into ag / au.
-template <int QT, int NT>
-__device__ __forceinline__ void gu_fold(const PfRaw<QT>& wg, const PfRaw<QT>& wu, int q, const gm_f32x4 (&pg)[kNT],
-                                        const gm_f32x4 (&pu)[kNT], gm_f32x4 (&ag)[kNT], gm_f32x4 (&au)[kNT]) {
-  const float dgl = pf_dscale<QT>(wg), dul = pf_dscale<QT>(wu);
+// A superblock's partial sums times the superblock factor of each accumulator
+// row (rows 4q + i, whose factors lanes 4q + i hold) into acc.
+template <int NT>
+__device__ __forceinline__ void pf_fold(float d, int q, const gm_f32x4 (&p)[NT], gm_f32x4 (&acc)[NT]) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const float dg = __shfl(dgl, 4 * q + i, 64), du = __shfl(dul, 4 * q + i, 64);
+    const float di = __shfl(d, 4 * q + i, 64);
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      ag[t][i] = fmaf(dg, pg[t][i], ag[t][i]);
-      au[t][i] = fmaf(du, pu[t][i], au[t][i]);
-    }
+    for (int t = 0; t < NT; ++t) acc[t][i] = fmaf(di, p[t][i], acc[t][i]);
   }
 }
 
 // One superblock column of two down row tiles against NT token tiles: f16
 // integer operands into the superblock's partial sums, then the partial sums
 // times the superblock factor of each accumulator row into acc.
-template <int QT, int NT>
+template <int QT, int NT, int ROWB>
 __device__ __forceinline__ void dn_superblock(const PfRaw<QT>& w0, const PfRaw<QT>& w1, int q, int l16,
-                                              const uint8_t* __restrict__ hbuf, int pitch,
-                                              const uint32_t* __restrict__ grid, const gm_u32x4* __restrict__ sgn,
-                                              gm_f32x4 (&acc)[2][kNT]) {
-  const gm_f32x2 s0 = pf_int_scales<QT>(w0, q), s1 = pf_int_scales<QT>(w1, q);
+                                              const uint8_t* hbuf, const uint32_t* __restrict__ grid,
+                                              const uint32_t* __restrict__ sgn, gm_f32x4 (&a0)[NT],
+                                              gm_f32x4 (&a1)[NT]) {
+  const PfF16Scale<QT> s0 = pf_f16_scales<QT>(w0, q), s1 = pf_f16_scales<QT>(w1, q);
   gm_f32x4 p0[NT], p1[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) { p0[t] = gm_f32x4{0.f, 0.f, 0.f, 0.f}; p1[t] = p0[t]; }
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
-    const float f0 = j < 4 ? s0.x : s0.y, f1 = j < 4 ? s1.x : s1.y;
-    const gm_f16x2 h0 = {(_Float16)f0, (_Float16)f0}, h1 = {(_Float16)f1, (_Float16)f1};
-    const gm_f16x2 c0 = {(_Float16)(-1152.f * f0), (_Float16)(-1152.f * f0)};
-    const gm_f16x2 c1 = {(_Float16)(-1152.f * f1), (_Float16)(-1152.f * f1)};
-    const gm_f16x8 A0 = a_f16<QT>(w0, j, h0, c0, grid, sgn);
-    const gm_f16x8 A1 = a_f16<QT>(w1, j, h1, c1, grid, sgn);
+    const gm_f16x8 A0 = a_f16<QT>(w0, j, s0.sh(j >> 2), s0.ch(j >> 2), grid, sgn);
+    const gm_f16x8 A1 = a_f16<QT>(w1, j, s1.sh(j >> 2), s1.ch(j >> 2), grid, sgn);
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      const gm_f16x8 B = __builtin_bit_cast(gm_f16x8, b_lds(hbuf + (t * 16 + l16) * pitch, q, j));
+      const gm_f16x8 B = b_lds<ROWB>(hbuf, t * 16 + l16, 4 * (2 * q + (j >> 2)) + (j & 3));
       p0[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A0, B, p0[t], 0, 0, 0);
       p1[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A1, B, p1[t], 0, 0, 0);
     }
     if (j & 1) issue_fence();
   }
-  const float d0l = pf_dscale<QT>(w0), d1l = pf_dscale<QT>(w1);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float d0 = __shfl(d0l, 4 * q + i, 64), d1 = __shfl(d1l, 4 * q + i, 64);
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      acc[0][t][i] = fmaf(d0, p0[t][i], acc[0][t][i]);
-      acc[1][t][i] = fmaf(d1, p1[t][i], acc[1][t][i]);
-    }
-  }
+  pf_fold<NT>(pf_dscale<QT>(w0), q, p0, a0);
+  pf_fold<NT>(pf_dscale<QT>(w1), q, p1, a1);
 }
 
 // ------------------------------------------------------------- h to f16
@@ -775,63 +753,178 @@ __global__ void __launch_bounds__(256) k_pf_h16(const uint16_t* __restrict__ hb,
   if (lane == 0) hsc[r] = m <= 3.4e38f ? __builtin_ldexpf(1.0f, e) : __builtin_nanf("");
 }
 
-// Activation chunk [c0, c0 + 256) of the segment's rows <-> registers: kSegTok rows
-// x 32 granules of 16 B, granule g = threadIdx + 256 i for i in [I0, I0 + N)
-// (rows past n repeat a valid row; their output columns are never stored).
-template <int N>
-struct ActRegs { gm_u32x4 v[N]; };
+// ------------------------------------------------ weight rows through LDS
+// A wave load that takes 16 weight rows, as the A operands want them, asks for
+// about five times the cache lines whose bytes it uses (a probe of the pattern:
+// 3.1 TB/s, of contiguous runs 6.9).  So the lanes of a wave take consecutive
+// 16-byte granules of its rows straight into LDS of its own, one step ahead, and
+// read the operands from there.
 
+// 16 bytes per lane into LDS at dst (the wave's, uniform) + 16 lane.
+__device__ __forceinline__ void lds_load16(const void* src, uint8_t* dst) {
+  __builtin_amdgcn_global_load_lds(src, dst, 16, 0, 0);
+}
+
+// Every lane takes part in every load: under a lane condition the compiler may
+// merge two loads whose LDS destinations then differ between lanes.  Buffers are
+// of whole loads, and lanes past the data read its last granule again.
+
+// N consecutive granules (lane l of load j: granule 64 j + l) into LDS.
 template <int N>
-__device__ __forceinline__ void act_load(ActRegs<N>& a, const uint16_t* __restrict__ src, int K,
-                                         const int32_t* __restrict__ rows, int c0, int i0 = 0) {
+__device__ __forceinline__ void run_lds_load(const uint8_t* __restrict__ src, uint8_t* __restrict__ buf) {
+  const int lane = threadIdx.x & 63;
 #pragma unroll
-  for (int i = 0; i < N; ++i) {
-    const int g = threadIdx.x + 256 * (i0 + i), r = g >> 5, c = g & 31;
-    a.v[i] = *reinterpret_cast<const gm_u32x4*>(src + (int64_t)rows[r] * K + c0 + 8 * c);
+  for (int j = 0; j < (N + 63) / 64; ++j) {
+    const int g = 64 * j + lane;
+    lds_load16(src + 16 * (64 * j + 64 <= N ? g : min(g, N - 1)), buf + 1024 * j);
   }
 }
 
-template <int N>
-__device__ __forceinline__ void act_store(const ActRegs<N>& a, uint8_t* __restrict__ buf, int pitch, int i0 = 0) {
+// One superblock of 16 gate and 16 up IQ4_XS rows: 9 granules per row of 136
+// bytes, the last one 8 bytes early so that it ends with the superblock.
+constexpr int kIq4G = 9, kIq4Pitch = 16 * kIq4G, kIq4Tile = 16 * kIq4Pitch;
+constexpr int kIq4Loads = (2 * 16 * kIq4G + 63) / 64;
+
+// The lane's byte offsets of those granules from the gate tile (up = the up
+// tile's distance from it).
+__device__ __forceinline__ void iq4_offsets(int64_t up, int rb, int64_t (&off)[kIq4Loads]) {
 #pragma unroll
-  for (int i = 0; i < N; ++i) {
-    const int g = threadIdx.x + 256 * (i0 + i), r = g >> 5, c = g & 31;
-    *reinterpret_cast<gm_u32x4*>(buf + r * pitch + 16 * c) = a.v[i];
+  for (int j = 0; j < kIq4Loads; ++j) {
+    const int id = min(64 * j + (int)(threadIdx.x & 63), 2 * 16 * kIq4G - 1), r = id / kIq4G, g = id - r * kIq4G;
+    off[j] = (r < 16 ? 0 : up) + (r & 15) * rb + 16 * g - (g == 8 ? 8 : 0);
   }
 }
 
-// Chunk [c0, c0 + kChunk) of the segment's kSegTok f16 activation rows into the
-// swizzled tile with global -> LDS loads (no registers, no wait here): wave
-// instruction m of wave w writes 1 KB, rows 2 mi and 2 mi + 1 (mi = NI w + m);
-// lane i lands at slot i & 31 of row 2 mi + (i >> 5) and so loads granule
-// (i & 31) ^ (row & 15) of that row.
-__device__ __forceinline__ void act_lds_load(const uint16_t* __restrict__ src, int K,
-                                             const int32_t* __restrict__ rows, int c0, uint8_t* __restrict__ tile) {
-  constexpr int NI = kSegTok * (kRowB / 16) / 256;                     // 1 KB loads per wave
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+__device__ __forceinline__ void iq4_lds_load(const uint8_t* __restrict__ gate, const int64_t (&off)[kIq4Loads],
+                                             uint8_t* __restrict__ buf) {
 #pragma unroll
-  for (int m = 0; m < NI; ++m) {
-    const int mi = wave * NI + m, r = 2 * mi + (lane >> 5), c = (lane & 31) ^ (r & 15);
-    __builtin_amdgcn_global_load_lds(src + (int64_t)rows[r] * K + c0 + 8 * c, tile + mi * 1024, 16, 0, 0);
-  }
+  for (int j = 0; j < kIq4Loads; ++j) lds_load16(gate + off[j], buf + 1024 * j);
 }
+
+__device__ __forceinline__ PfRaw<GM_QTYPE_IQ4_XS> iq4_lds_read(const uint8_t* __restrict__ buf, int l16, int q) {
+  PfRaw<GM_QTYPE_IQ4_XS> r;
+  const uint8_t* p = buf + l16 * kIq4Pitch;
+  const gm_u32x2 h = *reinterpret_cast<const gm_u32x2*>(p);
+  r.h0 = h.x; r.h1 = h.y;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const gm_u32x2 v = *reinterpret_cast<const gm_u32x2*>(p + 8 + 32 * q + 8 * i + (i == 3 && q == 3 ? 8 : 0));
+    r.q[2 * i] = v.x; r.q[2 * i + 1] = v.y;
+  }
+  return r;
+}
+
+// Every LDS read issued so far has its data: what the reads took may be overwritten.
+__device__ __forceinline__ void lds_reads_done() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
 // -------------------------------------------------------------- gate/up
-// Block = (segment, 64 rows of FF); wave w -> rows 16w .. 16w+15 of both the
-// gate and the up matrix, all of the segment's token tiles.
-template <int QT>
-__global__ void __launch_bounds__(256, kSegTok == 64 ? 2 : 3) k_pf_gateup(gm_moe_layer P, const int32_t* __restrict__ segs,
-                                                      const int32_t* __restrict__ offsets,
-                                                      const int32_t* __restrict__ sorted,
-                                                      const uint16_t* __restrict__ xh,
-                                                      const float* __restrict__ xsc, uint16_t* __restrict__ hb,
-                                                      int T, int n_row_tiles) {
+// Block = (segment of at most ST tokens, 64 rows of FF); wave w -> rows 16w ..
+// 16w+15 of both the gate and the up matrix, all of the segment's token tiles.
+// A step is an NH-th part of a superblock: its activations are in one of two LDS
+// buffers, the next step's on their way to the other (halves: four blocks of 32
+// tokens to a CU, or two of 64).  At D = 2048, FF = 512, E = 256, k = 8 what bounds
+// it is near even at T = 512: loads and barriers alone take 87 us (the rows' 285 MB
+// at 3.3 TB/s and as many activation bytes from L2), decoding and MFMA alone 76,
+// together 97 (113 with 16 rows to a load and the rows held in registers); at
+// T = 4096, in segments of 64, 315 (416 in segments of 32, decoded twice as often).
+template <int QT, int ST, int NH>
+struct GuShape {
+  static constexpr int ROWB = 512 / NH, TILE = ST * ROWB;              // bytes of an activation row and buffer
+  static constexpr int G = ROWB / 16, NI = 16 * ROWB / 4096;           // granules per row, DMAs per wave and token tile
+  static constexpr int WBYTES = QT == GM_QTYPE_IQ4_XS ? 4 * kIq4Loads * 1024 : 256 * 4 + 128 * 4;   // rows' way / tables
+  static constexpr size_t SMEM = 2 * TILE + WBYTES + 2 * ST * 4;
+};
+
+// The next step's activations into the tile (no registers, no wait here): DMA
+// instruction m of wave w writes 1 KB, granules 64 (NI w + m) .. + 63 of it.
+template <int NI>
+__device__ __forceinline__ void act_lds_load(const uint16_t* const (&ptr)[NI], int off, uint8_t* __restrict__ tile) {
+#pragma unroll
+  for (int m = 0; m < NI; ++m)
+    lds_load16(ptr[m] + off, tile + ((threadIdx.x >> 6) * NI + m) * 1024);
+}
+
+// The K loop over NT token tiles.
+template <int QT, int ST, int NH, int NT>
+__device__ __forceinline__ void gu_loop(const uint8_t* __restrict__ gt, const uint8_t* __restrict__ ut, int64_t rb,
+                                        int nsb, const uint16_t* const (&xp)[NT * GuShape<QT, ST, NH>::NI],
+                                        uint8_t* __restrict__ xl, uint8_t* __restrict__ wbuf,
+                                        const uint32_t* __restrict__ grid, const uint32_t* __restrict__ sgn,
+                                        gm_f32x4 (&ag)[NT], gm_f32x4 (&au)[NT]) {
+  using S = GuShape<QT, ST, NH>;
+  constexpr bool IQ4 = QT == GM_QTYPE_IQ4_XS;
+  constexpr int SBB = IQ4 ? GM_IQ4XS_BYTES : GM_IQ3XXS_BYTES;
+  const int lane = threadIdx.x & 63, q = lane >> 4, l16 = lane & 15;
+#pragma unroll
+  for (int t = 0; t < NT; ++t) { ag[t] = gm_f32x4{0.f, 0.f, 0.f, 0.f}; au[t] = ag[t]; }
+  act_lds_load<NT * S::NI>(xp, 0, xl);
+  int64_t woff[kIq4Loads];
+  PfRaw<QT> wg, wu;
+  if constexpr (IQ4) {
+    iq4_offsets(ut - gt, (int)rb, woff);
+    iq4_lds_load(gt, woff, wbuf);
+  } else {
+    wg = pf_load<QT>(gt + l16 * rb, q);
+    wu = pf_load<QT>(ut + l16 * rb, q);
+  }
+  __builtin_amdgcn_s_waitcnt(0);                                        // the first step is in LDS
+  __syncthreads();
+  for (int sb = 0; sb < nsb; ++sb) {
+    // next superblock's rows and, straight into the other LDS buffer, the next
+    // activations (that buffer's last reader finished before the barrier)
+    const bool more = sb + 1 < nsb;
+    PfRaw<QT> wgn, wun;
+    if constexpr (IQ4) {
+      wg = iq4_lds_read(wbuf, l16, q);
+      wu = iq4_lds_read(wbuf + kIq4Tile, l16, q);
+      lds_reads_done();
+    }
+    uint8_t* const x0 = xl + (NH == 1 && (sb & 1) ? S::TILE : 0);
+    uint8_t* const x1 = xl + (NH == 1 && (sb & 1) ? 0 : S::TILE);
+    if (NH == 2) act_lds_load<NT * S::NI>(xp, sb * kChunk + 32, x1);
+    else if (more) act_lds_load<NT * S::NI>(xp, (sb + 1) * kChunk, x1);
+    if constexpr (IQ4) {
+      if (more) iq4_lds_load(gt + (sb + 1) * SBB, woff, wbuf);
+    } else {
+      const int sn = more ? sb + 1 : sb;                         // the last step re-reads itself
+      wgn = pf_load<QT>(gt + l16 * rb + sn * SBB, q);
+      wun = pf_load<QT>(ut + l16 * rb + sn * SBB, q);
+    }
+    const PfF16Scale<QT> sg = pf_f16_scales<QT>(wg, q), su = pf_f16_scales<QT>(wu, q);
+    gm_f32x4 pg[NT], pu[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) { pg[t] = gm_f32x4{0.f, 0.f, 0.f, 0.f}; pu[t] = pg[t]; }
+    gu_half<QT, NT, NH, 0>(wg, wu, sg, su, q, l16, x0, grid, sgn, pg, pu);
+    if constexpr (NH == 2) {
+      __builtin_amdgcn_s_waitcnt(0);
+      __syncthreads();
+      if (more) act_lds_load<NT * S::NI>(xp, (sb + 1) * kChunk, x0);
+    }
+    gu_half<QT, NT, NH, 1>(wg, wu, sg, su, q, l16, NH == 2 ? x1 : x0, grid, sgn, pg, pu);
+    pf_fold<NT>(pf_dscale<QT>(wg), q, pg, ag);
+    pf_fold<NT>(pf_dscale<QT>(wu), q, pu, au);
+    if constexpr (!IQ4) {
+      wg = wgn;
+      wu = wun;
+    }
+    __builtin_amdgcn_s_waitcnt(0);                                      // the next step is in LDS
+    __syncthreads();
+  }
+}
+
+template <int QT, int ST, int NH>
+__global__ void __launch_bounds__(256, ST == 32 ? 4 : 3) k_pf_gateup(
+    gm_moe_layer P, const int32_t* __restrict__ segs, const int32_t* __restrict__ offsets,
+    const int32_t* __restrict__ sorted, const uint16_t* __restrict__ xh, const float* __restrict__ xsc,
+    uint16_t* __restrict__ hb, int T, int n_row_tiles) {
+  using S = GuShape<QT, ST, NH>;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  uint8_t* xl = smem;                                                   // [2][kSegTok][kRowB]
-  uint32_t* grid = reinterpret_cast<uint32_t*>(smem + 2 * kTileG);      // [256] (IQ3)
-  gm_u32x4* sgn = reinterpret_cast<gm_u32x4*>(grid + 256);              // [128] (IQ3)
-  int32_t* tok_row = reinterpret_cast<int32_t*>(sgn + 128);             // [64]
-  int32_t* out_row = tok_row + kSegTok;                                 // [kSegTok]
+  uint8_t* xl = smem;                                                   // [2][ST][ROWB]
+  uint8_t* wl = smem + 2 * S::TILE;                                     // [4 waves][gate, up tile, padding] (IQ4)
+  uint32_t* grid = reinterpret_cast<uint32_t*>(wl);                     // [256] (IQ3)
+  uint32_t* sgn = grid + 256;                                           // [128] (IQ3)
+  int32_t* tok_row = reinterpret_cast<int32_t*>(wl + S::WBYTES);        // [ST]
+  int32_t* out_row = tok_row + ST;                                      // [ST]
   int seg, rt;
   xcd_tile(blockIdx.x, n_row_tiles, seg, rt);
   if (seg >= segs[0]) return;
@@ -840,9 +933,9 @@ __global__ void __launch_bounds__(256, kSegTok == 64 ? 2 : 3) k_pf_gateup(gm_moe
   const bool shared = e == E;
   if constexpr (QT == GM_QTYPE_IQ3_XXS) {
     gm_stage_grid(grid);
-    pf_stage_signs_u8(sgn);
+    pf_stage_signs(sgn);
   }
-  if (threadIdx.x < kSegTok) {
+  if (threadIdx.x < ST) {
     const int c = threadIdx.x;
     int tr = 0, orow = 0;
     if (c < n) {
@@ -856,76 +949,112 @@ __global__ void __launch_bounds__(256, kSegTok == 64 ? 2 : 3) k_pf_gateup(gm_moe
   }
   __syncthreads();
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, q = lane >> 4, l16 = lane & 15;
-  const int row = rt * 64 + wave * 16 + l16;
-  const int64_t rb = gm_row_bytes(QT, D);
+  const int64_t rb = gm_row_bytes(QT, D), tile = (int64_t)(rt * 64 + wave * 16) * rb;   // FF % 64 == 0: whole tiles
   const uint8_t* gbase = shared ? static_cast<const uint8_t*>(P.gate_sh)
                                 : static_cast<const uint8_t*>(P.gate_exps) + (int64_t)e * FF * rb;
   const uint8_t* ubase = shared ? static_cast<const uint8_t*>(P.up_sh)
                                 : static_cast<const uint8_t*>(P.up_exps) + (int64_t)e * FF * rb;
-  const uint8_t* grow = gbase + (int64_t)(row < FF ? row : 0) * rb;
-  const uint8_t* urow = ubase + (int64_t)(row < FF ? row : 0) * rb;
-  constexpr int SBB = QT == GM_QTYPE_IQ4_XS ? GM_IQ4XS_BYTES : GM_IQ3XXS_BYTES;
-  const int nsb = D / kChunk, ntiles = (n + 15) >> 4;
-  gm_f32x4 ag[kNT], au[kNT];
+  const int ntiles = (n + 15) >> 4, r0 = rt * 64 + wave * 16 + 4 * q;
+  nt_dispatch<ST / 16>(ntiles, [&](auto nt) {
+    constexpr int NT = decltype(nt)::value;
+    // lane i of DMA instruction m: slot s of row r, which holds granule s ^ (r & 15)
+    const uint16_t* xp[NT * S::NI];
 #pragma unroll
-  for (int t = 0; t < kNT; ++t) { ag[t] = gm_f32x4{0.f, 0.f, 0.f, 0.f}; au[t] = ag[t]; }
-  act_lds_load(xh, D, tok_row, 0, xl);
-  PfRaw<QT> wg = pf_load<QT>(grow, q), wu = pf_load<QT>(urow, q);
-  __builtin_amdgcn_s_waitcnt(0);                                        // the first chunk is in LDS
-  __syncthreads();
-  for (int sb = 0; sb < nsb; ++sb) {
-    // next superblock's raw rows and, straight into the other LDS buffer, its
-    // activation chunk (that buffer's last reader finished before the barrier)
-    const int sn = sb + 1 < nsb ? sb + 1 : sb;                   // the last step re-reads itself
-    const PfRaw<QT> wgn = pf_load<QT>(grow + sn * SBB, q), wun = pf_load<QT>(urow + sn * SBB, q);
-    const uint8_t* xb = xl + (sb & 1) * kTileG;
-    if (sb + 1 < nsb) act_lds_load(xh, D, tok_row, (sb + 1) * kChunk, xl + ((sb + 1) & 1) * kTileG);
-    gm_f32x4 pg[kNT], pu[kNT];
+    for (int m = 0; m < NT * S::NI; ++m) {
+      const int id = 64 * (wave * (NT * S::NI) + m) + lane, r = id / S::G, g = (id % S::G) ^ (r & 15);
+      xp[m] = xh + (int64_t)tok_row[r] * D + 8 * (NH == 1 ? g : 8 * (g >> 2) + (g & 3));
+    }
+    gm_f32x4 ag[NT], au[NT];
+    gu_loop<QT, ST, NH, NT>(gbase + tile, ubase + tile, rb, D / kChunk, xp, xl, wl + wave * kIq4Loads * 1024, grid, sgn, ag,
+                            au);
+    // C layout: lane l holds rows 4 (l / 16) + i of the 16-row tile, column l % 16
 #pragma unroll
-    for (int t = 0; t < kNT; ++t) { pg[t] = gm_f32x4{0.f, 0.f, 0.f, 0.f}; pu[t] = pg[t]; }
-    nt_dispatch<kNT>(ntiles, [&](auto nt) { gu_half<QT, decltype(nt)::value, 0>(wg, wu, q, l16, xb, grid, sgn, pg, pu); });
-    nt_dispatch<kNT>(ntiles, [&](auto nt) {
-      gu_half<QT, decltype(nt)::value, 1>(wg, wu, q, l16, xb, grid, sgn, pg, pu);
-      gu_fold<QT, decltype(nt)::value>(wg, wu, q, pg, pu, ag, au);
-    });
-    wg = wgn;
-    wu = wun;
-    __builtin_amdgcn_s_waitcnt(0);                                      // the next chunk is in LDS
-    __syncthreads();
-  }
-  // C layout: lane l holds rows 4 (l / 16) + i of the 16-row tile, column l % 16
-  const int r0 = rt * 64 + wave * 16 + 4 * q;
+    for (int t = 0; t < NT; ++t) {
+      const int col = t * 16 + l16;
+      if (col < n) {
+        const float ds = xsc[tok_row[col]];                      // the token's f16 scale, undone exactly
+        const gm_f32x4 g = ag[t] * ds, u = au[t] * ds;
+        gm_f32x2 h01 = {gm_silu(g[0]) * u[0], gm_silu(g[1]) * u[1]};
+        gm_f32x2 h23 = {gm_silu(g[2]) * u[2], gm_silu(g[3]) * u[3]};
+        *reinterpret_cast<uint2*>(hb + (int64_t)out_row[col] * FF + r0) =
+            make_uint2(__builtin_bit_cast(uint32_t, __builtin_convertvector(h01, gm_bf16x2)),
+                       __builtin_bit_cast(uint32_t, __builtin_convertvector(h23, gm_bf16x2)));
+      }
+    }
+  });
+}
+
+// ------------------------------------------------------------------ down
+// Block of NW waves = (segment of at most ST tokens, rg_per_blk groups of 32 NW
+// rows of D).  The segment's whole h tile (ST rows x FF, FF = 256 NSB) is staged
+// in LDS once; the block then walks its row groups with the next group's rows on
+// their way into LDS.  Wave w -> row tiles 2w, 2w+1 (16 rows each) of a group.
+// Bound by the LDS gathers of the decode tables and VALU work about evenly (54% and
+// 50% busy): 64 us at the sizes above and T = 512 (72 before), 230 at T = 4096 (295).
+// Segments of 64: eight waves, one block to a CU (its LDS holds no second one).
+// NSB is exact, three superblocks too (FF = 768 would else read past its rows).
+template <int QT, int NSB, int ST, int NW>
+struct DnShape {
+  static constexpr int SBB = QT == GM_QTYPE_IQ4_XS ? GM_IQ4XS_BYTES : GM_IQ3XXS_BYTES;
+  static constexpr int ROWB = NSB * 512, RUN = 2 * NSB * SBB;           // bytes of an h row, granules of a wave's rows
+  static constexpr int WBUF = (RUN + 63) / 64 * 1024;                   // their LDS buffer
+  static constexpr size_t SMEM = ST * (size_t)ROWB + 256 * 4 + 128 * 4 + ST * 4 + NW * WBUF;
+};
+
+template <int QT, int NSB, int ST, int NW, int NT>
+__device__ __forceinline__ void dn_loop(const uint8_t* __restrict__ wrows, int64_t rb, uint8_t* __restrict__ wbuf,
+                                        const uint8_t* hl, const uint32_t* __restrict__ grid,
+                                        const uint32_t* __restrict__ sgn, int g0, int g1, int n,
+                                        const float (&cs)[NT], float* __restrict__ yrow, int D) {
+  using S = DnShape<QT, NSB, ST, NW>;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, q = lane >> 4, l16 = lane & 15;
+  PfRaw<QT> wc[2][NSB];
+  auto take = [&]() {
 #pragma unroll
-  for (int t = 0; t < kNT; ++t) {
-    const int col = t * 16 + l16;
-    if (t < ntiles && col < n && r0 < FF) {
-      const float ds = xsc[tok_row[col]];                        // the token's f16 scale, undone exactly
-      const gm_f32x4 g = ag[t] * ds, u = au[t] * ds;
-      gm_f32x2 h01 = {gm_silu(g[0]) * u[0], gm_silu(g[1]) * u[1]};
-      gm_f32x2 h23 = {gm_silu(g[2]) * u[2], gm_silu(g[3]) * u[3]};
-      *reinterpret_cast<uint2*>(hb + (int64_t)out_row[col] * FF + r0) =
-          make_uint2(__builtin_bit_cast(uint32_t, __builtin_convertvector(h01, gm_bf16x2)),
-                     __builtin_bit_cast(uint32_t, __builtin_convertvector(h23, gm_bf16x2)));
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+      for (int sb = 0; sb < NSB; ++sb) wc[m][sb] = pf_load<QT>(wbuf + ((m * 16 + l16) * NSB + sb) * S::SBB, q);
+    lds_reads_done();
+  };
+  take();
+  for (int g = g0; g < g1; ++g) {
+    if (g + 1 < g1) run_lds_load<S::RUN>(wrows + (int64_t)(g + 1) * (32 * NW) * rb, wbuf);
+    gm_f32x4 acc[2][NT];
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[m][t] = gm_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int sb = 0; sb < NSB; ++sb)
+      dn_superblock<QT, NT, S::ROWB>(wc[0][sb], wc[1][sb], q, l16, hl + sb * 512, grid, sgn, acc[0], acc[1]);
+    if (g + 1 < g1) {                                  // before this group's stores, which need not be waited for
+      __builtin_amdgcn_s_waitcnt(0);
+      take();
+    }
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      const int r0 = g * (32 * NW) + wave * 32 + m * 16 + 4 * q;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const int col = t * 16 + l16;
+        if (col < n) *reinterpret_cast<gm_f32x4*>(yrow + (int64_t)col * D + r0) = acc[m][t] * cs[t];
+      }
     }
   }
 }
 
-// ------------------------------------------------------------------ down
-// Block = (segment, rg_per_blk groups of 128 rows of D).  The segment's whole
-// h tile (kSegTok rows x FF, FF = 256 NSB) is staged in LDS once; the block then
-// walks its row groups with the next group's raw superblocks in flight.
-// Wave w -> row tiles 2w, 2w+1 (16 rows each) of a group.
-template <int QT, int NSB>
-__global__ void __launch_bounds__(256, NSB == 4 ? 1 : (kSegTok == 64 || QT == GM_QTYPE_IQ4_XS ? 2 : 3)) k_pf_down(gm_moe_layer P, const int32_t* __restrict__ segs,
-                                                    const int32_t* __restrict__ offsets,
-                                                    const uint16_t* __restrict__ hh, const float* __restrict__ hsc,
-                                                    float* __restrict__ yp, int T, int n_blk, int rg_per_blk) {
-  constexpr int PITCH = NSB * 2 * kChunk + 16;                          // bytes per LDS h row
+template <int QT, int NSB, int ST, int NW>
+__global__ void __launch_bounds__(64 * NW, NSB > 2 ? 1 : 2) k_pf_down(gm_moe_layer P, const int32_t* __restrict__ segs,
+                                                     const int32_t* __restrict__ offsets,
+                                                     const uint16_t* __restrict__ hh, const float* __restrict__ hsc,
+                                                     float* __restrict__ yp, int T, int n_blk, int rg_per_blk) {
+  using S = DnShape<QT, NSB, ST, NW>;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  uint8_t* hl = smem;                                                   // [64][PITCH]
-  uint32_t* grid = reinterpret_cast<uint32_t*>(smem + kSegTok * PITCH);
-  gm_u32x4* sgn = reinterpret_cast<gm_u32x4*>(grid + 256);
-  int32_t* in_row = reinterpret_cast<int32_t*>(sgn + 128);
+  uint8_t* hl = smem;                                                   // [ST][ROWB]
+  uint32_t* grid = reinterpret_cast<uint32_t*>(smem + ST * S::ROWB);    // [256]
+  uint32_t* sgn = grid + 256;                                           // [128]
+  int32_t* in_row = reinterpret_cast<int32_t*>(sgn + 128);              // [ST]
+  uint8_t* wl = reinterpret_cast<uint8_t*>(in_row + ST);                // [NW waves][32 rows]
   int seg, bi;
   xcd_tile(blockIdx.x, n_blk, seg, bi);
   if (seg >= segs[0]) return;
@@ -935,72 +1064,59 @@ __global__ void __launch_bounds__(256, NSB == 4 ? 1 : (kSegTok == 64 || QT == GM
   const int row0 = shared ? T * k + start : offsets[e] + start;        // rows of hb / yp
   if constexpr (QT == GM_QTYPE_IQ3_XXS) {
     gm_stage_grid(grid);
-    pf_stage_signs_u8(sgn);
+    pf_stage_signs(sgn);
   }
-  if (threadIdx.x < kSegTok) in_row[threadIdx.x] = row0 + (threadIdx.x < n ? threadIdx.x : 0);
+  if (threadIdx.x < ST) in_row[threadIdx.x] = row0 + (threadIdx.x < n ? threadIdx.x : 0);
   __syncthreads();
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, q = lane >> 4, l16 = lane & 15;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l16 = lane & 15;
   const int64_t rb = gm_row_bytes(QT, FF);
-  const uint8_t* base = shared ? static_cast<const uint8_t*>(P.down_sh)
-                               : static_cast<const uint8_t*>(P.down_exps) + (int64_t)e * D * rb;
-  constexpr int SBB = QT == GM_QTYPE_IQ4_XS ? GM_IQ4XS_BYTES : GM_IQ3XXS_BYTES;
-  const int n_groups = (D + 127) / 128, g0 = bi * rg_per_blk;
+  const uint8_t* wrows = (shared ? static_cast<const uint8_t*>(P.down_sh)
+                                 : static_cast<const uint8_t*>(P.down_exps) + (int64_t)e * D * rb) +
+                         (int64_t)(wave * 32) * rb;
+  const int n_groups = (D + 32 * NW - 1) / (32 * NW), g0 = bi * rg_per_blk;    // D % 256 == 0: whole groups
   const int g1 = g0 + rg_per_blk < n_groups ? g0 + rg_per_blk : n_groups;
-  auto row_ptr = [&](int g, int m) {
-    const int row = g * 128 + wave * 32 + m * 16 + l16;
-    return base + (int64_t)(row < D ? row : 0) * rb;
-  };
-  PfRaw<QT> wc[2][NSB];
+  uint8_t* wbuf = wl + wave * S::WBUF;
+  run_lds_load<S::RUN>(wrows + (int64_t)g0 * (32 * NW) * rb, wbuf);
+  constexpr int G = S::ROWB / 16, NI = ST * G / (64 * NW);
+  const int used = ((n + 15) & ~15) * G - 64 * __builtin_amdgcn_readfirstlane(wave);   // granules of the tiles in use
 #pragma unroll
-  for (int m = 0; m < 2; ++m)
-#pragma unroll
-    for (int sb = 0; sb < NSB; ++sb) wc[m][sb] = pf_load<QT>(row_ptr(g0, m) + sb * SBB, q);
-#pragma unroll
-  for (int sb = 0; sb < NSB; ++sb) {
-    ActRegs<kGran> ha;
-    act_load<kGran>(ha, hh, FF, in_row, sb * kChunk);
-    act_store<kGran>(ha, hl + sb * 2 * kChunk, PITCH);
+  for (int m = 0; m < NI; ++m) {                       // h rows, swizzled as b_lds reads them
+    if (64 * NW * m >= used) break;
+    const int id = 64 * (NW * m + wave) + lane, r = id / G, g = (id % G) ^ (r & 15);
+    lds_load16(hh + (int64_t)in_row[r] * FF + 8 * g, hl + (NW * m + wave) * 1024);
   }
+  __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
-  const int ntiles = (n + 15) >> 4;
-  float cs[kNT];                                                        // h scale of each output column
+  nt_dispatch<ST / 16>((n + 15) >> 4, [&](auto nt) {
+    constexpr int NT = decltype(nt)::value;
+    float cs[NT];                                                       // h scale of each output column
 #pragma unroll
-  for (int t = 0; t < kNT; ++t) cs[t] = hsc[in_row[t * 16 + l16]];
-  for (int g = g0; g < g1; ++g) {
-    const int gn = g + 1 < g1 ? g + 1 : g;
-    PfRaw<QT> wn[2][NSB];
-#pragma unroll
-    for (int m = 0; m < 2; ++m)
-#pragma unroll
-      for (int sb = 0; sb < NSB; ++sb) wn[m][sb] = pf_load<QT>(row_ptr(gn, m) + sb * SBB, q);
-    gm_f32x4 acc[2][kNT];
-#pragma unroll
-    for (int m = 0; m < 2; ++m)
-#pragma unroll
-      for (int t = 0; t < kNT; ++t) acc[m][t] = gm_f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int sb = 0; sb < NSB; ++sb) {
-      const uint8_t* hbuf = hl + sb * 2 * kChunk;
-      nt_dispatch<kNT>(ntiles, [&](auto nt) {
-        dn_superblock<QT, decltype(nt)::value>(wc[0][sb], wc[1][sb], q, l16, hbuf, PITCH, grid, sgn, acc);
-      });
-    }
-#pragma unroll
-    for (int m = 0; m < 2; ++m) {
-      const int r0 = g * 128 + wave * 32 + m * 16 + 4 * q;
-#pragma unroll
-      for (int t = 0; t < kNT; ++t) {
-        const int col = t * 16 + l16;
-        if (t < ntiles && col < n && r0 < D)
-          *reinterpret_cast<gm_f32x4*>(yp + (int64_t)(row0 + col) * D + r0) =
-              gm_f32x4{acc[m][t][0] * cs[t], acc[m][t][1] * cs[t], acc[m][t][2] * cs[t], acc[m][t][3] * cs[t]};
-      }
-    }
-#pragma unroll
-    for (int m = 0; m < 2; ++m)
-#pragma unroll
-      for (int sb = 0; sb < NSB; ++sb) wc[m][sb] = wn[m][sb];
-  }
+    for (int t = 0; t < NT; ++t) cs[t] = hsc[in_row[t * 16 + l16]];
+    dn_loop<QT, NSB, ST, NW, NT>(wrows, rb, wbuf, hl, grid, sgn, g0, g1, n, cs, yp + (int64_t)row0 * D, D);
+  });
+}
+
+template <int QT, int ST, int NH>
+int launch_gateup(const gm_moe_layer* L, const PfWs& w, int nseg, int T, hipStream_t s) {
+  const int nrt = L->FF / 64;
+  constexpr size_t smem = GuShape<QT, ST, NH>::SMEM;
+  if (int rc = gm_set_smem(k_pf_gateup<QT, ST, NH>, smem)) return rc;
+  hipLaunchKernelGGL((k_pf_gateup<QT, ST, NH>), dim3((nseg + 7) / 8 * 8 * nrt), dim3(256), smem, s, *L, w.segs,
+                     w.offsets, w.sorted, w.xh, w.xsc, w.hb, T, nrt);
+  GM_TRY(hipGetLastError());
+  return GM_OK;
+}
+
+template <int QT, int NSB, int ST, int NW>
+int launch_down(const gm_moe_layer* L, const PfWs& w, int nseg, int T, hipStream_t s) {
+  constexpr int kGroupsPerBlock = 2;
+  const int n_blk = ((L->D + 32 * NW - 1) / (32 * NW) + kGroupsPerBlock - 1) / kGroupsPerBlock;
+  constexpr size_t smem = DnShape<QT, NSB, ST, NW>::SMEM;
+  if (int rc = gm_set_smem(k_pf_down<QT, NSB, ST, NW>, smem)) return rc;
+  hipLaunchKernelGGL((k_pf_down<QT, NSB, ST, NW>), dim3((nseg + 7) / 8 * 8 * n_blk), dim3(64 * NW), smem, s, *L,
+                     w.segs, w.offsets, w.hh, w.hsc, w.yp, T, n_blk, kGroupsPerBlock);
+  GM_TRY(hipGetLastError());
+  return GM_OK;
 }
 
 // --------------------------------------------------------------- combine
@@ -1259,8 +1375,6 @@ __global__ void __launch_bounds__(256) k_pfs_down_i8(const uint8_t* __restrict__
   }
 }
 
-constexpr size_t kGemmSmem = 2 * (size_t)kTileG + 256 * 4 + 128 * 16 + 2 * kSegTok * 4;
-
 // Steps 1-3: prep and router (xn32: also the fp32 rows xn, or NULL), top-k and
 // dispatch into segs (shared_T: tokens of the shared expert's own segments, or 0).
 int pf_route(const gm_moe_layer* L, const float* x, int T, uint8_t* ws, const GmMoeWs& lay, const PfWs& w,
@@ -1325,20 +1439,14 @@ int prefill_t(const gm_moe_layer* L, const float* x, float* y, int T, int flags,
                      L->q_down_sh == GM_QTYPE_I8;
   const bool sh_f32 = sh_apart && !sh_i8;
   const size_t P = (size_t)T * k;
-  if (int rc = pf_route(L, x, T, ws, lay, w, sh_f32 ? w.xn : nullptr, sh_gemm ? T : 0, w.segs, kSegTok, s)) return rc;
+  const int seg = pf_seg(L, T), nseg = max_segments(T, k, E, seg);
+  if (int rc = pf_route(L, x, T, ws, lay, w, sh_f32 ? w.xn : nullptr, sh_gemm ? T : 0, w.segs, seg, s)) return rc;
   if (sh_f32) {                                      // shared expert rows yp[P + t], fp32
     if (int rc = gm_launch_gateup(L->q_gate_sh, L->gate_sh, L->up_sh, FF, D, w.xn, T, w.hsh, s)) return rc;
     if (int rc = gm_launch_matvec(L->q_down_sh, L->down_sh, D, FF, w.hsh, T, w.yp + P * D, s)) return rc;
   }
-  const int nseg = max_segments(T, k, E);
-  {
-    const int nrt = FF / 64;
-    const int nb = (nseg + 7) / 8 * 8 * nrt;
-    if (int rc = gm_set_smem(k_pf_gateup<QTG>, kGemmSmem)) return rc;
-    hipLaunchKernelGGL(k_pf_gateup<QTG>, dim3(nb), dim3(256), kGemmSmem, s, *L, w.segs, w.offsets, w.sorted, w.xh,
-                       w.xsc, w.hb, T, nrt);
-    GM_TRY(hipGetLastError());
-  }
+  if (int rc = seg == 64 ? launch_gateup<QTG, 64, 2>(L, w, nseg, T, s) : launch_gateup<QTG, 32, 2>(L, w, nseg, T, s))
+    return rc;
   if (sh_i8) {                                       // shared SwiGLU rows hb[P + t] (D % 256 == 0)
     const int nkw = sh_kparts(D / 32), tok = 16 * kShTiles * (4 / nkw);    // tokens per block
     hipLaunchKernelGGL(k_pfs_gateup_i8, dim3(FF / 16, (T + tok - 1) / tok), dim3(256), 0, s,
@@ -1351,30 +1459,14 @@ int prefill_t(const gm_moe_layer* L, const float* x, float* y, int T, int flags,
     hipLaunchKernelGGL(k_pf_h16, dim3((rows + 3) / 4), dim3(256), 0, s, w.hb, rows, FF, w.hh, w.hsc);
     GM_TRY(hipGetLastError());
   }
-  {
-    constexpr int kGroupsPerBlock = 2;
-    const int n_blk = ((D + 127) / 128 + kGroupsPerBlock - 1) / kGroupsPerBlock;
-    const int nb = (nseg + 7) / 8 * 8 * n_blk;
-    const size_t smem = kSegTok * (2 * (size_t)FF + 16) + 256 * 4 + 128 * 16 + kSegTok * 4;
-    switch (FF / kChunk) {
-      case 1:
-        if (int rc = gm_set_smem(k_pf_down<QTD, 1>, smem)) return rc;
-        hipLaunchKernelGGL((k_pf_down<QTD, 1>), dim3(nb), dim3(256), smem, s, *L, w.segs, w.offsets, w.hh, w.hsc, w.yp,
-                           T, n_blk, kGroupsPerBlock);
-        break;
-      case 2:
-        if (int rc = gm_set_smem(k_pf_down<QTD, 2>, smem)) return rc;
-        hipLaunchKernelGGL((k_pf_down<QTD, 2>), dim3(nb), dim3(256), smem, s, *L, w.segs, w.offsets, w.hh, w.hsc, w.yp,
-                           T, n_blk, kGroupsPerBlock);
-        break;
-      default:
-        if (int rc = gm_set_smem(k_pf_down<QTD, 4>, smem)) return rc;
-        hipLaunchKernelGGL((k_pf_down<QTD, 4>), dim3(nb), dim3(256), smem, s, *L, w.segs, w.offsets, w.hh, w.hsc, w.yp,
-                           T, n_blk, kGroupsPerBlock);
-        break;
-    }
-    GM_TRY(hipGetLastError());
+  int rc;
+  switch (FF / kChunk) {
+    case 1: rc = seg == 64 ? launch_down<QTD, 1, 64, 8>(L, w, nseg, T, s) : launch_down<QTD, 1, 32, 4>(L, w, nseg, T, s); break;
+    case 2: rc = seg == 64 ? launch_down<QTD, 2, 64, 8>(L, w, nseg, T, s) : launch_down<QTD, 2, 32, 4>(L, w, nseg, T, s); break;
+    case 3: rc = launch_down<QTD, 3, 32, 4>(L, w, nseg, T, s); break;
+    default: rc = launch_down<QTD, 4, 32, 4>(L, w, nseg, T, s); break;
   }
+  if (rc) return rc;
   if (sh_i8) {                                       // shared expert rows yp[P + t] (FF % 256 == 0)
     const int nkw = sh_kparts(FF / 32), tok = 16 * kShTiles * (4 / nkw);
     hipLaunchKernelGGL(k_pfs_down_i8, dim3(D / 16, (T + tok - 1) / tok), dim3(256), 0, s,

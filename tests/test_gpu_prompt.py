@@ -183,3 +183,24 @@ def test_moe_i8_prompt_in_a_small_workspace(gpu):
     L.check(L.lib().gm_moe_forward_noalloc(ctypes.byref(blk.struct), L.ptr(x), L.ptr(y), T, 0, L.stream_ptr()), "noalloc")
     ref = blk(x).double()
     assert float((y.double() - ref).norm() / ref.norm()) <= 3e-6
+
+
+# ---- MoE blocks with IQ routed experts (prefill.hip)
+# segments of 64 tokens (many pairs per expert and enough of them to fill the chip) in every
+# format pair, with one row group per block (D = 256) and ragged last segments; the SwiGLU width
+# of three superblocks, in segments of 32
+@pytest.mark.parametrize("D,FF,E,k,T,q_gate,q_down", [
+    (512, 512, 16, 4, 1040, QT.IQ4_XS, QT.IQ3_XXS),
+    (256, 256, 8, 4, 2053, QT.IQ3_XXS, QT.IQ4_XS),
+    (1024, 512, 12, 8, 515, QT.IQ3_XXS, QT.IQ3_XXS),
+    (256, 512, 16, 8, 601, QT.IQ4_XS, QT.IQ4_XS),
+    (512, 768, 8, 2, 77, QT.IQ4_XS, QT.IQ3_XXS),
+    (256, 768, 8, 2, 40, QT.IQ3_XXS, QT.IQ4_XS),
+])
+def test_moe_iq_prompt_segments(gpu, D, FF, E, k, T, q_gate, q_down):
+    """Against the oracle, to the prefill tests' tolerance (f16 and bf16 operands: 2^-9 of a
+    product each, max-norm over a row of sums)."""
+    from npu_amd import synth
+    from test_gpu_prefill import _check
+    h = synth.host_moe_layer(400 + T, D=D, FF=FF, E=E, k=k, q_gate=q_gate, q_down=q_down, bias=True)
+    _check(gpu, h, T, seed=T)
