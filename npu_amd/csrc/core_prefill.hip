@@ -368,8 +368,12 @@ struct ConvHead {
   }
 };
 
-// One wave per (head, 16 tokens): heads [0, Hk) a K head's q and k rows and
-// their product, heads [Hk, Hk + Hv) a V head's row.  conv[t][C] as mixed.
+// One wave per (head, 16 tokens): heads [0, Hk) a K head's q and k rows and the
+// products that k_pf_delta needs of them, heads [Hk, Hk + Hv) a V head's row.
+// conv[t][C] as mixed; kq[t][head][kKq]: k_t . q_t, k_(t-i) . k_t and k_(t-i) . q_t
+// for i = 1 .. 3 (those that leave a group of 4 tokens are not read).
+constexpr int kKq = 8;
+
 template <int CL>
 __global__ void __launch_bounds__(256) k_pf_conv(const float* __restrict__ mixed, const float* __restrict__ w,
                                                  const float* __restrict__ state, int T, int ck, int Hk, int Hv,
@@ -397,12 +401,17 @@ __global__ void __launch_bounds__(256) k_pf_conv(const float* __restrict__ mixed
   qh.init(w, state, mixed, cq, ck, C, t0);
   kh.init(w, state, mixed, ckk, ck, C, t0);
   const float qs = 1.0f / sqrtf((float)Sk);
+  float kp[3][CL];                                              // k of the 3 tokens before, the newest first
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int u = 0; u < CL; ++u) kp[i][u] = 0.f;
 #pragma unroll 2
   for (int t = t0; t < t1; ++t) {
     float a[CL], b[CL];
     qh.step(t, a);
     kh.step(t, b);
-    float sa = 0.f, sb = 0.f, sp = 0.f;
+    float sa = 0.f, sb = 0.f, sp[7] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int u = 0; u < CL; ++u) { sa = fmaf(a[u], a[u], sa); sb = fmaf(b[u], b[u], sb); }
     const float ra = sqrtf(fmaxf(gm_wave_sum64(sa), eps)), rb = sqrtf(fmaxf(gm_wave_sum64(sb), eps));
@@ -410,12 +419,25 @@ __global__ void __launch_bounds__(256) k_pf_conv(const float* __restrict__ mixed
     for (int u = 0; u < CL; ++u) {
       a[u] = a[u] / ra * qs;
       b[u] = b[u] / rb;
-      sp = fmaf(a[u], b[u], sp);
+      sp[0] = fmaf(a[u], b[u], sp[0]);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        sp[1 + i] = fmaf(kp[i][u], b[u], sp[1 + i]);
+        sp[4 + i] = fmaf(kp[i][u], a[u], sp[4 + i]);
+      }
+      kp[2][u] = kp[1][u];
+      kp[1][u] = kp[0][u];
+      kp[0][u] = b[u];
       conv[(int64_t)t * C + cq + lane + 64 * u] = a[u];
       conv[(int64_t)t * C + ckk + lane + 64 * u] = b[u];
     }
-    sp = gm_wave_sum64(sp);
-    if (lane == 0) kq[(int64_t)t * Hk + hd] = sp;
+    float sl = 0.f;                                             // lane i < 7: product i
+#pragma unroll
+    for (int i = 0; i < 7; ++i) {
+      const float v = gm_wave_sum64(sp[i]);
+      sl = lane == i ? v : sl;
+    }
+    if (lane < 7) kq[((int64_t)t * Hk + hd) * kKq + lane] = sl;
   }
 }
 
@@ -427,11 +449,15 @@ constexpr int kDeltaTok = S <= 128 ? 16 : 8;
 // hold a column (S / 16 rows each, four consecutive ones per 64), 4 columns per
 // wave.  Per token, with the state s of the token before:
 //   d = (v - e (s . k)) beta,  o = e (s . q) + (k . q) d,  s = e s + k d
-// (o = s_new . q written out, so both dot products run on the old state and one
-// reduction stands between two tokens).  k, q, v and the scalars of 16 tokens
-// are staged in LDS two buffers deep; o leaves through LDS in 64-byte pieces.
-// The first blocks also write the new conv state (its old value was read by
-// the launch before).
+// Four tokens at a time: the dot products of all four run on the state before
+// them, and what the tokens between add to it, d_i k_i scaled by the e in
+// between, enters through the products k_i . k_j and k_i . q_j of k_pf_conv, so
+// one reduction over the 16 lanes stands between two groups.  1000 tokens of 32
+// heads of 128 x 128: 189 us (216 with a reduction between two tokens).  256 blocks:
+// a wave is alone on its SIMD, and its issue, an instruction every 5 to 6 cycles,
+// is the kernel's time.  k, q, v and the scalars of 16 tokens are staged in LDS two
+// buffers deep; o leaves through LDS in 64-byte pieces.  The first blocks also
+// write the new conv state (its old value was read by the launch before).
 template <int S>
 __global__ void __launch_bounds__(256) k_pf_delta(float* __restrict__ state, const float* __restrict__ conv,
                                                   const float* __restrict__ ab, const float* __restrict__ kq, int T,
@@ -442,7 +468,7 @@ __global__ void __launch_bounds__(256) k_pf_delta(float* __restrict__ state, con
   constexpr int TOK = kDeltaTok<S>;
   constexpr int NKQ = TOK * 2 * S / 4 / 256;                    // 16-byte loads of k and q per thread and stage
   __shared__ __attribute__((aligned(16))) float skq[2][TOK][2][S];
-  __shared__ __attribute__((aligned(16))) float sc[2][TOK][4];       // e, beta, k . q
+  __shared__ __attribute__((aligned(16))) float sc[2][TOK][12];      // e, beta, the products of k_pf_conv
   __shared__ float sv[2][TOK][16], so[2][TOK][16];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, p = lane & 15, q = lane >> 4;
   const int hv = blockIdx.x, c0 = blockIdx.y * 16, hk = hv % Hk, C = (2 * Hk + Hv) * S;
@@ -468,7 +494,7 @@ __global__ void __launch_bounds__(256) k_pf_delta(float* __restrict__ state, con
 
   gm_f32x4 rkq[NKQ];
   float rv, rs;
-  const int tv = threadIdx.x >> 4, cv = threadIdx.x & 15;       // tokens x 16 columns, scalars in cv < 3
+  const int tv = threadIdx.x >> 4, cv = threadIdx.x & 15;       // tokens x 16 columns, scalars in cv < 9
   auto load = [&](int t0) {                                     // tokens past T repeat the last one, unused
 #pragma unroll
     for (int i = 0; i < NKQ; ++i) {
@@ -478,14 +504,14 @@ __global__ void __launch_bounds__(256) k_pf_delta(float* __restrict__ state, con
     }
     const int64_t t = min(t0 + tv, T - 1);
     rv = conv[t * C + 2 * Hk * S + hv * S + c0 + cv];
-    rs = cv == 2 ? kq[t * Hk + hk] : ab[t * 2 * Hv + (cv == 1 ? Hv : 0) + hv];
+    rs = cv >= 2 ? kq[(t * Hk + hk) * kKq + (cv < 9 ? cv - 2 : 0)] : ab[t * 2 * Hv + (cv == 1 ? Hv : 0) + hv];
   };
   auto stage = [&](int b) {
 #pragma unroll
     for (int i = 0; i < NKQ; ++i) reinterpret_cast<gm_f32x4*>(skq[b])[threadIdx.x + 256 * i] = rkq[i];
     if (tv < TOK) {
       sv[b][tv][cv] = rv;
-      if (cv < 3) sc[b][tv][cv] = rs;
+      if (cv < 9) sc[b][tv][cv] = rs;
     }
   };
   load(0);
@@ -521,11 +547,71 @@ __global__ void __launch_bounds__(256) k_pf_delta(float* __restrict__ state, con
         for (int j = 0; j < 4; ++j) s[4 * i + j] = fmaf(kv[i][j], d, e.x * s[4 * i + j]);
       if (p == 0) so[b][t][cw] = fmaf(e.z, d, e.x * sq);
     };
+    auto step4 = [&](int t) {
+      gm_f32x4 kv[4][NI], qv[4][NI];
+      float e[4], beta[4], v[4], kq0[4], kk[4][3], kq[4][3];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+          kv[j][i] = *reinterpret_cast<const gm_f32x4*>(&skq[b][t + j][0][64 * i + 4 * p]);
+          qv[j][i] = *reinterpret_cast<const gm_f32x4*>(&skq[b][t + j][1][64 * i + 4 * p]);
+        }
+        const gm_f32x4* r = reinterpret_cast<const gm_f32x4*>(sc[b][t + j]);
+        const gm_f32x4 r0 = r[0], r1 = r[1];
+        e[j] = r0.x; beta[j] = r0.y; kq0[j] = r0.z;
+        kk[j][0] = r0.w; kk[j][1] = r1.x; kk[j][2] = r1.y;
+        kq[j][0] = r1.z; kq[j][1] = r1.w; kq[j][2] = sc[b][t + j][8];
+        v[j] = sv[b][t + j][cw];
+      }
+      float a[4], c[4];                                         // s . k_j and s . q_j
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        float as[NI], cs[NI];
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+          as[i] = s[4 * i] * kv[j][i].x;
+          cs[i] = s[4 * i] * qv[j][i].x;
+#pragma unroll
+          for (int u = 1; u < 4; ++u) {
+            as[i] = fmaf(s[4 * i + u], kv[j][i][u], as[i]);
+            cs[i] = fmaf(s[4 * i + u], qv[j][i][u], cs[i]);
+          }
+        }
+#pragma unroll
+        for (int i = 1; i < NI; ++i) { as[0] += as[i]; cs[0] += cs[i]; }
+        a[j] = gm_row_sum16(as[0]);
+        c[j] = gm_row_sum16(cs[0]);
+      }
+      float d[4], out = 0.f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        d[j] = (v[j] - e[j] * a[j]) * beta[j];
+        const float oj = fmaf(kq0[j], d[j], e[j] * c[j]);
+        out = (p & 3) == j ? oj : out;
+#pragma unroll
+        for (int l = j + 1; l < 4; ++l) {                       // token j's state under the later tokens
+          a[l] = fmaf(kk[l][l - j - 1], d[j], e[j] * a[l]);
+          c[l] = fmaf(kq[l][l - j - 1], d[j], e[j] * c[l]);
+        }
+      }
+      so[b][t + (p & 3)][cw] = out;                             // four lanes the same value: no branch in the chain
+      const float e23 = e[2] * e[3], e13 = e[1] * e23, e03 = e[0] * e13;
+      const float d0 = d[0] * e13, d1 = d[1] * e23, d2 = d[2] * e[3];
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          s[4 * i + u] = fmaf(kv[3][i][u], d[3],
+                              fmaf(kv[2][i][u], d2, fmaf(kv[1][i][u], d1, fmaf(kv[0][i][u], d0, e03 * s[4 * i + u]))));
+    };
     if (n == TOK) {                                             // unrolled: the next tokens' LDS reads run ahead
 #pragma unroll
-      for (int t = 0; t < TOK; ++t) step(t);
+      for (int t = 0; t < TOK; t += 4) step4(t);
     } else {
-      for (int t = 0; t < n; ++t) step(t);
+      int t = 0;
+      for (; t + 4 <= n; t += 4) step4(t);
+      for (; t < n; ++t) step(t);
     }
     stage(b ^ 1);
     __syncthreads();
@@ -594,7 +680,7 @@ SsmWs ssm_layout(const gm_ssm_layer* L, int T) {
   w.z = o; o = align256(o + Tz * di * 4);
   w.ab = o; o = align256(o + Tz * 2 * L->n_v_heads * 4);
   w.conv = o; o = align256(o + Tz * C * 4);
-  w.kq = o; o = align256(o + Tz * L->n_k_heads * 4);
+  w.kq = o; o = align256(o + Tz * L->n_k_heads * kKq * 4);
   w.o = o; o = align256(o + Tz * di * 4);
   w.total = o;
   return w;
