@@ -53,11 +53,11 @@ GmMoeWs gm_moe_ws_layout(const gm_moe_layer* L, int T) {
   w.yp = o; o = align256(o + (Td * k + Td) * (size_t)L->D * 4);
   w.pre = o; o = align256(o + gm_prefill_scratch_bytes(L, T));     // every T: gm_moe_prefill takes any T
   w.acc = o; o = align256(o + 2 * gm_acc_bytes(L->E));
-  const size_t b8 = T > GM_DECODE_MAX_T && gm_pf8_ok(L) ? align256(gm_pf8_scratch_bytes(L, T)) : 0;
-  w.pre8 = o; o += b8;
-  w.tl = o; o = align256(o + GM_TL_BYTES);                   // last: the timeline tool reads the end
+  w.tl = o; o = align256(o + GM_TL_BYTES);                   // the timeline tool reads the end at T <= 8
+  w.total_min = o;
+  // last, since a workspace may come without it
+  w.pre8 = o; o += T > GM_DECODE_MAX_T && gm_pf8_ok(L) ? align256(gm_pf8_scratch_bytes(L, T)) : 0;
   w.total = o;
-  w.total_min = o - b8;
   return w;
 }
 

@@ -87,10 +87,10 @@ struct GmMoeWs {
   size_t yp;       // f32 [T * k + T][D]  per-pair / shared partial outputs (decode, T > 1)
   size_t pre;      // prefill scratch (see prefill.hip)
   size_t acc;      // T = 1 router accumulators, two buffers of gm_acc_bytes(E) (moe_decode.h)
+  size_t tl;       // per-block timestamps (profiling build only, else empty)
+  size_t total_min;  // up to here: I8 layers then run T > GM_DECODE_MAX_T as decode chunks
   size_t pre8;     // prefill scratch of layers with I8 routed experts (T > GM_DECODE_MAX_T, else empty)
-  size_t tl;       // per-block timestamps (profiling build only, else empty); last region
   size_t total;
-  size_t total_min;  // without pre8: I8 layers then run T > GM_DECODE_MAX_T as decode chunks
 };
 
 // T = 1 router accumulators (layout in moe_decode.h): GM_ACC_COPIES copies of
