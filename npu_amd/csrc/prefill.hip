@@ -1489,11 +1489,13 @@ size_t gm_prefill_scratch_bytes(const gm_moe_layer* L, int T) {
 }
 
 // Layers whose routed experts (and shared expert, if any) are I8 rows, on the
-// GEMMs of prefill_i8.hip: fp32-exact activations, as their decode kernels have.
+// GEMMs of prefill_i8.hip: fp32-exact activations, as their decode kernels have,
+// and the widths that those take (the same layer in a smaller workspace runs on
+// them, and wider ones are refused there).
 bool gm_pf8_ok(const gm_moe_layer* L) {
   const bool sh = !L->gate_sh || (L->q_gate_sh == GM_QTYPE_I8 && L->q_down_sh == GM_QTYPE_I8);
   return L->q_gate == GM_QTYPE_I8 && L->q_down == GM_QTYPE_I8 && sh && L->D % kChunk == 0 && L->FF % kChunk == 0 &&
-         router_split(L->D) <= kRouterSplit;
+         L->D <= 4096 && L->FF <= 2048;                         // router_split <= kRouterSplit
 }
 
 struct Pf8Ws {

@@ -100,6 +100,24 @@ def test_workspace_sizing_and_layer_validation():
     assert rc == L.GM_EINVAL and "16-byte aligned" in L.last_error()
 
 
+@pytest.mark.parametrize("kw,ok", [(dict(D=4096, FF=256, FF_sh=256), True), (dict(D=256, FF=2048, FF_sh=2048), True),
+                                   (dict(D=4608, FF=256, FF_sh=256), False), (dict(D=256, FF=2304, FF_sh=2304), False)])
+def test_i8_prompts_take_the_widths_of_the_decode_kernels(kw, ok):
+    """A layer with I8 experts is as wide as its decode kernels take, whichever kernels its
+    tokens run on: wider ones have no scratch for the prompt GEMMs and are refused."""
+    lib = L.lib()
+    i8 = dict(q_gate=L.GM_QTYPE_I8, q_up=L.GM_QTYPE_I8, q_down=L.GM_QTYPE_I8, E=4, k=2)
+    s = _layer(**i8, **kw)
+    need = lib.gm_moe_workspace_bytes(ctypes.byref(s), 16)
+    assert need > 0
+    assert lib.gm_moe_prefill(ctypes.byref(s), 1 << 20, 1 << 21, 16, 0, 1 << 24, 256, None) == L.GM_EWORKSPACE
+    least = int(re.search(r"< (\d+) needed", L.last_error()).group(1))
+    assert (least < need) == ok
+    if not ok:
+        assert lib.gm_moe_prefill(ctypes.byref(s), 1 << 20, 1 << 21, 16, 0, 1 << 24, need, None) == L.GM_EINVAL
+        assert "D <= 4096 and FF <= 2048" in L.last_error()
+
+
 def test_chain_path_query_without_gpu():
     """gm_moe_chain_fused reports the accumulator-linked path (1) only at T = 1 and the
     combine-linked path (2) only at 2 <= T <= 8, decode shapes with D a multiple of 256 up to
