@@ -89,6 +89,43 @@ struct AttnP {
   float scale;
 };
 
+// Whether the wave's V tile (k_pf_attn) holds an infinity or NaN.
+template <int DV>
+__device__ __forceinline__ bool v_not_finite(const float* V, const int (&vo)[4]) {
+  bool odd = false;
+#pragma unroll
+  for (int g = 0; g < DV; ++g)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const gm_f32x4 v = *reinterpret_cast<const gm_f32x4*>(V + vo[i] + 64 * g);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) odd |= !(fabsf(v[c]) < __builtin_inff());
+    }
+  return __any(odd);
+}
+
+// A tile's part of 64 output dims of k_pf_attn without the MFMAs: each row adds
+// the keys up to its last one and never multiplies a later one.
+template <int Dh>
+__device__ __forceinline__ void v_masked(const float* V, int g, int key0, int last, const float (&p)[4],
+                                         gm_f32x4 (&w)[4]) {
+  const int lane = threadIdx.x & 63, l16 = lane & 15, q = lane >> 4;
+#pragma unroll 1
+  for (int k4 = 0; k4 < 4; ++k4)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int key = 4 * k4 + i;
+      const float pk = __shfl(p[i], 16 * k4 + l16, 64);
+      if (key0 + key > last) continue;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const gm_f32x4 v = *reinterpret_cast<const gm_f32x4*>(V + key * Dh + 4 * ((16 * g + 4 * q + e) ^ key));
+#pragma unroll
+        for (int c = 0; c < 4; ++c) w[c][e] = fmaf(pk, v[c], w[c][e]);
+      }
+    }
+}
+
 // Attention of 64 query rows (16 per wave) of one kv head over one part of
 // their keys, on v_mfma_f32_16x16x4_f32.  A kv head's rows are its T tokens x G
 // = Hq / Hkv heads, head fastest, so a block's rows span few positions and
@@ -124,6 +161,7 @@ __global__ void __launch_bounds__(256, DV <= 4 ? 2 : 1) k_pf_attn(AttnP P) {
   const int64_t ldq = (int64_t)(2 * P.Hq + 2 * P.Hkv) * Dh;
   const float* qrow = P.qkv + t * ldq + (int64_t)2 * Dh * h;
   const int last = P.pos0 + t;                                             // the row's last key
+  const int first = __builtin_amdgcn_readfirstlane(last);                  // the least of the wave's
   const int nkeys = P.pos0 + min((blk * 64 + 63) / G, P.T - 1) + 1;        // of the block
   const int ntile = (nkeys + 15) / 16, per = (ntile + P.nsplit - 1) / P.nsplit;
   const int i0 = split * per, i1 = min(i0 + per, ntile);
@@ -189,16 +227,23 @@ __global__ void __launch_bounds__(256, DV <= 4 ? 2 : 1) k_pf_attn(AttnP P) {
     for (int i = 0; i < 4; ++i) p[i] = expf(p[i] - mr);
     l = fmaf(l, a, (p[0] + p[1]) + (p[2] + p[3]));
     m = mn;
+    // a key that is masked for some of the wave's rows has probability 0 there, and
+    // 0 times a V value that is not finite would be NaN
+    const bool odd = it * 16 + 15 > first && v_not_finite<DV>(V, vo);
 #pragma unroll
     for (int g = 0; g < DV; ++g) {
       gm_f32x4 w[4];
 #pragma unroll
       for (int c = 0; c < 4; ++c) w[c] = gm_f32x4{0.f, 0.f, 0.f, 0.f};
+      if (!odd) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const gm_f32x4 v = *reinterpret_cast<const gm_f32x4*>(V + vo[i] + 64 * g);
+        for (int i = 0; i < 4; ++i) {
+          const gm_f32x4 v = *reinterpret_cast<const gm_f32x4*>(V + vo[i] + 64 * g);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) w[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[c], p[i], w[c], 0, 0, 0);
+          for (int c = 0; c < 4; ++c) w[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[c], p[i], w[c], 0, 0, 0);
+        }
+      } else {
+        v_masked<Dh>(V, g, it * 16, last, p, w);
       }
 #pragma unroll
       for (int c = 0; c < 4; ++c)

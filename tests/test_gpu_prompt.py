@@ -87,6 +87,36 @@ def test_attention_prompts(gpu, kw, parts):
     assert not nc.k[pos:].any()                            # nothing past the filled positions
 
 
+# eight, three and one row a position, on a cache whose keys are cut into parts and without one
+@pytest.mark.parametrize("kw,prefix", [(dict(n_head=8, n_head_kv=1, head_dim=256), 300),
+                                       (dict(n_head=6, n_head_kv=2, head_dim=64), 0),
+                                       (dict(n_head=2, n_head_kv=2, head_dim=128), 400)])
+def test_attention_prompt_non_finite_token(gpu, kw, prefix):
+    """A token with a NaN or infinity reaches itself and the tokens after it, as one token at a
+    time: the finite outputs are the same ones, with the same values to fp32 sums (2-norm)."""
+    from npu_amd import qwen_core as QN
+    print(f"attention non-finite case {kw} {prefix}", flush=True)
+    ocfg, ncfg = _cfgs(**kw)
+    NL = QN.AttnLayer(i=0, **_attn(ocfg, 33))
+    T = 61
+    cos, sin = QN.build_partial_rope_cache(ocfg.rope_dim, prefix + T, ocfg.rope_theta)
+    g = torch.Generator().manual_seed(34)
+    x = torch.randn(1, T, ocfg.d_model, generator=g)
+    x[0, 21, 5], x[0, 45, 7] = float("nan"), float("inf")
+    x = x.to(gpu)
+    caches = [QN.KVCache(ncfg, prefix + T) for _ in range(2)]
+    k, v = (torch.randn(prefix, ocfg.n_head_kv, ocfg.head_dim, generator=g).to(gpu) for _ in range(2))
+    for c in caches:
+        c.k[:prefix], c.v[:prefix], c.length = k, v, prefix
+    y, _ = QN.attn_forward(x, NL, ncfg, cos, sin, caches[0], prefix)
+    steps = [QN.attn_forward(x[:, t:t + 1], NL, ncfg, cos, sin, caches[1], prefix + t)[0] for t in range(T)]
+    ref = torch.cat(steps, 1)
+    assert torch.equal(y.isfinite(), ref.isfinite())
+    assert bool(y[0, :21].isfinite().all()) and not y[0, 21:].isfinite().any()
+    # each within 5e-7 of 64 bits
+    assert float((y[0, :21] - ref[0, :21]).double().norm() / ref[0, :21].double().norm()) <= 1e-6
+
+
 # d_state 64 / 128 / 256, prompts around the 16 staged tokens (8 at 256) and past the part of
 # 1024, conv kernels of 1, 2 and 8 taps, and a prompt shorter than the conv state
 @pytest.mark.parametrize("kw,parts", [
