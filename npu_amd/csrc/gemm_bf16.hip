@@ -29,6 +29,8 @@
 #include "bf16_split.h"
 #include "kernels.h"
 
+#include <type_traits>
+
 namespace {
 
 constexpr int kBK = 64;                       // k values per step (two 32-wide MFMA k-steps)
@@ -110,7 +112,8 @@ __global__ void __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) k_gemm_bf16(GemmArg
   load(min(s0, nstep - 1));
   stage(0);
   __syncthreads();
-  for (int i = 0; i < chunk; ++i) {
+  auto step = [&](int i, auto odd) {
+    constexpr Sign sign = step_sign(decltype(odd)::value);
     const int s = s0 + i;
     gm_f32x4 xc[CT][2][2];
 #pragma unroll
@@ -127,7 +130,7 @@ __global__ void __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) k_gemm_bf16(GemmArg
 #pragma unroll
       for (int c = 0; c < CT; ++c)
 #pragma unroll
-        for (int h = 0; h < 2; ++h) split3(xc[c][h][0], xc[c][h][1], pl[c][h]);
+        for (int h = 0; h < 2; ++h) split3(xc[c][h][0], xc[c][h][1], pl[c][h], sign);
       const bool half = s * kBK + 32 >= K;                      // K % 64 == 32: half a last step
       constexpr int RG = 2;                                     // row tiles at a time: two independent chains
 #pragma unroll
@@ -165,11 +168,15 @@ __global__ void __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) k_gemm_bf16(GemmArg
 #pragma unroll
         for (int r = 0; r < RG; ++r)
 #pragma unroll
-          for (int c = 0; c < CT; ++c) acc[r0 + r][c] += d[r][c];
+          for (int c = 0; c < CT; ++c) acc[r0 + r][c] += sign.f * d[r][c];
       }
     }
     if (more) stage((i + 1) & 1);
     __syncthreads();
+  };
+  for (int i = 0; i < chunk; i += 2) {                          // the signs as constants
+    step(i, std::integral_constant<int, 0>{});
+    if (i + 1 < chunk) step(i + 1, std::integral_constant<int, 1>{});
   }
   if constexpr (KS > 1) {                                       // K parts added in part order
     gm_f32x4* red = reinterpret_cast<gm_f32x4*>(smem);

@@ -295,8 +295,9 @@ __global__ void __launch_bounds__(64 * WPB) k_mv_bf16_mfma(const uint16_t* __res
     for (int c = 0; c < NC; c += NS) {
       gm_u32x4 pl[NS][3];
       gm_f32x4 d[RT];
+      const Sign sign = STEPS ? step_sign((c0 / 32 + c) / NS + wave) : Sign{0u, 1.f};
 #pragma unroll
-      for (int u = 0; u < NS; ++u) split3(xa[c + u], xb[c + u], pl[u]);
+      for (int u = 0; u < NS; ++u) split3(xa[c + u], xb[c + u], pl[u], sign);
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) d[rt] = STEPS ? gm_f32x4{0.f, 0.f, 0.f, 0.f} : acc[rt];
 #pragma unroll
@@ -308,7 +309,7 @@ __global__ void __launch_bounds__(64 * WPB) k_mv_bf16_mfma(const uint16_t* __res
             d[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gm_bf16x8, a[rt][c + u]),
                                                             __builtin_bit_cast(gm_bf16x8, pl[u][STEPS ? 2 - i : i]), d[rt], 0, 0, 0);
 #pragma unroll
-      for (int rt = 0; rt < RT; ++rt) acc[rt] = STEPS ? acc[rt] + d[rt] : d[rt];
+      for (int rt = 0; rt < RT; ++rt) acc[rt] = STEPS ? acc[rt] + sign.f * d[rt] : d[rt];
     }
   }
   if (wave > 0) {

@@ -30,6 +30,33 @@ def test_gemm_bf16_tiles(gpu, M, K, T):
     assert float((y - ref).norm() / ref.norm()) <= 1e-6
 
 
+# the three tile shapes, and the few-token kernel as the core layers' prompts run it
+@pytest.mark.parametrize("M,T", [(9216, 300), (9216, 120), (9216, 57), (1024, 12)])
+def test_bf16_products_unbiased(gpu, M, T):
+    """The mean error of a prompt's v rows against 64 bits, in units of their size: an attention
+    over them averages out everything else.  Rounding errors of either sign leave 1.2e-7 over
+    the root of their number (at most 1e-9 here); sums that all round down leave 2e-8 to 3e-8."""
+    from npu_amd import qwen_core as QN
+    print(f"gemm bias case M={M} T={T}", flush=True)
+    D, Hkv, Dh = 2048, 1, 256
+    cfg = QN.Config(d_model=D, n_head=(M - 2 * Hkv * Dh) // (2 * Dh), n_head_kv=Hkv, head_dim=Dh, rope_dim=0)
+    g = torch.Generator().manual_seed(M + T)
+    bf = lambda *s: (torch.randn(*s, generator=g) * 0.02).to(torch.bfloat16).float()
+    Hq = cfg.n_head
+    ones = torch.ones(Dh)
+    layer = QN.AttnLayer(i=0, attn_norm=torch.ones(D), post_norm=torch.ones(D), wq=bf(2 * Hq * Dh, D), wk=bf(Hkv * Dh, D),
+                         wv=bf(Hkv * Dh, D), wo=bf(D, Hq * Dh), q_norm=ones, k_norm=ones)
+    err, n, size = 0.0, 0, 0.0
+    for _ in range(max(1, 400 // T)):
+        x = torch.randn(1, T, D, generator=g)
+        _, c = QN.attn_forward(x.to(gpu), layer, cfg, torch.zeros(T, 0), torch.zeros(T, 0), None, 0)
+        xd = x[0].double()
+        ref = (xd * (xd.square().mean(1, keepdim=True) + cfg.rms_eps).rsqrt()) @ layer.wv.double().T
+        e = c.v[:T, 0].cpu().double() - ref
+        err, n, size = err + float(e.sum()), n + e.numel(), size + float(ref.square().sum())
+    assert abs(err / n) / (size / n) ** 0.5 <= 3e-9, err / n / (size / n) ** 0.5
+
+
 # ---- prompts through the core layers (gm_attn_prefill / gm_ssm_prefill)
 def _cfgs(**kw):
     from npu_amd import qwen_core as QN
