@@ -185,7 +185,7 @@ int gm_moe_forward(const gm_moe_layer* L, const float* x, float* y, int T, int f
  * qwen/forward.py:494-560 via _npu_routed_expert).  gm_moe_prefill: the
  * grouped f16/bf16-MFMA GEMMs for any T >= 1 (the reference runs prefill through
  * the CPU loop of qwen/forward.py:622-663).  A layer with I8 routed (and shared)
- * experts runs more than 8 tokens as grouped GEMMs of fp32-exact planes; a layer
+ * experts runs more than 8 tokens as grouped GEMMs on two f16 planes of x; a layer
  * with BF16 routed experts, or one with I8 and a workspace of less than
  * gm_moe_workspace_bytes (as large as it was without those planes), as decode
  * chunks of at most 8 tokens.  A shared

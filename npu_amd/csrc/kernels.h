@@ -158,8 +158,7 @@ int gm_pf8_run(const gm_moe_layer* L, const float* x, float* y, int T, int flags
 struct GmPf8Rows {
   uint16_t* hi;
   uint16_t* lo;
-  float* scale;    // per row: 2^-s of the rows held times 2^s
-  float* sums;     // per 32 values of a row
+  float* meta;     // per 32 values of a row: their sum times 2^s, and 2^-s (they are held times 2^s)
 };
 int gm_pf8_split(const float* src, int rows, int K, const GmPf8Rows& a, hipStream_t s);
 int gm_pf8_gemm(const gm_moe_layer* L, bool down, const GmPf8Rows& a, const int32_t* segs, int nseg,

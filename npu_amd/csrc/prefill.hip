@@ -1489,8 +1489,8 @@ size_t gm_prefill_scratch_bytes(const gm_moe_layer* L, int T) {
 }
 
 // Layers whose routed experts (and shared expert, if any) are I8 rows, on the
-// GEMMs of prefill_i8.hip: fp32-exact activations, as their decode kernels have,
-// and the widths that those take (the same layer in a smaller workspace runs on
+// GEMMs of prefill_i8.hip: activations to 2^-23 of each sub-block's largest, as
+// their decode kernels have, and the widths that those take (the same layer in a smaller workspace runs on
 // them, and wider ones are refused there).
 bool gm_pf8_ok(const gm_moe_layer* L) {
   const bool sh = !L->gate_sh || (L->q_gate_sh == GM_QTYPE_I8 && L->q_down_sh == GM_QTYPE_I8);
@@ -1512,10 +1512,9 @@ static Pf8Ws pf8_layout(const gm_moe_layer* L, int T, const PfWs& w, uint8_t* ba
   Pf8Ws v{};
   v.segs = reinterpret_cast<int32_t*>(take((1 + 4 * (size_t)max_segments(T, L->k, L->E, pf8_seg(L, T))) * 4));
   v.xn = reinterpret_cast<float*>(take(T * D * 4));
-  v.xr = GmPf8Rows{w.xh, reinterpret_cast<uint16_t*>(take(T * D * 2)), w.xsc,
-                   reinterpret_cast<float*>(take(T * (D / 32) * 4))};
+  v.xr = GmPf8Rows{w.xh, reinterpret_cast<uint16_t*>(take(T * D * 2)), reinterpret_cast<float*>(take(T * (D / 32) * 8))};
   v.h = reinterpret_cast<float*>(take((P + T) * FF * 4));
-  v.hr = GmPf8Rows{w.hh, w.hb, w.hsc, reinterpret_cast<float*>(take((P + T) * (FF / 32) * 4))};
+  v.hr = GmPf8Rows{w.hh, w.hb, reinterpret_cast<float*>(take((P + T) * (FF / 32) * 8))};
   if (total) *total = o;
   return v;
 }

@@ -1,15 +1,17 @@
 // Grouped GEMMs over routed experts held as I8 rows (Q8_0 / Q4_K / Q5_K / Q6_K
 // tensors, transcoded), for the MoE prefill (prefill.hip): segments of at
-// most 16 or 32 tokens per expert, with fp32-exact activations as the decode
+// most 16 or 32 tokens per expert, with activations no less exact than the decode
 // kernels of these layers have them.
 //
-// Activations: each row times a power of two (its largest magnitude in [2^14,
-// 2^15)), split into two f16 planes hi + lo (hi rounded, lo the rest rounded:
-// 2^-24 of each value, where the decode kernels' limbs keep 2^-23 of each
-// sub-block's largest), with the sum of every 32 values for the offsets.
+// Activations: each sub-block of 32 times a power of two (its largest magnitude in
+// [2^14, 2^15)), split into two f16 planes hi + lo (hi rounded, lo the rest
+// rounded): within 2^-23 of each value down to 2^-16 of the sub-block's largest,
+// within 2^-39 of that below; the decode kernels' limbs keep 2^-23 of the
+// sub-block's largest.  With them the sub-block's sum, for the offsets, and its
+// scale 2^-s.
 // Weights: int8 quants are exact in f16; the two scales and the offset of a
-// sub-block of 32 are applied in fp32 to its two half sums:
-//   y += s0 (q[0..15] . x) + s1 (q[16..31] . x) + off sum(x)
+// sub-block of 32 are applied in fp32 to its two half sums, then the activations':
+//   y += 2^-s (s0 (q[0..15] . x) + s1 (q[16..31] . x) + off sum(x))
 // v_mfma_f32_16x16x32_f16 with the tokens as A and the weight rows as B, so the
 // lane that decodes a row's quants also holds its scales for all its outputs;
 // the half sums come from B operands whose other half is zero.
@@ -20,48 +22,49 @@ using namespace gm_moe;
 
 typedef _Float16 gm_f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 gm_f16x2 __attribute__((ext_vector_type(2)));
+typedef float gm_f32x2 __attribute__((ext_vector_type(2)));
 
 namespace {
 
-// fp32 rows -> planes hi, lo, the row's scale 2^-s and the sums of 32 (of the
-// scaled values).  One wave per row; K % 256 == 0.
+// fp32 rows -> planes hi, lo and meta [row][K / 32][2]: the sum of a sub-block's
+// scaled values and its scale.  One wave per row, 8 lanes per sub-block; K % 256
+// == 0.  (One scale per row left a sub-block 2^-24 of the row's largest 15 bits.)
 __global__ void __launch_bounds__(256) k_pf8_split(const float* __restrict__ src, int rows, int K,
                                                    uint16_t* __restrict__ hi, uint16_t* __restrict__ lo,
-                                                   float* __restrict__ scale, float* __restrict__ sums) {
+                                                   float* __restrict__ meta) {
   const int r = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (r >= rows) return;
   const gm_f32x4* x = reinterpret_cast<const gm_f32x4*>(src + (int64_t)r * K);
-  float m = 0.f;
-#pragma unroll 8
-  for (int i = lane; i < K / 4; i += 64) {
-    const gm_f32x4 v = x[i];
-    m = fmaxf(m, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
-  const int sh = 15 - (m > 0.f && m <= 3.4e38f ? max(__builtin_amdgcn_frexp_expf(m), -100) : 0);
   uint2* ph = reinterpret_cast<uint2*>(hi + (int64_t)r * K);
   uint2* pl = reinterpret_cast<uint2*>(lo + (int64_t)r * K);
-#pragma unroll 4
-  for (int i = lane; i < K / 4; i += 64) {
-    const gm_f32x4 v = x[i];
-    _Float16 h[4], l[4];
-    float s = 0.f;
+  gm_f32x2* pm = reinterpret_cast<gm_f32x2*>(meta) + (int64_t)r * (K / 32);
+  const int n = K / 256;
+  constexpr int NL = 4;                                         // steps whose loads go out together
+  for (int s0 = 0; s0 < n; s0 += NL) {
+    gm_f32x4 v[NL];
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const float f = __builtin_ldexpf(v[c], sh);
-      h[c] = (_Float16)f;
-      l[c] = (_Float16)(f - (float)h[c]);
-      s += f;
+    for (int u = 0; u < NL; ++u) v[u] = x[64 * min(s0 + u, n - 1) + lane];
+#pragma unroll
+    for (int u = 0; u < NL; ++u) {
+      if (s0 + u >= n) break;                                   // uniform
+      const int i = 64 * (s0 + u) + lane;
+      const float m = gm_max8(fmaxf(fmaxf(fabsf(v[u].x), fabsf(v[u].y)), fmaxf(fabsf(v[u].z), fabsf(v[u].w))));
+      const int sh = 15 - (m > 0.f && m <= 3.4e38f ? max(__builtin_amdgcn_frexp_expf(m), -100) : 0);
+      _Float16 h[4], l[4];
+      float f[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        f[c] = __builtin_ldexpf(v[u][c], sh);
+        h[c] = (_Float16)f[c];
+        l[c] = (_Float16)(f[c] - (float)h[c]);
+      }
+      const gm_f16x2 h01 = {h[0], h[1]}, h23 = {h[2], h[3]}, l01 = {l[0], l[1]}, l23 = {l[2], l[3]};
+      ph[i] = make_uint2(__builtin_bit_cast(uint32_t, h01), __builtin_bit_cast(uint32_t, h23));
+      pl[i] = make_uint2(__builtin_bit_cast(uint32_t, l01), __builtin_bit_cast(uint32_t, l23));
+      const float s = gm_sum8((f[0] + f[1]) + (f[2] + f[3]));
+      if ((lane & 7) == 0) pm[i / 8] = gm_f32x2{s, __builtin_ldexpf(1.0f, -sh)};
     }
-    const gm_f16x2 h01 = {h[0], h[1]}, h23 = {h[2], h[3]}, l01 = {l[0], l[1]}, l23 = {l[2], l[3]};
-    ph[i] = make_uint2(__builtin_bit_cast(uint32_t, h01), __builtin_bit_cast(uint32_t, h23));
-    pl[i] = make_uint2(__builtin_bit_cast(uint32_t, l01), __builtin_bit_cast(uint32_t, l23));
-#pragma unroll
-    for (int o = 1; o < 8; o <<= 1) s += __shfl_xor(s, o, 64);
-    if ((lane & 7) == 0) sums[(int64_t)r * (K / 32) + i / 8] = s;
   }
-  if (lane == 0) scale[r] = __builtin_ldexpf(1.0f, -sh);
 }
 
 // Four int8 -> f16: 0x6400 | (b ^ 0x80) is 1024 + 128 + b, exactly.
@@ -90,8 +93,7 @@ struct Gemm8 {
   const uint8_t* wsh[2];   // the shared expert's rows, or NULL
   const uint16_t* hi;      // activation rows [.][K]
   const uint16_t* lo;
-  const float* scale;
-  const float* sums;       // [.][K / 32]
+  const float* meta;       // [.][K / 32][2]: sum, scale
   float* out;              // [P + T][M]
   const int32_t* segs;
   const int32_t* offsets;
@@ -99,49 +101,35 @@ struct Gemm8 {
   int T, k, E, M, K, nrt;
 };
 
-// Waits until at most n (0 .. 5 steps' worth) of the wave's loads are outstanding.
-template <int L>
-__device__ __forceinline__ void wait_steps(int n) {
-#define GM_VM(v) __builtin_amdgcn_s_waitcnt(((v) & 15) | ((v) >> 4) << 14 | 0xf70)
-  switch (n) {                                                  // uniform
-    case 0: GM_VM(0); break;
-    case 1: GM_VM(L); break;
-    case 2: GM_VM(2 * L); break;
-    case 3: GM_VM(3 * L); break;
-    case 4: GM_VM(4 * L); break;
-    default: GM_VM(5 * L); break;
-  }
-#undef GM_VM
-}
-
 // Block = (segment of at most 16 NT tokens, RTB tiles of 64 weight rows): wave w rows
 // 16 w .. 16 w + 15 of a tile of NMAT matrices, all of the segment's tokens.
-// NMAT = 2: out = silu(gate) up; 1: out = down row times the activation row's scale.
+// NMAT = 2: out = silu(gate) up; 1: out = the down row.
 //
 // Bound by the weights' way from HBM.  A step is 128 k (four sub-blocks); its
-// weights (into the wave's own LDS), activation planes and sums (into the block's)
-// come straight from global memory, NST - 1 steps ahead.  A load instruction
+// weights (into the wave's own LDS), activation planes, sums and scales (into the
+// block's) come straight from global memory, one step ahead.  A load instruction
 // covers 5 1/3 weight rows of 192 contiguous bytes; loaded to registers as the MFMA
 // wants them, 16 rows by an instruction, they came at 2.3 TB/s whatever was in
 // flight (a probe of the two patterns alone: 3.1 and 6.9 TB/s).  Two buffers and
-// two or three blocks to a CU: one block with four or seven buffers (NST = 4 / 7)
-// had as much in flight but one wave per SIMD.
+// two (gate/up) or three (down) blocks of 16 tokens to a CU: one block with four or
+// seven buffers had as much in flight but one wave per SIMD.  A gate/up block of 32
+// tokens is alone on its CU, two of them do not fit its LDS.
 // D = 2048, FF = 512, 256 experts, 150 tokens (Q5_K / Q6_K, 1.2 GB of I8 rows), us:
 //   gate/up 348 (16 rows an instruction) -> 270 (through LDS) -> 217 (a step's LDS
 //   reads together, the next loads not waited for before them); down 177 -> 123
 //   -> 111; 256 k a step: 316; one block of four buffers: 275 (down, seven: 184)
+// Kernel durations with one scale per activation row 198 and 103, per sub-block 192
+// and 101 (the activations' addresses are formed once, not per step).
 // Granule g (16 bytes) of row r's step sits at position (g + 2 (r >> 2)) % 12 of
 // its 12: the 16 rows' reads of 32 bytes fall evenly on the banks.
-template <int NMAT, int NT, int RTB, int NST>
+template <int NMAT, int NT, int RTB>
 __global__ void __launch_bounds__(256) k_pf8_gemm(Gemm8 P) {
   constexpr int kStep = 128, kRowB = 2 * kStep, kWRow = 192, NW = 4;
   constexpr int SEG = 16 * NT, PLANE = SEG * kRowB, NA = 2 * PLANE / 1024 / NW;   // act loads per wave and step
   constexpr int WB = NMAT * 16 * kWRow;                         // a wave's weight bytes per step
-  constexpr int STAGE = 2 * PLANE + NW * WB + 4 * SEG * 4;      // planes, weights, sums [4][SEG]
-  constexpr int NL = 3 * NMAT + NA + 1;                         // loads per wave and step
-  static_assert(NL * (NST - 2) < 64 && NST - 2 <= 5, "vmcnt");
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];   // [NST][STAGE], then
-  int32_t* in_row = reinterpret_cast<int32_t*>(smem + NST * STAGE);  // [SEG]
+  constexpr int STAGE = 2 * PLANE + NW * WB + 8 * SEG * 4;      // planes, weights, meta [4][sum, scale][SEG]
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];   // [2][STAGE], then
+  int32_t* in_row = reinterpret_cast<int32_t*>(smem + 2 * STAGE);  // [SEG]
   int32_t* out_row = in_row + SEG;
   const int slot = blockIdx.x >> 3;                             // as xcd_tile of prefill.hip
   const int seg = (slot / P.nrt) * 8 + (blockIdx.x & 7), rt = slot % P.nrt;
@@ -174,17 +162,17 @@ __global__ void __launch_bounds__(256) k_pf8_gemm(Gemm8 P) {
     qo[s] = l16 * kWRow + 16 * ((3 * s + (q >> 1) + turn(l16)) % 12) + 8 * (q & 1);
     mo[s] = l16 * kWRow + 16 * ((3 * s + 2 + turn(l16)) % 12);
   }
-  // each wave brings 4 SEG / NW of a step's sums, one per lane
-  const int si = wave * SEG + (lane % SEG);
-  const float* sp = P.sums + (int64_t)in_row[si % SEG] * (K / 32) + si / SEG;
-  int ar[NA];                                                   // the lane's activation rows: 4 rows an instruction
+  // a step's 8 SEG sums and scales, one per lane of the first SEG / 8 waves (all their
+  // lanes: see lds_load16 of prefill.hip)
+  const int mi = 64 * wave + lane;
+  const float* mp = P.meta + ((int64_t)in_row[mi % SEG] * (K / 32) + mi / (2 * SEG)) * 2 + mi / SEG % 2;
+  const bool brings = __builtin_amdgcn_readfirstlane(wave) < SEG / 8;
+  const uint16_t* ap[NA];                                       // the lane's activations: 4 rows an instruction
 #pragma unroll
-  for (int m = 0; m < NA; ++m) ar[m] = in_row[4 * ((NA * wave + m) % (SEG / 4)) + (lane >> 4)];
-  float ds[NT][4];
-#pragma unroll
-  for (int t = 0; t < NT; ++t)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) ds[t][i] = P.scale[in_row[16 * t + 4 * q + i]];
+  for (int m = 0; m < NA; ++m) {
+    const int id = NA * wave + m, r = 4 * (id % (SEG / 4)) + (lane >> 4);
+    ap[m] = (id / (SEG / 4) ? P.lo : P.hi) + (int64_t)in_row[r] * K + 8 * (l16 ^ (r & 15));
+  }
   auto load = [&](int it, int b) {
     const int tile = it / ns, s = it - tile * ns;
     uint8_t* st = smem + b * STAGE;
@@ -195,35 +183,28 @@ __global__ void __launch_bounds__(256) k_pf8_gemm(Gemm8 P) {
         to_lds<16>(wp[i] + (int64_t)tile * 16 * NW * rb + s * kWRow + wo[j],
                    st + 2 * PLANE + wave * WB + i * 16 * kWRow + j * 1024);
 #pragma unroll
-    for (int m = 0; m < NA; ++m) {
-      const int id = NA * wave + m, pl = id / (SEG / 4), r4 = id % (SEG / 4), r = 4 * r4 + (lane >> 4);
-      to_lds<16>((pl ? P.lo : P.hi) + (int64_t)ar[m] * K + s * kStep + 8 * (l16 ^ (r & 15)),
-                 st + pl * PLANE + r4 * 1024);
-    }
-    if (lane < SEG) to_lds<4>(sp + s * 4, st + 2 * PLANE + NW * WB + wave * SEG * 4);
+    for (int m = 0; m < NA; ++m) to_lds<16>(ap[m] + s * kStep, st + (NA * wave + m) * 1024);
+    if (brings) to_lds<4>(mp + s * 8, st + 2 * PLANE + NW * WB + wave * 256);
   };
   gm_f32x4 acc[NMAT][NT];
 #pragma unroll
   for (int i = 0; i < NMAT; ++i)
 #pragma unroll
     for (int t = 0; t < NT; ++t) acc[i][t] = gm_f32x4{0.f, 0.f, 0.f, 0.f};
-  __builtin_amdgcn_s_waitcnt(0);                                // every other load is in: only steps count below
-  const int ahead = total < NST - 1 ? total : NST - 1;
-  for (int i = 0; i < ahead; ++i) load(i, i);
+  load(0, 0);
   const bool low = q < 2;                                       // the lane's octet is in the first half
-  for (int it = 0, b = 0; it < total; ++it, b = b + 1 < NST ? b + 1 : 0) {
-    const int rest = total - 1 - it;                            // steps after this one, NST - 2 of them on their way
-    wait_steps<NL>(rest < NST - 2 ? rest : NST - 2);
+  for (int it = 0; it < total; ++it) {
+    __builtin_amdgcn_s_waitcnt(0xf70);                          // vmcnt(0)
     lds_barrier();                                              // everyone's part of step it; step it - 1 is done with
-    if (it + NST - 1 < total) load(it + NST - 1, b == 0 ? NST - 1 : b - 1);
-    const uint8_t* st = smem + b * STAGE;
+    if (it + 1 < total) load(it + 1, (it + 1) & 1);
+    const uint8_t* st = smem + (it & 1) * STAGE;
     const uint8_t* wb = st + 2 * PLANE + wave * WB;
-    const float* sums = reinterpret_cast<const float*>(st + 2 * PLANE + NW * WB);
+    const float* meta = reinterpret_cast<const float*>(st + 2 * PLANE + NW * WB);
     constexpr int GS = NT == 1 ? 4 : 2;                         // sub-blocks whose LDS reads go out together
 #pragma unroll
     for (int s0 = 0; s0 < 4; s0 += GS) {
       gm_f16x8 ah[GS][NT], al[GS][NT];
-      gm_f32x4 xs[GS][NT], sc[GS][NMAT];                        // sc: s0, s1, off
+      gm_f32x4 xs[GS][NT], xe[GS][NT], sc[GS][NMAT];            // sums, scales; sc: s0, s1, off
       gm_u32x2 w[GS][NMAT];
 #pragma unroll
       for (int u = 0; u < GS; ++u) {
@@ -238,7 +219,8 @@ __global__ void __launch_bounds__(256) k_pf8_gemm(Gemm8 P) {
           const int o = (16 * t + l16) * kRowB + 16 * ((4 * s + q) ^ l16);
           ah[u][t] = *reinterpret_cast<const gm_f16x8*>(st + o);
           al[u][t] = *reinterpret_cast<const gm_f16x8*>(st + PLANE + o);
-          xs[u][t] = *reinterpret_cast<const gm_f32x4*>(sums + s * SEG + 16 * t + 4 * q);
+          xs[u][t] = *reinterpret_cast<const gm_f32x4*>(meta + 2 * s * SEG + 16 * t + 4 * q);
+          xe[u][t] = *reinterpret_cast<const gm_f32x4*>(meta + (2 * s + 1) * SEG + 16 * t + 4 * q);
         }
       }
       issue_fence();
@@ -261,7 +243,8 @@ __global__ void __launch_bounds__(256) k_pf8_gemm(Gemm8 P) {
             d1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[u][t], B1, d1, 0, 0, 0);
 #pragma unroll
             for (int c = 0; c < 4; ++c)
-              acc[i][t][c] += fmaf(sc[u][i].x, d0[c], fmaf(sc[u][i].y, d1[c], sc[u][i].z * xs[u][t][c]));
+              acc[i][t][c] = fmaf(xe[u][t][c], fmaf(sc[u][i].x, d0[c], fmaf(sc[u][i].y, d1[c], sc[u][i].z * xs[u][t][c])),
+                                  acc[i][t][c]);
           }
         }
     }
@@ -274,8 +257,8 @@ __global__ void __launch_bounds__(256) k_pf8_gemm(Gemm8 P) {
         for (int i = 0; i < 4; ++i) {
           const int c = 16 * t + 4 * q + i;
           if (c < n) {
-            float v = acc[0][t][i] * ds[t][i];
-            if constexpr (NMAT == 2) v = gm_silu(v) * (acc[NMAT - 1][t][i] * ds[t][i]);
+            float v = acc[0][t][i];
+            if constexpr (NMAT == 2) v = gm_silu(v) * acc[NMAT - 1][t][i];
             P.out[(int64_t)out_row[c] * P.M + row] = v;
           }
 #pragma unroll
@@ -285,13 +268,13 @@ __global__ void __launch_bounds__(256) k_pf8_gemm(Gemm8 P) {
   }
 }
 
-template <int NMAT, int NT, int RTB, int NST>
+template <int NMAT, int NT, int RTB>
 int launch8(Gemm8 P, int nseg, hipStream_t s) {
-  constexpr size_t smem = NST * (2 * 16 * NT * 256 + 4 * NMAT * 16 * 192 + 4 * 16 * NT * 4) + 2 * 16 * NT * 4;
-  static_assert(smem <= 160 * 1024, "LDS of a CU");
+  constexpr size_t smem = 2 * (2 * 16 * NT * 256 + 4 * NMAT * 16 * 192 + 8 * 16 * NT * 4) + 2 * 16 * NT * 4;
+  static_assert((NT > 1 ? 1 : NMAT == 2 ? 2 : 3) * smem <= 160 * 1024, "LDS of a CU");
   P.nrt = P.M / (64 * RTB);
-  if (int rc = gm_set_smem(k_pf8_gemm<NMAT, NT, RTB, NST>, smem)) return rc;
-  hipLaunchKernelGGL((k_pf8_gemm<NMAT, NT, RTB, NST>), dim3((unsigned)((nseg + 7) / 8 * 8 * P.nrt)), dim3(256), smem, s, P);
+  if (int rc = gm_set_smem(k_pf8_gemm<NMAT, NT, RTB>, smem)) return rc;
+  hipLaunchKernelGGL((k_pf8_gemm<NMAT, NT, RTB>), dim3((unsigned)((nseg + 7) / 8 * 8 * P.nrt)), dim3(256), smem, s, P);
   GM_TRY(hipGetLastError());
   return GM_OK;
 }
@@ -299,7 +282,7 @@ int launch8(Gemm8 P, int nseg, hipStream_t s) {
 }  // namespace
 
 int gm_pf8_split(const float* src, int rows, int K, const GmPf8Rows& a, hipStream_t s) {
-  hipLaunchKernelGGL(k_pf8_split, dim3((rows + 3) / 4), dim3(256), 0, s, src, rows, K, a.hi, a.lo, a.scale, a.sums);
+  hipLaunchKernelGGL(k_pf8_split, dim3((rows + 3) / 4), dim3(256), 0, s, src, rows, K, a.hi, a.lo, a.meta);
   GM_TRY(hipGetLastError());
   return GM_OK;
 }
@@ -313,12 +296,12 @@ int gm_pf8_gemm(const gm_moe_layer* L, bool down, const GmPf8Rows& a, const int3
   P.w[1] = u8(down ? nullptr : L->up_exps);
   P.wsh[0] = u8(down ? L->down_sh : L->gate_sh);
   P.wsh[1] = u8(down ? nullptr : L->up_sh);
-  P.hi = a.hi; P.lo = a.lo; P.scale = a.scale; P.sums = a.sums;
+  P.hi = a.hi; P.lo = a.lo; P.meta = a.meta;
   P.out = out; P.segs = segs; P.offsets = offsets; P.sorted = down ? nullptr : sorted;
   P.T = T; P.k = L->k; P.E = L->E; P.M = M; P.K = K;
-  // M % 256 == 0: whole tiles.  As many steps in flight as the LDS holds.
-  if (seg_tok == 16 && down) return launch8<1, 1, 4, 2>(P, nseg, s);
-  if (seg_tok == 16) return launch8<2, 1, 1, 2>(P, nseg, s);
-  if (down) return launch8<1, 2, 4, 2>(P, nseg, s);
-  return launch8<2, 2, 1, 2>(P, nseg, s);
+  // M % 256 == 0: whole tiles
+  if (seg_tok == 16 && down) return launch8<1, 1, 4>(P, nseg, s);
+  if (seg_tok == 16) return launch8<2, 1, 1>(P, nseg, s);
+  if (down) return launch8<1, 2, 4>(P, nseg, s);
+  return launch8<2, 2, 1>(P, nseg, s);
 }

@@ -224,6 +224,38 @@ def test_moe_i8_prompts(gpu, D, FF, E, k, T, q_gate, q_down, shared):
     assert torch.equal(y, blk(x, residual=True))           # fixed order: the same bits again
 
 
+@pytest.mark.parametrize("side", ["x", "h"])
+def test_moe_i8_prompt_quiet_sub_blocks(gpu, side):
+    """Activations beside an outlier of their row that meets zero weights only, so that all of
+    the outputs comes from the quiet ones: as exact as through the decode kernels (each
+    sub-block of 32 to 2^-23 of its own largest), bar as above."""
+    from npu_amd import synth
+    from npu_amd.moe import GpuMoeBlock
+    D, FF, E, k, T = 512, 256, 4, 2, 40
+    print(f"i8 quiet case {side}", flush=True)
+    h = synth.host_moe_layer(370, D=D, FF=FF, E=E, k=k, q_gate=QT.Q8_0, q_down=QT.Q8_0)
+    half = lambda v: np.frombuffer(np.float16(v).tobytes(), np.uint8)
+    blocks = lambda w: w.reshape(*w.shape[:-1], -1, 34)    # 34 bytes per 32 weights, the scale first
+    x = torch.randn(T, D, generator=torch.Generator().manual_seed(371))
+    if side == "x":
+        x[:, 3] = 2.0 ** 24
+        for w in (h.gate, h.up, h.gate_sh, h.up_sh):
+            blocks(w)[..., 0, :2] = 0
+        h.router[:, 3] = 0
+        h.sh_gate_inp[3] = 0
+    else:                                                  # hidden value 5 at about 2^20 times the others and more
+        for w in (h.gate, h.up, h.gate_sh, h.up_sh):
+            blocks(w)[..., 5, :, :2] = half(2000.0)
+        for w in (h.down, h.down_sh):
+            blocks(w)[..., 0, :2] = 0
+    blk = GpuMoeBlock.from_host(h, device=gpu)
+    x = x.to(gpu)
+    y = blk(x).double()
+    ref = torch.cat([blk(x[t:t + 8]) for t in range(0, T, 8)]).double()
+    err = (y - ref).norm(dim=1) / ref.norm(dim=1)
+    assert float(err.max()) <= 3e-6, float(err.max())
+
+
 def test_moe_i8_prompt_in_a_small_workspace(gpu):
     """A workspace too small for the planes of the I8 GEMMs still runs the tokens (as decode
     chunks): the static scratch of gm_moe_forward_noalloc, at a T that fits an IQ layer."""
