@@ -312,7 +312,10 @@ __global__ void __launch_bounds__(256) k_pf_attn_merge(AttnP P, int Dh) {
 // ------------------------------------------------------------ Gated DeltaNet
 // exp(g) and beta for 16 tokens x 64 of the 2 Hv alpha / beta rows (fp32
 // weights) on v_mfma_f32_16x16x4_f32: the block's 8 waves take every eighth
-// 16-wide k-step (all four row tiles each) and are added in LDS in wave order.
+// 16-wide k-step (all four row tiles each) and are added pairwise in LDS order.
+// Each k-step is summed by itself and four of them pairwise: beta at D = 2048
+// within 7.5e-8 of 64 bits (one chain through all of a wave's steps: 1.8e-7,
+// which the state of the delta rule feels most).
 // ab[t][r]: r < Hv exp(softplus(alpha_r . h + dt_bias) a), else beta.
 __global__ void __launch_bounds__(512) k_pf_ab(const float* __restrict__ alpha, const float* __restrict__ beta,
                                                const float* __restrict__ dt_bias, const float* __restrict__ a,
@@ -331,15 +334,43 @@ __global__ void __launch_bounds__(512) k_pf_ab(const float* __restrict__ alpha, 
   gm_f32x4 acc[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) acc[j] = gm_f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-  for (int k = 16 * wave; k < D; k += 128) {
-    const gm_f32x4 x = *reinterpret_cast<const gm_f32x4*>(xr + k);
+  auto load = [&](int k, gm_f32x4& x, gm_f32x4 (&w)[4]) {
+    x = *reinterpret_cast<const gm_f32x4*>(xr + k);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const gm_f32x4 w = *reinterpret_cast<const gm_f32x4*>(wr[j] + k);
+    for (int j = 0; j < 4; ++j) w[j] = *reinterpret_cast<const gm_f32x4*>(wr[j] + k);
+  };
+  auto step = [&](const gm_f32x4& x, const gm_f32x4& w) {
+    gm_f32x4 d = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[e], x[e], acc[j], 0, 0, 0);
+    for (int e = 0; e < 4; ++e) d = __builtin_amdgcn_mfma_f32_16x16x4f32(w[e], x[e], d, 0, 0, 0);
+    return d;
+  };
+  int k = 16 * wave;
+  if (k + 384 < D) {                                            // four steps at a time, the next four on their way
+    gm_f32x4 xn[4], wn[4][4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) load(k + 128 * u, xn[u], wn[u]);
+    for (; k + 384 < D; k += 512) {
+      gm_f32x4 x[4], w[4][4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        x[u] = xn[u];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w[u][j] = wn[u][j];
+      }
+      const int k1 = k + 512 + 384 < D ? k + 512 : k;           // the last round reloads, unused
+#pragma unroll
+      for (int u = 0; u < 4; ++u) load(k1 + 128 * u, xn[u], wn[u]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        acc[j] += (step(x[0], w[0][j]) + step(x[1], w[1][j])) + (step(x[2], w[2][j]) + step(x[3], w[3][j]));
     }
+  }
+  for (; k < D; k += 128) {
+    gm_f32x4 x, w[4];
+    load(k, x, w);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[j] += step(x, w[j]);
   }
   if (wave > 0) {
 #pragma unroll
@@ -348,9 +379,9 @@ __global__ void __launch_bounds__(512) k_pf_ab(const float* __restrict__ alpha, 
   __syncthreads();
   if (wave > 0 || tok >= T) return;
 #pragma unroll
-  for (int v = 0; v < 7; ++v)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[j] += red[v][j][lane];
+  for (int j = 0; j < 4; ++j)
+    acc[j] = ((acc[j] + red[0][j][lane]) + (red[1][j][lane] + red[2][j][lane])) +
+             ((red[3][j][lane] + red[4][j][lane]) + (red[5][j][lane] + red[6][j][lane]));
 #pragma unroll
   for (int j = 0; j < 4; ++j)
 #pragma unroll

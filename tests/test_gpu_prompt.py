@@ -185,6 +185,40 @@ def test_ssm_prompts(gpu, kw, parts):
             assert _rel(ns[0], os_[0]) <= 1e-5, f"part {i}: conv state"
 
 
+def test_ssm_prompt_no_less_exact_than_steps(gpu):
+    """A prompt's outputs and new state against 64 bits, beside the error of the same tokens one
+    at a time.  Both are sums of some 1e6 rounding errors of either sign, whose norms over as
+    many values differ by less than a hundredth by chance; the bar leaves five."""
+    from npu_amd import qwen_core as QN
+    from oracle import qwen_core as QC
+    kw = dict(d_model=2048, ssm_d_inner=1024, ssm_d_state=128, ssm_n_k_heads=4, ssm_n_v_heads=8)
+    print("ssm precision case", flush=True)
+    ocfg, ncfg = _cfgs(**kw)
+    g = torch.Generator().manual_seed(51)
+    D, Hv, Hk, S = 2048, 8, 4, 128
+    C = 2 * Hk * S + Hv * S
+    r = lambda *s, sc=1.0: torch.randn(*s, generator=g) * sc
+    bf = lambda *s: r(*s, sc=0.02).to(torch.bfloat16).float()
+    W = dict(attn_norm=1 + r(D, sc=0.1), post_norm=1 + r(D, sc=0.1), w_in=bf(C, D), w_gate=bf(Hv * S, D),
+             conv1d=r(C, 4, sc=0.5), a=-torch.rand(Hv, generator=g), alpha=r(Hv, D, sc=0.05), beta=r(Hv, D, sc=0.05),
+             dt_bias=r(Hv, sc=0.5), ssm_norm=1 + r(S, sc=0.1), w_out=bf(D, Hv * S))
+    T = 500
+    x = r(1, T, D)
+    ref, (_, Sr) = QC.ssm_forward(x.double(), QC.SSMW(**{n: t.double() for n, t in W.items()}), ocfg,
+                                  (torch.zeros(1, C, 3).double(), torch.zeros(1, Hv, S, S).double()))
+    layer = QN.SSMLayer(i=0, **W)
+    y, st = QN.ssm_forward(x.to(gpu), layer, ncfg, None)
+    steps, ss = [], None
+    for t in range(T):
+        yt, ss = QN.ssm_forward(x[:, t:t + 1].to(gpu), layer, ncfg, ss)
+        steps.append(yt)
+    err = lambda a, b: float((a.double().cpu() - b).norm() / b.norm())
+    y1, s1 = torch.cat(steps, 1), ss[1]
+    print(f"y {err(y, ref):.3e} against {err(y1, ref):.3e}, state {err(st[1], Sr):.3e} against {err(s1, Sr):.3e}", flush=True)
+    assert err(y, ref) <= 1.05 * err(y1, ref)
+    assert err(st[1], Sr) <= 1.05 * err(s1, Sr)
+
+
 # ---- MoE blocks with I8 routed experts over more than 8 tokens (prefill_i8.hip)
 def _i8_block(gpu, D, FF, E, k, q_gate, q_down, shared, seed):
     from npu_amd import synth
