@@ -9,6 +9,10 @@
 // within 2^-39 of that below; the decode kernels' limbs keep 2^-23 of the
 // sub-block's largest.  With them the sub-block's sum, for the offsets, and its
 // scale 2^-s.
+// Every other sub-block is held negated, with a negative scale: the f16 MFMA rounds
+// its sums towards -infinity as the bf16 one does (bf16_split.h), which quants and
+// offsets of one sign do not average out (Q8_0 / Q5_K experts at D = 2048: error
+// against 64 bits 1.05e-6, now 1.8e-7; the decode kernels 5.4e-7).
 // Weights: int8 quants are exact in f16; the two scales and the offset of a
 // sub-block of 32 are applied in fp32 to its two half sums, then the activations':
 //   y += 2^-s (s0 (q[0..15] . x) + s1 (q[16..31] . x) + off sum(x))
@@ -54,7 +58,7 @@ __global__ void __launch_bounds__(256) k_pf8_split(const float* __restrict__ src
       float f[4];
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        f[c] = __builtin_ldexpf(v[u][c], sh);
+        f[c] = __builtin_ldexpf(lane & 8 ? -v[u][c] : v[u][c], sh);
         h[c] = (_Float16)f[c];
         l[c] = (_Float16)(f[c] - (float)h[c]);
       }
@@ -62,7 +66,7 @@ __global__ void __launch_bounds__(256) k_pf8_split(const float* __restrict__ src
       ph[i] = make_uint2(__builtin_bit_cast(uint32_t, h01), __builtin_bit_cast(uint32_t, h23));
       pl[i] = make_uint2(__builtin_bit_cast(uint32_t, l01), __builtin_bit_cast(uint32_t, l23));
       const float s = gm_sum8((f[0] + f[1]) + (f[2] + f[3]));
-      if ((lane & 7) == 0) pm[i / 8] = gm_f32x2{s, __builtin_ldexpf(1.0f, -sh)};
+      if ((lane & 7) == 0) pm[i / 8] = gm_f32x2{s, __builtin_ldexpf(lane & 8 ? -1.0f : 1.0f, -sh)};
     }
   }
 }
@@ -200,6 +204,7 @@ __global__ void __launch_bounds__(256) k_pf8_gemm(Gemm8 P) {
     const uint8_t* st = smem + (it & 1) * STAGE;
     const uint8_t* wb = st + 2 * PLANE + wave * WB;
     const float* meta = reinterpret_cast<const float*>(st + 2 * PLANE + NW * WB);
+    gm_f32x4 part[NMAT][NT];                                    // the step's sums: a fourth of the running sum's additions
     constexpr int GS = NT == 1 ? 4 : 2;                         // sub-blocks whose LDS reads go out together
 #pragma unroll
     for (int s0 = 0; s0 < 4; s0 += GS) {
@@ -242,12 +247,17 @@ __global__ void __launch_bounds__(256) k_pf8_gemm(Gemm8 P) {
             d0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[u][t], B0, d0, 0, 0, 0);
             d1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[u][t], B1, d1, 0, 0, 0);
 #pragma unroll
-            for (int c = 0; c < 4; ++c)
-              acc[i][t][c] = fmaf(xe[u][t][c], fmaf(sc[u][i].x, d0[c], fmaf(sc[u][i].y, d1[c], sc[u][i].z * xs[u][t][c])),
-                                  acc[i][t][c]);
+            for (int c = 0; c < 4; ++c) {
+              const float v = fmaf(sc[u][i].x, d0[c], fmaf(sc[u][i].y, d1[c], sc[u][i].z * xs[u][t][c]));
+              part[i][t][c] = s0 + u == 0 ? xe[u][t][c] * v : fmaf(xe[u][t][c], v, part[i][t][c]);
+            }
           }
         }
     }
+#pragma unroll
+    for (int i = 0; i < NMAT; ++i)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[i][t] += part[i][t];
     if ((it + 1) % ns == 0) {
       // a row tile is done: lane l holds tokens 4 (l / 16) + i of a token tile, weight row l % 16
       const int row = row0 + (it / ns) * 16 * NW + l16;

@@ -290,6 +290,26 @@ def test_moe_i8_prompt_quiet_sub_blocks(gpu, side):
     assert float(err.max()) <= 3e-6, float(err.max())
 
 
+@pytest.mark.parametrize("q_gate,q_down", [(QT.Q8_0, QT.Q5_K), (QT.Q6_K, QT.Q6_K), (QT.Q4_K, QT.Q5_K)])
+def test_moe_i8_prompt_no_less_exact_than_steps(gpu, q_gate, q_down):
+    """Against 64 bits, beside the error of the decode kernels on the same tokens (both are some
+    80,000 sums of rounding errors of either sign: norms that chance alone moves by less than a
+    hundredth; the bar leaves five)."""
+    from npu_amd import synth
+    from npu_amd.moe import GpuMoeBlock
+    from oracle import moe as OM
+    T = 40
+    print(f"i8 precision case {q_gate} {q_down}", flush=True)
+    h = synth.host_moe_layer(380, D=2048, FF=512, E=8, k=8, q_gate=q_gate, q_down=q_down)
+    blk = GpuMoeBlock.from_host(h, device=gpu)
+    x = torch.randn(T, 2048, generator=torch.Generator().manual_seed(381))
+    ref = OM.moe_forward_dense64(x, OM.OracleLayer(h))
+    err = lambda y: float((y.cpu().double() - ref).norm() / ref.norm())
+    y, steps = blk(x.to(gpu)), torch.cat([blk(x[t:t + 8].to(gpu)) for t in range(0, T, 8)])
+    print(f"{err(y):.3e} against {err(steps):.3e}", flush=True)
+    assert err(y) <= 1.05 * err(steps)
+
+
 def test_moe_i8_prompt_in_a_small_workspace(gpu):
     """A workspace too small for the planes of the I8 GEMMs still runs the tokens (as decode
     chunks): the static scratch of gm_moe_forward_noalloc, at a T that fits an IQ layer."""
