@@ -139,13 +139,17 @@ __device__ __forceinline__ void v_masked(const float* V, int g, int key0, int la
 //                 tiles c); the lane gets dims 64 g + 16 q + 4 i + c of query l16
 // so neither the scores nor K or V are ever transposed.  16-byte granule g of
 // an LDS row r sits at g ^ (r & 15): the 16 keys that a wave reads at once hit
-// different banks.  Scores are added up 32 dims at a time, and a tile's part of
-// the output is formed by itself, then o a + part (chains of MFMAs through all
-// dims and keys: error against 64 bits 6.1e-7 at 1021 tokens on 300, one token
-// at a time 3.3e-7).
+// different banks.  Scores are added up SC MFMAs at a time, and a tile's part of
+// the output is formed by itself (OC chains), then o a + part (chains of MFMAs
+// through all dims and keys: error of the layer against 64 bits 6.1e-7 at 1021
+// tokens on 300 with heads of 256, one token at a time 3.3e-7).  Short chains for
+// heads of up to 128, whose projections round less: 64 tokens on 500 with heads of
+// 128 2.5e-7 -> 2.2e-7, one token at a time 2.2e-7.  For 256 the long ones: 2.5e-7
+// against 3.0e-7, and the short ones cost 175 -> 207 us at 1021 tokens on 300.
 template <int DV>
 __global__ void __launch_bounds__(256, DV <= 4 ? 2 : 1) k_pf_attn(AttnP P) {
   constexpr int Dh = 64 * DV, NG = Dh / 4, NS = Dh / 16, TILE = 16 * Dh;   // floats of 16 rows
+  constexpr int SC = DV <= 2 ? 2 : 8, OC = DV <= 2 ? 2 : 1;                // MFMAs in a chain of scores; chains of outputs
   extern __shared__ __attribute__((aligned(16))) float sm[];               // [2][K, V][TILE]
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l16 = lane & 15, q = lane >> 4;
   const int G = P.Hq / P.Hkv, R = P.T * G;
@@ -202,18 +206,25 @@ __global__ void __launch_bounds__(256, DV <= 4 ? 2 : 1) k_pf_attn(AttnP P) {
     const float* V = K + TILE;
     gm_f32x4 sc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int s = 0; s < NS; s += 4) {                                      // 64 dims: two chains of 8 MFMAs
-      gm_f32x4 d[2];
+    for (int s = 0; s < NS; s += 4) {                                      // 64 dims, 16 MFMAs
+      constexpr int NC = 16 / SC;
+      gm_f32x4 d[NC];
 #pragma unroll
-      for (int c = 0; c < 2; ++c) d[c] = gm_f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int c = 0; c < NC; ++c) d[c] = gm_f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const gm_f32x4 k = *reinterpret_cast<const gm_f32x4*>(K + ko[u] + 16 * s);
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          d[u & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[j], qv[s + u][j], d[u & 1], 0, 0, 0);
+        for (int j = 0; j < 4; ++j) {
+          gm_f32x4& a = d[NC == 2 ? u & 1 : 2 * u + j / 2];
+          a = __builtin_amdgcn_mfma_f32_16x16x4f32(k[j], qv[s + u][j], a, 0, 0, 0);
+        }
       }
-      sc += d[0] + d[1];
+#pragma unroll
+      for (int h = NC / 2; h > 0; h /= 2)
+#pragma unroll
+        for (int c = 0; c < h; ++c) d[c] += d[c + h];
+      sc += d[0];
     }
     float p[4];
 #pragma unroll
@@ -232,23 +243,28 @@ __global__ void __launch_bounds__(256, DV <= 4 ? 2 : 1) k_pf_attn(AttnP P) {
     const bool odd = it * 16 + 15 > first && v_not_finite<DV>(V, vo);
 #pragma unroll
     for (int g = 0; g < DV; ++g) {
-      gm_f32x4 w[4];
+      gm_f32x4 w[OC][4];
 #pragma unroll
-      for (int c = 0; c < 4; ++c) w[c] = gm_f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int h = 0; h < OC; ++h)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) w[h][c] = gm_f32x4{0.f, 0.f, 0.f, 0.f};
       if (!odd) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const gm_f32x4 v = *reinterpret_cast<const gm_f32x4*>(V + vo[i] + 64 * g);
 #pragma unroll
-          for (int c = 0; c < 4; ++c) w[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[c], p[i], w[c], 0, 0, 0);
+          for (int c = 0; c < 4; ++c)
+            w[i * OC / 4][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[c], p[i], w[i * OC / 4][c], 0, 0, 0);
         }
       } else {
-        v_masked<Dh>(V, g, it * 16, last, p, w);
+        v_masked<Dh>(V, g, it * 16, last, p, w[0]);
       }
 #pragma unroll
-      for (int c = 0; c < 4; ++c)
+      for (int c = 0; c < 4; ++c) {
+        if constexpr (OC == 2) w[0][c] += w[1][c];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o[g][c][e] = fmaf(o[g][c][e], a, w[c][e]);
+        for (int e = 0; e < 4; ++e) o[g][c][e] = fmaf(o[g][c][e], a, w[0][c][e]);
+      }
     }
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();

@@ -144,6 +144,51 @@ def test_attention_prompt_non_finite_token(gpu, kw, prefix):
     assert float((y[0, :21] - ref[0, :21]).double().norm() / ref[0, :21].double().norm()) <= 1e-6
 
 
+# 128 and 256 dims a head, on a cache whose keys are cut into parts
+@pytest.mark.parametrize("kw", [dict(), dict(d_model=1024, n_head=8, n_head_kv=1, head_dim=256)])
+def test_attention_prompt_no_less_exact_than_steps(gpu, kw):
+    """A prompt's outputs, k and v against 64 bits, beside the error of the same tokens one at a
+    time: sums of some 60,000 rounding errors of either sign and more, whose norms chance moves
+    by less than a hundredth; the bar leaves two."""
+    from npu_amd import qwen_core as QN
+    print(f"attention precision case {kw}", flush=True)
+    ocfg, ncfg = _cfgs(**kw)
+    W = _attn(ocfg, 61)
+    W["q_norm"], W["k_norm"] = W["q_norm"] / 2, W["k_norm"] / 2        # scores of about one
+    T, prefix = 120, 500
+    Hq, Hkv, Dh, rd = ocfg.n_head, ocfg.n_head_kv, ocfg.head_dim, ocfg.rope_dim
+    cos, sin = QN.build_partial_rope_cache(rd, prefix + T, ocfg.rope_theta)
+    g = torch.Generator().manual_seed(62)
+    x = torch.randn(1, T, ocfg.d_model, generator=g)
+    k0, v0 = torch.randn(prefix, Hkv, Dh, generator=g), 0.5 * torch.randn(prefix, Hkv, Dh, generator=g)
+    # in 64 bits
+    w64 = {n: t.double() for n, t in W.items()}
+    rms = lambda t, w: t * (t.square().mean(-1, keepdim=True) + ocfg.rms_eps).rsqrt() * w
+    h = rms(x[0].double(), w64["attn_norm"])
+    q, gate = (h @ w64["wq"].T).reshape(T, Hq, 2, Dh).unbind(2)
+    k, v = (h @ w64["wk"].T).reshape(T, Hkv, Dh), (h @ w64["wv"].T).reshape(T, Hkv, Dh)
+    c, s = (t[prefix:, None].double() for t in (cos, sin))
+    rope = lambda t: torch.cat([t[..., :rd] * c + torch.cat([-t[..., rd // 2:rd], t[..., :rd // 2]], -1) * s, t[..., rd:]], -1)
+    q, k = rope(rms(q, w64["q_norm"])), rope(rms(k, w64["k_norm"]))
+    ka, va = (torch.cat([p.double(), t]).repeat_interleave(Hq // Hkv, 1) for p, t in ((k0, k), (v0, v)))
+    mask = torch.arange(prefix + T)[None] > prefix + torch.arange(T)[:, None]
+    sc = torch.stack([q[:, i] @ ka[:, i].T for i in range(Hq)]) / Dh ** 0.5
+    pr = torch.softmax(sc.masked_fill(mask, float("-inf")), -1)
+    o = torch.stack([pr[i] @ va[:, i] for i in range(Hq)], 1) * torch.sigmoid(gate)
+    ref = (o.reshape(T, -1) @ w64["wo"].T, k, v)
+    layer = QN.AttnLayer(i=0, **W)
+
+    def run(parts):
+        cache = QN.KVCache(ncfg, prefix + T)
+        cache.k[:prefix], cache.v[:prefix], cache.length = k0.to(gpu), v0.to(gpu), prefix
+        ys = [QN.attn_forward(xp.to(gpu), layer, ncfg, cos, sin, cache, cache.length)[0] for xp in x.split(parts, 1)]
+        return torch.cat(ys, 1)[0], cache.k[prefix:], cache.v[prefix:]
+    err = lambda a, b: float((a.double().cpu() - b).norm() / b.norm())
+    for n, a, b, r in zip("ykv", run(T), run(1), ref):
+        print(f"{n} {err(a, r):.3e} against {err(b, r):.3e}", flush=True)
+        assert err(a, r) <= 1.02 * err(b, r), n
+
+
 # d_state 64 / 128 / 256, prompts around the 16 staged tokens (8 at 256) and past the part of
 # 1024, conv kernels of 1, 2 and 8 taps, and a prompt shorter than the conv state
 @pytest.mark.parametrize("kw,parts", [
