@@ -243,11 +243,16 @@ bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0;
 //   the same with K split over two halves of a 512-thread block (>= 128):
 //     M = 2048 K = 4096 T = 1000 (256 tiles) 73 against 84 us, M = 9216 T = 120 (144) 35 against 41;
 //   below that 64 x 64 tiles with K split over four quarters of a 1024-thread
-//     block: M = 9216 T = 57 (72) 23 against 33 us, M = 2048 K = 4096 T = 300 (80) 44 against 64;
-//   fewer than 48 of those leave most CUs idle, and the few-token kernel's
-//     16-row blocks win: M = 2048 K = 4096 T = 57 25 against 36 us (T = 100, 64 tiles: 44 against 40).
-bool gm_gemm_bf16_takes(int rows, int T) {
-  return T > 16 && (int64_t)((rows + 63) / 64) * ((T + 63) / 64) >= 48;
+//     block: M = 9216 T = 57 (72) 23 against 33 us, M = 2048 K = 4096 T = 300 (80) 44 against 64.
+// Such a tile takes as long whatever part of the chip the tiles fill, while the
+// few-token kernel's time goes with its 16 x 16 tiles; these are counted (few-token
+// kernel / this one, us):
+//   K = 4096, M = 2048: T = 65 (640) 31 / 40, 96 (768) 36 / 40, 97 (896) 42 / 40
+//   K = 2048, M = 3072: T = 64 (768) 20 / 22, 65 (960) 23 / 22; M = 4096: T = 33 (768) 17 / 19, 49 (1024) 23 / 22
+//   up to 32 tokens, K = 2048: M = 4096 (512) 13 / 18, 6144 (768) 18 / 17
+//   K = 512, M = 4096: T = 65 (1280) 8.4 / 8.7, 96 (1536) 11 / 9
+bool gm_gemm_bf16_takes(int rows, int K, int T) {
+  return T > 16 && (int64_t)((rows + 15) / 16) * ((T + 15) / 16) >= (T <= 32 ? 736 : K < 1024 ? 1300 : 800);
 }
 
 int gm_launch_gemm_bf16(const uint16_t* w, int M, const uint16_t* w2, int M2, int K, const float* x, int T,

@@ -30,7 +30,7 @@ int gm_launch_dense(const uint16_t* w, int M, const uint16_t* w2, int M2, int K,
 // Many tokens (gemm_bf16.hip): y = x W^T (+ add, [T][M]) and, when w2 is given,
 // y2 = x W2^T in the same launch.  K % 32 == 0; w, w2 and x 16-byte aligned.
 // gm_gemm_bf16_takes: whether a call is large enough for it.
-bool gm_gemm_bf16_takes(int rows, int T);
+bool gm_gemm_bf16_takes(int rows, int K, int T);
 int gm_launch_gemm_bf16(const uint16_t* w, int M, const uint16_t* w2, int M2, int K, const float* x, int T,
                         const float* add, float* y, float* y2, hipStream_t s);
 int gm_launch_gateup(int qtype, const void* wg, const void* wu, int FF, int D, const float* x, int n_tok,

@@ -426,13 +426,13 @@ int launch_mv1(const uint16_t* w, int M, int K, const float* x, float* y, const 
 // tokens per column tile.
 int gm_launch_mv_bf16(const uint16_t* w, int M, int K, const float* x, int n_tok, float* y, hipStream_t s) {
   if (n_tok == 1) return launch_mv1(w, M, K, x, y, nullptr, s);
-  if (gm_gemm_bf16_takes(M, n_tok)) return gm_launch_gemm_bf16(w, M, nullptr, 0, K, x, n_tok, nullptr, y, nullptr, s);
+  if (gm_gemm_bf16_takes(M, K, n_tok)) return gm_launch_gemm_bf16(w, M, nullptr, 0, K, x, n_tok, nullptr, y, nullptr, s);
   return launch_mfma<false>(w, M, K, x, n_tok, nullptr, y, s);
 }
 
 int gm_launch_dense(const uint16_t* w, int M, const uint16_t* w2, int M2, int K, const float* x, int T,
                     const float* add, float* y, float* y2, hipStream_t s) {
-  if (gm_gemm_bf16_takes(M + (w2 ? M2 : 0), T)) return gm_launch_gemm_bf16(w, M, w2, M2, K, x, T, add, y, y2, s);
+  if (gm_gemm_bf16_takes(M + (w2 ? M2 : 0), K, T)) return gm_launch_gemm_bf16(w, M, w2, M2, K, x, T, add, y, y2, s);
   if (int rc = launch_mfma<true>(w, M, K, x, T, add, y, s)) return rc;
   return w2 ? launch_mfma<true>(w2, M2, K, x, T, nullptr, y2, s) : GM_OK;
 }
