@@ -10,12 +10,14 @@ from npu_amd.gguf_types import GGMLQuantizationType as QT
 pytestmark = pytest.mark.gpu
 
 
-# (M, K, T): 128 x 64 tiles with an odd M (scalar stores) and a last half step, K split in
-# two with a K of one step; K split in four with a last part that is short, and
+# (M, K, T): 128 x 64 tiles with an odd M (scalar stores) and a last half step, in few steps
+# and in 17 (both LDS buffers in turn); K split in two with a K of one step, and with an odd
+# count of steps and a short second part; K split in four with a last part that is short, and
 # parts that hold no step at all, one token past a tile; the few-token kernel's last sizes and
 # the first ones that the tiles take: over 16 tokens, over 32, and for a short K
 @pytest.mark.parametrize("M,K,T", [(4099, 96, 700), (4096, 32, 300), (2050, 1056, 260), (3072, 160, 65),
-                                   (3072, 2048, 17), (3072, 2048, 16), (5872, 2048, 32), (5888, 2048, 17), (3184, 1024, 64),
+                                   (3072, 2048, 17), (3072, 2048, 16), (4099, 1056, 700), (2050, 1056, 520),
+                                   (3072, 160, 129), (5872, 2048, 32), (5888, 2048, 17), (3184, 1024, 64),
                                    (3200, 1024, 64), (5184, 544, 64), (5200, 544, 64)])
 def test_gemm_bf16_tiles(gpu, M, K, T):
     g = torch.Generator().manual_seed(M + K + T)
@@ -263,6 +265,39 @@ def test_ssm_prompt_no_less_exact_than_steps(gpu):
     print(f"y {err(y, ref):.3e} against {err(y1, ref):.3e}, state {err(st[1], Sr):.3e} against {err(s1, Sr):.3e}", flush=True)
     assert err(y, ref) <= 1.05 * err(y1, ref)
     assert err(st[1], Sr) <= 1.05 * err(s1, Sr)
+
+
+# wide enough for the 128 x 64 tiles in the input projections (of two matrices in the DeltaNet
+# layer) and for the same with K split in two in the output projection with its residual
+@pytest.mark.parametrize("kind", ["attn", "ssm"])
+def test_wide_core_prompts(gpu, kind):
+    """Against the same tokens one at a time: each within 4e-7 of 64 bits (2-norm)."""
+    from npu_amd import qwen_core as QN
+    print(f"wide prompt case {kind}", flush=True)
+    ocfg, ncfg = _cfgs(d_model=2048, n_head=16, n_head_kv=2, head_dim=256, rope_dim=64, ssm_d_inner=4096,
+                       ssm_d_state=128, ssm_n_k_heads=16, ssm_n_v_heads=32)
+    T, g = 520, torch.Generator().manual_seed(71)
+    r = lambda *s, sc=1.0: torch.randn(*s, generator=g) * sc
+    bf = lambda *s: r(*s, sc=0.02).to(torch.bfloat16).float()
+    x = r(1, T, 2048).to(gpu)
+    if kind == "attn":
+        layer = QN.AttnLayer(i=0, **_attn(ocfg, 72))
+        cos, sin = QN.build_partial_rope_cache(64, T, ocfg.rope_theta)
+        call = lambda xp, st: QN.attn_forward(xp, layer, ncfg, cos, sin, st, st.length if st else 0, residual=True)
+    else:
+        layer = QN.SSMLayer(i=0, attn_norm=1 + r(2048, sc=0.1), post_norm=1 + r(2048, sc=0.1), w_in=bf(8192, 2048),
+                            w_gate=bf(4096, 2048), conv1d=r(8192, 4, sc=0.5), a=-torch.rand(32, generator=g),
+                            alpha=r(32, 2048, sc=0.05), beta=r(32, 2048, sc=0.05), dt_bias=r(32, sc=0.5),
+                            ssm_norm=1 + r(128, sc=0.1), w_out=bf(2048, 4096))
+        call = lambda xp, st: QN.ssm_forward(xp, layer, ncfg, st, residual=True)
+    y, st = call(x, None)
+    ys, ss = [], None
+    for t in range(T):
+        yt, ss = call(x[:, t:t + 1], ss)
+        ys.append(yt)
+    state = lambda s: (s.k[:T], s.v[:T]) if kind == "attn" else s
+    for a, b in zip((y - x, *state(st)), (torch.cat(ys, 1) - x, *state(ss))):
+        assert float((a - b).double().norm() / b.double().norm()) <= 1e-6
 
 
 # ---- MoE blocks with I8 routed experts over more than 8 tokens (prefill_i8.hip)
