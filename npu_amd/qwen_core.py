@@ -19,7 +19,7 @@ reference concatenates a ``[B, T, n_head, head_dim]`` cache per step, repeating 
 head over its q heads); the Gated DeltaNet state is ``(conv_state [1, C, k - 1],
 S [1, Hv, Sk, Sv])``, the reference's tuple, as device tensors updated in place.
 Several tokens (a prompt) are one call per core layer too (``gm_attn_prefill`` /
-``gm_ssm_prefill``), every launch over all tokens; the MoE block then takes the
+``gm_ssm_prefill``), every launch over all tokens (two tokens mostly two steps); the MoE block then takes the
 layer's T tokens at once.  There is no CPU path: without the built library every
 call raises.
 """
@@ -173,6 +173,15 @@ class GpuAttn:
         L.check(rc, "gm_attn_prefill")
 
 
+def _as_steps(T: int, D: int, cached: int = 0) -> bool:
+    """Whether T tokens go one at a time: one, or two where two steps take less time than the
+    prompt's launches, whose latencies hardly depend on T.  us a call, steps / prompt, for two
+    tokens: DeltaNet at D = 2048 56 / 70, at D = 512 56 / 49; attention at D = 2048 49 / 64 (500
+    positions cached) and 93 / 95 (4000), but 50 / 46 on none, at D = 512 48 / 33 on none,
+    49 / 49 (3000) and 48 / 57 (4000).  Three tokens: 75 / 73, 68 / 66, 139 / 96."""
+    return T == 1 or (T == 2 and (D >= 1024 or cached >= 3500))
+
+
 class KVCache:
     """One attention layer's cache, ``[max_pos][n_head_kv][head_dim]`` fp32 for k and v,
     and the number of positions filled."""
@@ -218,7 +227,8 @@ def attn_forward(x: torch.Tensor, layer: AttnLayer, cfg: Config, cos: torch.Tens
     cd, sd = _rope_on_device(cos, sin)
     y = torch.empty_like(xd)
     with profile("attn.decode"):
-        if T > 1 and kv_cache.k.data_ptr() % 16 == 0 and kv_cache.v.data_ptr() % 16 == 0:
+        aligned = kv_cache.k.data_ptr() % 16 == 0 and kv_cache.v.data_ptr() % 16 == 0
+        if T > 0 and aligned and not _as_steps(T, D, start_pos):
             layer.gpu.prompt(xd, kv_cache, start_pos, cd, sd, residual, y)
             kv_cache.length += T
         else:
@@ -342,10 +352,11 @@ def ssm_forward(x: torch.Tensor, layer: SSMLayer, cfg: Config, ssm_state, *, res
     xd = x.reshape(T, D).to(device(), torch.float32).contiguous()
     y = torch.empty_like(xd)
     with profile("ssm.decode"):
-        if T > 1:
+        if T > 0 and not _as_steps(T, D):
             layer.gpu.prompt(xd, state, residual, y)
-        elif T == 1:
-            layer.gpu.step(xd[0], state, residual, y[0], moe_link)
+        else:
+            for t in range(T):
+                layer.gpu.step(xd[t], state, residual, y[t], moe_link)
     y = y.view(1, T, D)
     return (y.cpu() if on_host else y), state
 

@@ -267,6 +267,49 @@ def test_ssm_prompt_no_less_exact_than_steps(gpu):
     assert err(st[1], Sr) <= 1.05 * err(s1, Sr)
 
 
+# the widths from which two tokens are two steps, and those below where they are a prompt; past
+# 3500 cached positions an attention layer of any width
+@pytest.mark.parametrize("D,prefix,steps", [(1024, 3, True), (992, 3, False), (512, 3500, True), (512, 3499, False)])
+def test_two_tokens(gpu, D, prefix, steps, monkeypatch):
+    """Two tokens go the faster way: the bits of two single calls, or one prompt call."""
+    from npu_amd import qwen_core as QN
+    print(f"two tokens case {D} {prefix}", flush=True)
+    ocfg, ncfg = _cfgs(d_model=D)
+    g = torch.Generator().manual_seed(81)
+    r = lambda *s, sc=1.0: torch.randn(*s, generator=g) * sc
+    bf = lambda *s: r(*s, sc=0.03).to(torch.bfloat16).float()
+    A = QN.AttnLayer(i=0, **_attn(ocfg, 82))
+    S = QN.SSMLayer(i=0, attn_norm=1 + r(D, sc=0.1), post_norm=1 + r(D, sc=0.1), w_in=bf(512, D), w_gate=bf(256, D),
+                    conv1d=r(512, 4, sc=0.5), a=-torch.rand(4, generator=g), alpha=r(4, D, sc=0.05),
+                    beta=r(4, D, sc=0.05), dt_bias=r(4, sc=0.5), ssm_norm=1 + r(64, sc=0.1), w_out=bf(D, 256))
+    cos, sin = QN.build_partial_rope_cache(ocfg.rope_dim, prefix + 2, ocfg.rope_theta)
+    x = r(1, 2, D).to(gpu)
+    k, v = r(prefix, 2, 128).to(gpu), r(prefix, 2, 128).to(gpu)
+    prompts = []
+    for cls in (QN.GpuAttn, QN.GpuSsm):
+        monkeypatch.setattr(cls, "prompt", lambda self, *a, _f=cls.prompt, _c=cls: (prompts.append(_c), _f(self, *a))[1])
+
+    def attn(parts):
+        c = QN.KVCache(ncfg, prefix + 2)
+        c.k[:prefix], c.v[:prefix], c.length = k, v, prefix
+        y = torch.cat([QN.attn_forward(xp, A, ncfg, cos, sin, c, c.length)[0] for xp in x.split(parts, 1)], 1)
+        assert c.length == prefix + 2
+        return y, c.k, c.v
+
+    def ssm(parts):
+        st, ys = None, []
+        for xp in x.split(parts, 1):
+            y, st = QN.ssm_forward(xp, S, ncfg, st)
+            ys.append(y)
+        return torch.cat(ys, 1), *st
+
+    for fn, cls, one in ((attn, QN.GpuAttn, steps), (ssm, QN.GpuSsm, D >= 1024)):
+        two, single = fn(2), fn(1)
+        assert (cls not in prompts) == one
+        for a, b in zip(two, single):
+            assert torch.equal(a, b) if one else float((a - b).norm() / b.norm()) <= 1e-6
+
+
 # wide enough for the 128 x 64 tiles in the input projections (of two matrices in the DeltaNet
 # layer) and for the same with K split in two in the output projection with its residual
 @pytest.mark.parametrize("kind", ["attn", "ssm"])
