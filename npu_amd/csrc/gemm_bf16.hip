@@ -9,14 +9,14 @@
 // which makes the operands' way, not the matrix cores, the bound:
 //  * the weights of a tile (16 RT rows x 64 k) go through LDS, since every wave
 //    of a block needs all of them;
-//  * a wave has 16 CT tokens of its own, whose x goes from global memory to
+//  * a wave has 16 tokens of its own, whose x goes from global memory to
 //    registers and is split there, once per block (planes formed beforehand and
 //    loaded instead, 6 bytes a value against 4: 134.6 -> 168 us at M = 9216,
 //    K = 2048, T = 1021);
 //  * both are loaded one step ahead in registers; what one block waits for its
 //    loads (1.2 us a step when alone on a CU) two or three others fill.
-// One token tile per wave (CT = 1) against two at the same row count: 136
-// against 163 us there, 57 against 73 at T = 300 (more blocks, three to a CU).
+// One token tile per wave against two at the same row count: 136 against 163 us
+// there, 57 against 73 at T = 300 (more blocks, three to a CU).
 // A step's 64 k are summed by themselves, the lower planes first, two row tiles'
 // chains of MFMAs in turn, and then added to the running sum: error against 64
 // bits 1.2e-7 (one chain through all steps: 5e-7 at K = 2048, 7e-7 at 4096; the
@@ -47,7 +47,7 @@ struct GemmArgs {
   int vec;               // y, y2, add rows 16-byte aligned: four outputs per store
 };
 
-template <int RT, int CT, int KS>
+template <int RT, int KS>
 __global__ void __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) k_gemm_bf16(GemmArgs P) {
   constexpr int NA = RT / 2;                                    // 16-byte granules of A per thread and step
   constexpr int ABUF = RT * 16 * 2 * kBK;                       // bytes of one A tile
@@ -56,7 +56,7 @@ __global__ void __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) k_gemm_bf16(GemmArg
   if ((int)(blockIdx.x >> 3) >= P.per_xcd || tile >= P.tiles) return;
   const int grp = KS > 1 ? threadIdx.x >> 8 : 0, tid = threadIdx.x & 255;
   const int wave = tid >> 6, lane = tid & 63, l16 = lane & 15, q = lane >> 4;
-  const int row0 = (tile / P.nc) * (16 * RT), tok0 = (tile % P.nc) * (64 * CT) + wave * (16 * CT);
+  const int row0 = (tile / P.nc) * (16 * RT), tok0 = (tile % P.nc) * 64 + wave * 16;
   const int Mt = P.M + P.M2, K = P.K;
   uint8_t* abuf = smem + grp * 2 * ABUF;
 
@@ -74,23 +74,19 @@ __global__ void __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) k_gemm_bf16(GemmArg
     agran[j] = g;
     aoff[j] = r * (2 * kBK) + 16 * sl + 8 * ((g >> 1) & 1);
   }
-  const float* xp[CT];
-#pragma unroll
-  for (int c = 0; c < CT; ++c) xp[c] = P.x + (int64_t)min(tok0 + 16 * c + l16, P.T - 1) * K + 4 * q;
+  const int tok = tok0 + l16;
+  const float* xp = P.x + (int64_t)min(tok, P.T - 1) * K + 4 * q;
 
   const int nstep = (K + kBK - 1) / kBK, chunk = (nstep + KS - 1) / KS;
   const int s0 = grp * chunk, s1 = min(s0 + chunk, nstep);
   gm_u32x4 ar[NA];
-  gm_f32x4 xr[CT][2][2];
+  gm_f32x4 xr[2][2];
   auto load = [&](int s) {                                      // past the row: its last granule again, unused
     const int k0 = s * kBK;
 #pragma unroll
-    for (int c = 0; c < CT; ++c)
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int p = 0; p < 2; ++p)
-          xr[c][h][p] = *reinterpret_cast<const gm_f32x4*>(xp[c] + min(k0 + 32 * h, K - 32) + 16 * p);
+      for (int p = 0; p < 2; ++p) xr[h][p] = *reinterpret_cast<const gm_f32x4*>(xp + min(k0 + 32 * h, K - 32) + 16 * p);
 #pragma unroll
     for (int j = 0; j < NA; ++j)
       ar[j] = *reinterpret_cast<const gm_u32x4*>(ap[j] + min(k0 + 8 * agran[j], K - 8));
@@ -103,11 +99,9 @@ __global__ void __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) k_gemm_bf16(GemmArg
     }
   };
 
-  gm_f32x4 acc[RT][CT];
+  gm_f32x4 acc[RT];
 #pragma unroll
-  for (int r = 0; r < RT; ++r)
-#pragma unroll
-    for (int c = 0; c < CT; ++c) acc[r][c] = gm_f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int r = 0; r < RT; ++r) acc[r] = gm_f32x4{0.f, 0.f, 0.f, 0.f};
 
   load(min(s0, nstep - 1));
   stage(0);
@@ -115,44 +109,36 @@ __global__ void __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) k_gemm_bf16(GemmArg
   auto step = [&](int i, auto odd) {
     constexpr Sign sign = step_sign(decltype(odd)::value);
     const int s = s0 + i;
-    gm_f32x4 xc[CT][2][2];
+    gm_f32x4 xc[2][2];
 #pragma unroll
-    for (int c = 0; c < CT; ++c)
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int p = 0; p < 2; ++p) xc[c][h][p] = xr[c][h][p];
+      for (int p = 0; p < 2; ++p) xc[h][p] = xr[h][p];
     const bool more = i + 1 < chunk;
     if (more) load(min(s + 1, nstep - 1));
     if (s < s1) {
       const uint8_t* A = abuf + (i & 1) * ABUF;
-      gm_u32x4 pl[CT][2][3];
+      gm_u32x4 pl[2][3];
 #pragma unroll
-      for (int c = 0; c < CT; ++c)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) split3(xc[c][h][0], xc[c][h][1], pl[c][h], sign);
+      for (int h = 0; h < 2; ++h) split3(xc[h][0], xc[h][1], pl[h], sign);
       const bool half = s * kBK + 32 >= K;                      // K % 64 == 32: half a last step
       constexpr int RG = 2;                                     // row tiles at a time: two independent chains
 #pragma unroll
       for (int r0 = 0; r0 < RT; r0 += RG) {
         gm_bf16x8 a[RG][2];
-        gm_f32x4 d[RG][CT];
+        gm_f32x4 d[RG];
 #pragma unroll
         for (int r = 0; r < RG; ++r) {
           const int ra = 16 * (r0 + r) + l16;
 #pragma unroll
           for (int h = 0; h < 2; ++h)
             a[r][h] = *reinterpret_cast<const gm_bf16x8*>(A + ra * (2 * kBK) + 16 * ((4 * h + q) ^ ((ra >> 1) & 7)));
-#pragma unroll
-          for (int c = 0; c < CT; ++c) d[r][c] = gm_f32x4{0.f, 0.f, 0.f, 0.f};
+          d[r] = gm_f32x4{0.f, 0.f, 0.f, 0.f};
         }
         auto mul = [&](int h, int p) {
 #pragma unroll
           for (int r = 0; r < RG; ++r)
-#pragma unroll
-            for (int c = 0; c < CT; ++c)
-              d[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[r][h], __builtin_bit_cast(gm_bf16x8, pl[c][h][p]),
-                                                                d[r][c], 0, 0, 0);
+            d[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[r][h], __builtin_bit_cast(gm_bf16x8, pl[h][p]), d[r], 0, 0, 0);
         };
         if (!half) {
           mul(1, 2);
@@ -166,9 +152,7 @@ __global__ void __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) k_gemm_bf16(GemmArg
         }
         mul(0, 0);
 #pragma unroll
-        for (int r = 0; r < RG; ++r)
-#pragma unroll
-          for (int c = 0; c < CT; ++c) acc[r0 + r][c] += sign.f * d[r][c];
+        for (int r = 0; r < RG; ++r) acc[r0 + r] += sign.f * d[r];
       }
     }
     if (more) stage((i + 1) & 1);
@@ -182,54 +166,46 @@ __global__ void __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) k_gemm_bf16(GemmArg
     gm_f32x4* red = reinterpret_cast<gm_f32x4*>(smem);
     if (grp > 0) {
 #pragma unroll
-      for (int r = 0; r < RT; ++r)
-#pragma unroll
-        for (int c = 0; c < CT; ++c) red[((((grp - 1) * 4 + wave) * RT + r) * CT + c) * 64 + lane] = acc[r][c];
+      for (int r = 0; r < RT; ++r) red[(((grp - 1) * 4 + wave) * RT + r) * 64 + lane] = acc[r];
     }
     __syncthreads();
     if (grp > 0) return;
 #pragma unroll
     for (int g = 0; g < KS - 1; ++g)
 #pragma unroll
-      for (int r = 0; r < RT; ++r)
-#pragma unroll
-        for (int c = 0; c < CT; ++c) acc[r][c] += red[(((g * 4 + wave) * RT + r) * CT + c) * 64 + lane];
+      for (int r = 0; r < RT; ++r) acc[r] += red[((g * 4 + wave) * RT + r) * 64 + lane];
   }
   // C layout: lane l holds rows 4 (l / 16) + i of a row tile, token column l % 16
+  if (tok >= P.T) return;
 #pragma unroll
-  for (int c = 0; c < CT; ++c) {
-    const int tok = tok0 + 16 * c + l16;
-    if (tok >= P.T) continue;
+  for (int r = 0; r < RT; ++r) {
+    const int row = row0 + 16 * r + 4 * q;
+    if (row >= Mt) continue;
+    if (P.vec) {                                                // M % 4 == 0: four rows of one matrix
+      const bool one = row < P.M;
+      const int64_t o = one ? (int64_t)tok * P.M + row : (int64_t)tok * P.M2 + (row - P.M);
+      gm_f32x4 v = acc[r];
+      if (P.add && one) v = *reinterpret_cast<const gm_f32x4*>(P.add + o) + v;
+      *reinterpret_cast<gm_f32x4*>((one ? P.y : P.y2) + o) = v;
+    } else {
 #pragma unroll
-    for (int r = 0; r < RT; ++r) {
-      const int row = row0 + 16 * r + 4 * q;
-      if (row >= Mt) continue;
-      if (P.vec) {                                              // M % 4 == 0: four rows of one matrix
-        const bool one = row < P.M;
-        const int64_t o = one ? (int64_t)tok * P.M + row : (int64_t)tok * P.M2 + (row - P.M);
-        gm_f32x4 v = acc[r][c];
-        if (P.add && one) v = *reinterpret_cast<const gm_f32x4*>(P.add + o) + v;
-        *reinterpret_cast<gm_f32x4*>((one ? P.y : P.y2) + o) = v;
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int m = row + i;
-          if (m >= Mt) break;
-          const bool one = m < P.M;
-          const int64_t o = one ? (int64_t)tok * P.M + m : (int64_t)tok * P.M2 + (m - P.M);
-          (one ? P.y : P.y2)[o] = P.add && one ? P.add[o] + acc[r][c][i] : acc[r][c][i];
-        }
+      for (int i = 0; i < 4; ++i) {
+        const int m = row + i;
+        if (m >= Mt) break;
+        const bool one = m < P.M;
+        const int64_t o = one ? (int64_t)tok * P.M + m : (int64_t)tok * P.M2 + (m - P.M);
+        (one ? P.y : P.y2)[o] = P.add && one ? P.add[o] + acc[r][i] : acc[r][i];
       }
     }
   }
 }
 
-template <int RT, int CT, int KS>
+template <int RT, int KS>
 int launch(GemmArgs P, hipStream_t s) {
-  P.nc = (P.T + 64 * CT - 1) / (64 * CT);
+  P.nc = (P.T + 63) / 64;
   P.tiles = ((P.M + P.M2 + 16 * RT - 1) / (16 * RT)) * P.nc;
   P.per_xcd = (P.tiles + 7) / 8;
-  hipLaunchKernelGGL((k_gemm_bf16<RT, CT, KS>), dim3(8 * P.per_xcd), dim3(256 * KS), 0, s, P);
+  hipLaunchKernelGGL((k_gemm_bf16<RT, KS>), dim3(8 * P.per_xcd), dim3(256 * KS), 0, s, P);
   GM_TRY(hipGetLastError());
   return GM_OK;
 }
@@ -261,7 +237,7 @@ int gm_launch_gemm_bf16(const uint16_t* w, int M, const uint16_t* w2, int M2, in
   P.vec = M % 4 == 0 && P.M2 % 4 == 0 && aligned16(y) && aligned16(y2) && aligned16(add);
   const int64_t t128 = (int64_t)((M + P.M2 + 127) / 128) * ((T + 63) / 64);
   if (t128 >= INT32_MAX / 16) return gm_fail_arg("gemm_bf16: %d rows x %d tokens is too large", M + P.M2, T);
-  if (t128 >= 300) return launch<8, 1, 1>(P, s);
-  if (t128 >= 128) return launch<8, 1, 2>(P, s);
-  return launch<4, 1, 4>(P, s);
+  if (t128 >= 300) return launch<8, 1>(P, s);
+  if (t128 >= 128) return launch<8, 2>(P, s);
+  return launch<4, 4>(P, s);
 }

@@ -629,8 +629,8 @@ __device__ __forceinline__ gm_f16x8 a_f16(const PfRaw<QT>& r, int j, gm_f16x2 sc
 // g ^ (r & 15) of its row, so that the 16 rows a wave reads at once hit 16
 // different bank groups without padding.  The B operand of k-step j, the 8
 // activations of the lane's k-slots, is granule 4 (2q + (j >> 2)) + (j & 3) of a
-// superblock; a gate/up row holds NH-th parts of superblocks (NH = 2: the
-// k-steps of one half, granules 4q + (j & 3)).
+// superblock; a gate/up row holds halves of superblocks (the k-steps of one
+// half, granules 4q + (j & 3)).
 template <int ROWB>
 __device__ __forceinline__ gm_f16x8 b_lds(const uint8_t* tile, int r, int g) {
   return __builtin_bit_cast(gm_f16x8, *reinterpret_cast<const gm_u32x4*>(tile + r * ROWB + 16 * (g ^ (r & 15))));
@@ -639,7 +639,7 @@ __device__ __forceinline__ gm_f16x8 b_lds(const uint8_t* tile, int r, int g) {
 // Half H (k-steps 4H .. 4H+3) of one superblock column of the gate and up
 // rows against NT token tiles: f16 integer operands into the superblock's
 // partial sums pg / pu.
-template <int QT, int NT, int NH, int H>
+template <int QT, int NT, int H>
 __device__ __forceinline__ void gu_half(const PfRaw<QT>& wg, const PfRaw<QT>& wu, const PfF16Scale<QT>& sg,
                                         const PfF16Scale<QT>& su, int q, int l16, const uint8_t* __restrict__ xb,
                                         const uint32_t* __restrict__ grid, const uint32_t* __restrict__ sgn,
@@ -648,10 +648,10 @@ __device__ __forceinline__ void gu_half(const PfRaw<QT>& wg, const PfRaw<QT>& wu
   for (int j = 4 * H; j < 4 * H + 4; ++j) {
     const gm_f16x8 A = a_f16<QT>(wg, j, sg.sh(H), sg.ch(H), grid, sgn);
     const gm_f16x8 U = a_f16<QT>(wu, j, su.sh(H), su.ch(H), grid, sgn);
-    const int g = NH == 1 ? 4 * (2 * q + H) + (j & 3) : 4 * q + (j & 3);
+    const int g = 4 * q + (j & 3);
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      const gm_f16x8 B = b_lds<512 / NH>(xb, t * 16 + l16, g);
+      const gm_f16x8 B = b_lds<256>(xb, t * 16 + l16, g);
       pg[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, B, pg[t], 0, 0, 0);
       pu[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(U, B, pu[t], 0, 0, 0);
     }
@@ -820,16 +820,17 @@ __device__ __forceinline__ void lds_reads_done() { asm volatile("s_waitcnt lgkmc
 // -------------------------------------------------------------- gate/up
 // Block = (segment of at most ST tokens, 64 rows of FF); wave w -> rows 16w ..
 // 16w+15 of both the gate and the up matrix, all of the segment's token tiles.
-// A step is an NH-th part of a superblock: its activations are in one of two LDS
-// buffers, the next step's on their way to the other (halves: four blocks of 32
-// tokens to a CU, or two of 64).  At D = 2048, FF = 512, E = 256, k = 8 what bounds
+// A step is half a superblock: its activations are in one of two LDS buffers, the
+// next step's on their way to the other (four blocks of 32 tokens to a CU, or three
+// of 64).  IQ3_XXS rows come to registers, 16 rows a load: as decoded there they
+// have not been tried through LDS.  At D = 2048, FF = 512, E = 256, k = 8 what bounds
 // it is near even at T = 512: loads and barriers alone take 87 us (the rows' 285 MB
 // at 3.3 TB/s and as many activation bytes from L2), decoding and MFMA alone 76,
 // together 97 (113 with 16 rows to a load and the rows held in registers); at
 // T = 4096, in segments of 64, 315 (416 in segments of 32, decoded twice as often).
-template <int QT, int ST, int NH>
+template <int QT, int ST>
 struct GuShape {
-  static constexpr int ROWB = 512 / NH, TILE = ST * ROWB;              // bytes of an activation row and buffer
+  static constexpr int ROWB = 256, TILE = ST * ROWB;              // bytes of an activation row and buffer
   static constexpr int G = ROWB / 16, NI = 16 * ROWB / 4096;           // granules per row, DMAs per wave and token tile
   static constexpr int WBYTES = QT == GM_QTYPE_IQ4_XS ? 4 * kIq4Loads * 1024 : 256 * 4 + 128 * 4;   // rows' way / tables
   static constexpr size_t SMEM = 2 * TILE + WBYTES + 2 * ST * 4;
@@ -845,13 +846,13 @@ __device__ __forceinline__ void act_lds_load(const uint16_t* const (&ptr)[NI], i
 }
 
 // The K loop over NT token tiles.
-template <int QT, int ST, int NH, int NT>
+template <int QT, int ST, int NT>
 __device__ __forceinline__ void gu_loop(const uint8_t* __restrict__ gt, const uint8_t* __restrict__ ut, int64_t rb,
-                                        int nsb, const uint16_t* const (&xp)[NT * GuShape<QT, ST, NH>::NI],
+                                        int nsb, const uint16_t* const (&xp)[NT * GuShape<QT, ST>::NI],
                                         uint8_t* __restrict__ xl, uint8_t* __restrict__ wbuf,
                                         const uint32_t* __restrict__ grid, const uint32_t* __restrict__ sgn,
                                         gm_f32x4 (&ag)[NT], gm_f32x4 (&au)[NT]) {
-  using S = GuShape<QT, ST, NH>;
+  using S = GuShape<QT, ST>;
   constexpr bool IQ4 = QT == GM_QTYPE_IQ4_XS;
   constexpr int SBB = IQ4 ? GM_IQ4XS_BYTES : GM_IQ3XXS_BYTES;
   const int lane = threadIdx.x & 63, q = lane >> 4, l16 = lane & 15;
@@ -879,10 +880,7 @@ __device__ __forceinline__ void gu_loop(const uint8_t* __restrict__ gt, const ui
       wu = iq4_lds_read(wbuf + kIq4Tile, l16, q);
       lds_reads_done();
     }
-    uint8_t* const x0 = xl + (NH == 1 && (sb & 1) ? S::TILE : 0);
-    uint8_t* const x1 = xl + (NH == 1 && (sb & 1) ? 0 : S::TILE);
-    if (NH == 2) act_lds_load<NT * S::NI>(xp, sb * kChunk + 32, x1);
-    else if (more) act_lds_load<NT * S::NI>(xp, (sb + 1) * kChunk, x1);
+    act_lds_load<NT * S::NI>(xp, sb * kChunk + 32, xl + S::TILE);
     if constexpr (IQ4) {
       if (more) iq4_lds_load(gt + (sb + 1) * SBB, woff, wbuf);
     } else {
@@ -894,13 +892,11 @@ __device__ __forceinline__ void gu_loop(const uint8_t* __restrict__ gt, const ui
     gm_f32x4 pg[NT], pu[NT];
 #pragma unroll
     for (int t = 0; t < NT; ++t) { pg[t] = gm_f32x4{0.f, 0.f, 0.f, 0.f}; pu[t] = pg[t]; }
-    gu_half<QT, NT, NH, 0>(wg, wu, sg, su, q, l16, x0, grid, sgn, pg, pu);
-    if constexpr (NH == 2) {
-      __builtin_amdgcn_s_waitcnt(0);
-      __syncthreads();
-      if (more) act_lds_load<NT * S::NI>(xp, (sb + 1) * kChunk, x0);
-    }
-    gu_half<QT, NT, NH, 1>(wg, wu, sg, su, q, l16, NH == 2 ? x1 : x0, grid, sgn, pg, pu);
+    gu_half<QT, NT, 0>(wg, wu, sg, su, q, l16, xl, grid, sgn, pg, pu);
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    if (more) act_lds_load<NT * S::NI>(xp, (sb + 1) * kChunk, xl);
+    gu_half<QT, NT, 1>(wg, wu, sg, su, q, l16, xl + S::TILE, grid, sgn, pg, pu);
     pf_fold<NT>(pf_dscale<QT>(wg), q, pg, ag);
     pf_fold<NT>(pf_dscale<QT>(wu), q, pu, au);
     if constexpr (!IQ4) {
@@ -912,12 +908,12 @@ __device__ __forceinline__ void gu_loop(const uint8_t* __restrict__ gt, const ui
   }
 }
 
-template <int QT, int ST, int NH>
+template <int QT, int ST>
 __global__ void __launch_bounds__(256, ST == 32 ? 4 : 3) k_pf_gateup(
     gm_moe_layer P, const int32_t* __restrict__ segs, const int32_t* __restrict__ offsets,
     const int32_t* __restrict__ sorted, const uint16_t* __restrict__ xh, const float* __restrict__ xsc,
     uint16_t* __restrict__ hb, int T, int n_row_tiles) {
-  using S = GuShape<QT, ST, NH>;
+  using S = GuShape<QT, ST>;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   uint8_t* xl = smem;                                                   // [2][ST][ROWB]
   uint8_t* wl = smem + 2 * S::TILE;                                     // [4 waves][gate, up tile, padding] (IQ4)
@@ -962,10 +958,10 @@ __global__ void __launch_bounds__(256, ST == 32 ? 4 : 3) k_pf_gateup(
 #pragma unroll
     for (int m = 0; m < NT * S::NI; ++m) {
       const int id = 64 * (wave * (NT * S::NI) + m) + lane, r = id / S::G, g = (id % S::G) ^ (r & 15);
-      xp[m] = xh + (int64_t)tok_row[r] * D + 8 * (NH == 1 ? g : 8 * (g >> 2) + (g & 3));
+      xp[m] = xh + (int64_t)tok_row[r] * D + 8 * (8 * (g >> 2) + (g & 3));
     }
     gm_f32x4 ag[NT], au[NT];
-    gu_loop<QT, ST, NH, NT>(gbase + tile, ubase + tile, rb, D / kChunk, xp, xl, wl + wave * kIq4Loads * 1024, grid, sgn, ag,
+    gu_loop<QT, ST, NT>(gbase + tile, ubase + tile, rb, D / kChunk, xp, xl, wl + wave * kIq4Loads * 1024, grid, sgn, ag,
                             au);
     // C layout: lane l holds rows 4 (l / 16) + i of the 16-row tile, column l % 16
 #pragma unroll
@@ -1096,12 +1092,12 @@ __global__ void __launch_bounds__(64 * NW, NSB > 2 ? 1 : 2) k_pf_down(gm_moe_lay
   });
 }
 
-template <int QT, int ST, int NH>
+template <int QT, int ST>
 int launch_gateup(const gm_moe_layer* L, const PfWs& w, int nseg, int T, hipStream_t s) {
   const int nrt = L->FF / 64;
-  constexpr size_t smem = GuShape<QT, ST, NH>::SMEM;
-  if (int rc = gm_set_smem(k_pf_gateup<QT, ST, NH>, smem)) return rc;
-  hipLaunchKernelGGL((k_pf_gateup<QT, ST, NH>), dim3((nseg + 7) / 8 * 8 * nrt), dim3(256), smem, s, *L, w.segs,
+  constexpr size_t smem = GuShape<QT, ST>::SMEM;
+  if (int rc = gm_set_smem(k_pf_gateup<QT, ST>, smem)) return rc;
+  hipLaunchKernelGGL((k_pf_gateup<QT, ST>), dim3((nseg + 7) / 8 * 8 * nrt), dim3(256), smem, s, *L, w.segs,
                      w.offsets, w.sorted, w.xh, w.xsc, w.hb, T, nrt);
   GM_TRY(hipGetLastError());
   return GM_OK;
@@ -1445,7 +1441,7 @@ int prefill_t(const gm_moe_layer* L, const float* x, float* y, int T, int flags,
     if (int rc = gm_launch_gateup(L->q_gate_sh, L->gate_sh, L->up_sh, FF, D, w.xn, T, w.hsh, s)) return rc;
     if (int rc = gm_launch_matvec(L->q_down_sh, L->down_sh, D, FF, w.hsh, T, w.yp + P * D, s)) return rc;
   }
-  if (int rc = seg == 64 ? launch_gateup<QTG, 64, 2>(L, w, nseg, T, s) : launch_gateup<QTG, 32, 2>(L, w, nseg, T, s))
+  if (int rc = seg == 64 ? launch_gateup<QTG, 64>(L, w, nseg, T, s) : launch_gateup<QTG, 32>(L, w, nseg, T, s))
     return rc;
   if (sh_i8) {                                       // shared SwiGLU rows hb[P + t] (D % 256 == 0)
     const int nkw = sh_kparts(D / 32), tok = 16 * kShTiles * (4 / nkw);    // tokens per block
