@@ -153,8 +153,9 @@ bool gm_pf8_ok(const gm_moe_layer* L);
 size_t gm_pf8_scratch_bytes(const gm_moe_layer* L, int T);
 int gm_pf8_run(const gm_moe_layer* L, const float* x, float* y, int T, int flags, uint8_t* ws, const GmMoeWs& lay,
                hipStream_t s);
-// Their GEMMs (prefill_i8.hip) on activation rows split into two f16 planes;
-// seg_tok: 16 or 32 tokens at most per segment.
+// Their GEMMs (prefill_i8.hip) on activation rows split into two f16 planes, over
+// segments of at most kPf8Seg tokens.
+constexpr int kPf8Seg = 16;
 struct GmPf8Rows {
   uint16_t* hi;
   uint16_t* lo;
@@ -162,7 +163,7 @@ struct GmPf8Rows {
 };
 int gm_pf8_split(const float* src, int rows, int K, const GmPf8Rows& a, hipStream_t s);
 int gm_pf8_gemm(const gm_moe_layer* L, bool down, const GmPf8Rows& a, const int32_t* segs, int nseg,
-                const int32_t* offsets, const int32_t* sorted, int T, int seg_tok, float* out, hipStream_t s);
+                const int32_t* offsets, const int32_t* sorted, int T, float* out, hipStream_t s);
 int gm_launch_dispatch(const int32_t* ids, int T, int k, int E, int32_t* counts, int32_t* offsets,
                        int32_t* sorted_pairs, hipStream_t s);
 // Dispatch plus (inv != NULL) the inverse permutation and (segs != NULL) the

@@ -118,10 +118,6 @@ int pf_seg(const gm_moe_layer* L, int T) {
   return L->FF <= 2 * kChunk && pairs >= 28 * (int64_t)L->E && pairs / 64 * (L->FF / 64) >= 512 ? 64 : kSegMin;
 }
 
-// Tokens per segment of the I8 GEMMs: 16 while the experts have about that many
-// (one MFMA tile, two blocks to a CU), else 32.
-int pf8_seg(const gm_moe_layer* L, int T) { return T * L->k <= 24 * L->E ? 16 : 32; }
-
 PfWs pf_layout(const gm_moe_layer* L, int T, uint8_t* base, size_t* total) {
   const size_t P = (size_t)T * L->k, E = L->E;
   size_t o = 0;
@@ -1495,7 +1491,7 @@ bool gm_pf8_ok(const gm_moe_layer* L) {
 }
 
 struct Pf8Ws {
-  int32_t* segs;       // the segment list (more segments than PfWs's where they are of 16)
+  int32_t* segs;       // the segment list (of kPf8Seg tokens: more of them than PfWs's)
   float* xn;           // [T][D] fp32 rows
   float* h;            // [P + T][FF] fp32 SwiGLU rows
   GmPf8Rows xr, hr;    // their planes (hi of both and lo of h in PfWs's f16 rows)
@@ -1506,7 +1502,7 @@ static Pf8Ws pf8_layout(const gm_moe_layer* L, int T, const PfWs& w, uint8_t* ba
   size_t o = 0;
   auto take = [&](size_t bytes) { uint8_t* p = base ? base + o : nullptr; o = align256(o + bytes); return p; };
   Pf8Ws v{};
-  v.segs = reinterpret_cast<int32_t*>(take((1 + 4 * (size_t)max_segments(T, L->k, L->E, pf8_seg(L, T))) * 4));
+  v.segs = reinterpret_cast<int32_t*>(take((1 + 4 * (size_t)max_segments(T, L->k, L->E, kPf8Seg)) * 4));
   v.xn = reinterpret_cast<float*>(take(T * D * 4));
   v.xr = GmPf8Rows{w.xh, reinterpret_cast<uint16_t*>(take(T * D * 2)), reinterpret_cast<float*>(take(T * (D / 32) * 8))};
   v.h = reinterpret_cast<float*>(take((P + T) * FF * 4));
@@ -1527,12 +1523,12 @@ int gm_pf8_run(const gm_moe_layer* L, const float* x, float* y, int T, int flags
   const PfWs w = pf_layout(L, T, ws + lay.pre, nullptr);
   const Pf8Ws v = pf8_layout(L, T, w, ws + lay.pre8, nullptr);
   const bool has_sh = L->gate_sh != nullptr;
-  const int seg = pf8_seg(L, T), nseg = max_segments(T, k, L->E, seg);
-  if (int rc = pf_route(L, x, T, ws, lay, w, v.xn, has_sh ? T : 0, v.segs, seg, s)) return rc;
+  const int nseg = max_segments(T, k, L->E, kPf8Seg);
+  if (int rc = pf_route(L, x, T, ws, lay, w, v.xn, has_sh ? T : 0, v.segs, kPf8Seg, s)) return rc;
   if (int rc = gm_pf8_split(v.xn, T, D, v.xr, s)) return rc;
-  if (int rc = gm_pf8_gemm(L, false, v.xr, v.segs, nseg, w.offsets, w.sorted, T, seg, v.h, s)) return rc;
+  if (int rc = gm_pf8_gemm(L, false, v.xr, v.segs, nseg, w.offsets, w.sorted, T, v.h, s)) return rc;
   if (int rc = gm_pf8_split(v.h, T * k + (has_sh ? T : 0), FF, v.hr, s)) return rc;
-  if (int rc = gm_pf8_gemm(L, true, v.hr, v.segs, nseg, w.offsets, w.sorted, T, seg, w.yp, s)) return rc;
+  if (int rc = gm_pf8_gemm(L, true, v.hr, v.segs, nseg, w.offsets, w.sorted, T, w.yp, s)) return rc;
   hipLaunchKernelGGL(k_pf_combine, dim3(T), dim3(256), 0, s, x, w.yp, w.inv, reinterpret_cast<float*>(ws + lay.wts),
                      reinterpret_cast<float*>(ws + lay.shg), T, k, D, has_sh ? 1 : 0, flags, y);
   GM_TRY(hipGetLastError());

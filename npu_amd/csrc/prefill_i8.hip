@@ -1,7 +1,7 @@
 // Grouped GEMMs over routed experts held as I8 rows (Q8_0 / Q4_K / Q5_K / Q6_K
-// tensors, transcoded), for the MoE prefill (prefill.hip): segments of at
-// most 16 or 32 tokens per expert, with activations no less exact than the decode
-// kernels of these layers have them.
+// tensors, transcoded), for the MoE prefill (prefill.hip): segments of at most 16
+// tokens per expert, with activations no less exact than the decode kernels of
+// these layers have them.
 //
 // Activations: each sub-block of 32 times a power of two (its largest magnitude in
 // [2^14, 2^15)), split into two f16 planes hi + lo (hi rounded, lo the rest
@@ -105,7 +105,7 @@ struct Gemm8 {
   int T, k, E, M, K, nrt;
 };
 
-// Block = (segment of at most 16 NT tokens, RTB tiles of 64 weight rows): wave w rows
+// Block = (segment of at most 16 tokens, RTB tiles of 64 weight rows): wave w rows
 // 16 w .. 16 w + 15 of a tile of NMAT matrices, all of the segment's tokens.
 // NMAT = 2: out = silu(gate) up; 1: out = the down row.
 //
@@ -115,9 +115,11 @@ struct Gemm8 {
 // covers 5 1/3 weight rows of 192 contiguous bytes; loaded to registers as the MFMA
 // wants them, 16 rows by an instruction, they came at 2.3 TB/s whatever was in
 // flight (a probe of the two patterns alone: 3.1 and 6.9 TB/s).  Two buffers and
-// two (gate/up) or three (down) blocks of 16 tokens to a CU: one block with four or
-// seven buffers had as much in flight but one wave per SIMD.  A gate/up block of 32
-// tokens is alone on its CU, two of them do not fit its LDS.
+// two (gate/up) or three (down) blocks to a CU: one block with four or seven buffers
+// had as much in flight but one wave per SIMD.  Segments of 32 tokens leave one
+// gate/up block to a CU, and are slower however many tokens an expert has (block at
+// D = 2048, FF = 512, 256 experts, k = 8: T = 500 559 against 422 us, 1000 794 / 678,
+// 2500 1568 / 1431; at D = 512, FF = 256, 16 experts, k = 4: 100 49 / 43, 1000 85 / 81).
 // D = 2048, FF = 512, 256 experts, 150 tokens (Q5_K / Q6_K, 1.2 GB of I8 rows), us:
 //   gate/up 348 (16 rows an instruction) -> 270 (through LDS) -> 217 (a step's LDS
 //   reads together, the next loads not waited for before them); down 177 -> 123
@@ -126,10 +128,10 @@ struct Gemm8 {
 // and 101 (the activations' addresses are formed once, not per step).
 // Granule g (16 bytes) of row r's step sits at position (g + 2 (r >> 2)) % 12 of
 // its 12: the 16 rows' reads of 32 bytes fall evenly on the banks.
-template <int NMAT, int NT, int RTB>
+template <int NMAT, int RTB>
 __global__ void __launch_bounds__(256) k_pf8_gemm(Gemm8 P) {
   constexpr int kStep = 128, kRowB = 2 * kStep, kWRow = 192, NW = 4;
-  constexpr int SEG = 16 * NT, PLANE = SEG * kRowB, NA = 2 * PLANE / 1024 / NW;   // act loads per wave and step
+  constexpr int SEG = kPf8Seg, PLANE = SEG * kRowB, NA = 2 * PLANE / 1024 / NW;   // act loads per wave and step
   constexpr int WB = NMAT * 16 * kWRow;                         // a wave's weight bytes per step
   constexpr int STAGE = 2 * PLANE + NW * WB + 8 * SEG * 4;      // planes, weights, meta [4][sum, scale][SEG]
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];   // [2][STAGE], then
@@ -190,11 +192,9 @@ __global__ void __launch_bounds__(256) k_pf8_gemm(Gemm8 P) {
     for (int m = 0; m < NA; ++m) to_lds<16>(ap[m] + s * kStep, st + (NA * wave + m) * 1024);
     if (brings) to_lds<4>(mp + s * 8, st + 2 * PLANE + NW * WB + wave * 256);
   };
-  gm_f32x4 acc[NMAT][NT];
+  gm_f32x4 acc[NMAT];
 #pragma unroll
-  for (int i = 0; i < NMAT; ++i)
-#pragma unroll
-    for (int t = 0; t < NT; ++t) acc[i][t] = gm_f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < NMAT; ++i) acc[i] = gm_f32x4{0.f, 0.f, 0.f, 0.f};
   load(0, 0);
   const bool low = q < 2;                                       // the lane's octet is in the first half
   for (int it = 0; it < total; ++it) {
@@ -204,87 +204,72 @@ __global__ void __launch_bounds__(256) k_pf8_gemm(Gemm8 P) {
     const uint8_t* st = smem + (it & 1) * STAGE;
     const uint8_t* wb = st + 2 * PLANE + wave * WB;
     const float* meta = reinterpret_cast<const float*>(st + 2 * PLANE + NW * WB);
-    gm_f32x4 part[NMAT][NT];                                    // the step's sums: a fourth of the running sum's additions
-    constexpr int GS = NT == 1 ? 4 : 2;                         // sub-blocks whose LDS reads go out together
+    gm_f32x4 part[NMAT];                                        // the step's sums: a fourth of the running sum's additions
+    gm_f16x8 ah[4], al[4];                                      // the LDS reads of all four sub-blocks go out together
+    gm_f32x4 xs[4], xe[4], sc[4][NMAT];                         // sums, scales; sc: s0, s1, off
+    gm_u32x2 w[4][NMAT];
 #pragma unroll
-    for (int s0 = 0; s0 < 4; s0 += GS) {
-      gm_f16x8 ah[GS][NT], al[GS][NT];
-      gm_f32x4 xs[GS][NT], xe[GS][NT], sc[GS][NMAT];            // sums, scales; sc: s0, s1, off
-      gm_u32x2 w[GS][NMAT];
+    for (int s = 0; s < 4; ++s) {
 #pragma unroll
-      for (int u = 0; u < GS; ++u) {
-        const int s = s0 + u;
+      for (int i = 0; i < NMAT; ++i) {
+        w[s][i] = *reinterpret_cast<const gm_u32x2*>(wb + i * 16 * kWRow + qo[s]);
+        sc[s][i] = *reinterpret_cast<const gm_f32x4*>(wb + i * 16 * kWRow + mo[s]);
+      }
+      const int o = l16 * kRowB + 16 * ((4 * s + q) ^ l16);
+      ah[s] = *reinterpret_cast<const gm_f16x8*>(st + o);
+      al[s] = *reinterpret_cast<const gm_f16x8*>(st + PLANE + o);
+      xs[s] = *reinterpret_cast<const gm_f32x4*>(meta + 2 * s * SEG + 4 * q);
+      xe[s] = *reinterpret_cast<const gm_f32x4*>(meta + (2 * s + 1) * SEG + 4 * q);
+    }
+    issue_fence();
 #pragma unroll
-        for (int i = 0; i < NMAT; ++i) {
-          w[u][i] = *reinterpret_cast<const gm_u32x2*>(wb + i * 16 * kWRow + qo[s]);
-          sc[u][i] = *reinterpret_cast<const gm_f32x4*>(wb + i * 16 * kWRow + mo[s]);
-        }
+    for (int s = 0; s < 4; ++s)
 #pragma unroll
-        for (int t = 0; t < NT; ++t) {
-          const int o = (16 * t + l16) * kRowB + 16 * ((4 * s + q) ^ l16);
-          ah[u][t] = *reinterpret_cast<const gm_f16x8*>(st + o);
-          al[u][t] = *reinterpret_cast<const gm_f16x8*>(st + PLANE + o);
-          xs[u][t] = *reinterpret_cast<const gm_f32x4*>(meta + 2 * s * SEG + 16 * t + 4 * q);
-          xe[u][t] = *reinterpret_cast<const gm_f32x4*>(meta + (2 * s + 1) * SEG + 16 * t + 4 * q);
+      for (int i = 0; i < NMAT; ++i) {
+        uint32_t o[4];
+        i8x4_f16(w[s][i].x, o[0], o[1]);
+        i8x4_f16(w[s][i].y, o[2], o[3]);
+        const gm_u32x4 b0 = {low ? o[0] : 0u, low ? o[1] : 0u, low ? o[2] : 0u, low ? o[3] : 0u};
+        const gm_u32x4 b1 = {low ? 0u : o[0], low ? 0u : o[1], low ? 0u : o[2], low ? 0u : o[3]};
+        const gm_f16x8 B0 = __builtin_bit_cast(gm_f16x8, b0), B1 = __builtin_bit_cast(gm_f16x8, b1);
+        const gm_f32x4 z = {0.f, 0.f, 0.f, 0.f};
+        gm_f32x4 d0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[s], B0, z, 0, 0, 0);
+        gm_f32x4 d1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[s], B1, z, 0, 0, 0);
+        d0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[s], B0, d0, 0, 0, 0);
+        d1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[s], B1, d1, 0, 0, 0);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const float v = fmaf(sc[s][i].x, d0[c], fmaf(sc[s][i].y, d1[c], sc[s][i].z * xs[s][c]));
+          part[i][c] = s == 0 ? xe[s][c] * v : fmaf(xe[s][c], v, part[i][c]);
         }
       }
-      issue_fence();
 #pragma unroll
-      for (int u = 0; u < GS; ++u)
-#pragma unroll
-        for (int i = 0; i < NMAT; ++i) {
-          uint32_t o[4];
-          i8x4_f16(w[u][i].x, o[0], o[1]);
-          i8x4_f16(w[u][i].y, o[2], o[3]);
-          const gm_u32x4 b0 = {low ? o[0] : 0u, low ? o[1] : 0u, low ? o[2] : 0u, low ? o[3] : 0u};
-          const gm_u32x4 b1 = {low ? 0u : o[0], low ? 0u : o[1], low ? 0u : o[2], low ? 0u : o[3]};
-          const gm_f16x8 B0 = __builtin_bit_cast(gm_f16x8, b0), B1 = __builtin_bit_cast(gm_f16x8, b1);
-#pragma unroll
-          for (int t = 0; t < NT; ++t) {
-            const gm_f32x4 z = {0.f, 0.f, 0.f, 0.f};
-            gm_f32x4 d0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[u][t], B0, z, 0, 0, 0);
-            gm_f32x4 d1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[u][t], B1, z, 0, 0, 0);
-            d0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[u][t], B0, d0, 0, 0, 0);
-            d1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[u][t], B1, d1, 0, 0, 0);
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-              const float v = fmaf(sc[u][i].x, d0[c], fmaf(sc[u][i].y, d1[c], sc[u][i].z * xs[u][t][c]));
-              part[i][t][c] = s0 + u == 0 ? xe[u][t][c] * v : fmaf(xe[u][t][c], v, part[i][t][c]);
-            }
-          }
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < NMAT; ++i)
-#pragma unroll
-      for (int t = 0; t < NT; ++t) acc[i][t] += part[i][t];
+    for (int i = 0; i < NMAT; ++i) acc[i] += part[i];
     if ((it + 1) % ns == 0) {
-      // a row tile is done: lane l holds tokens 4 (l / 16) + i of a token tile, weight row l % 16
+      // a row tile is done: lane l holds tokens 4 (l / 16) + i, weight row l % 16
       const int row = row0 + (it / ns) * 16 * NW + l16;
 #pragma unroll
-      for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int c = 16 * t + 4 * q + i;
-          if (c < n) {
-            float v = acc[0][t][i];
-            if constexpr (NMAT == 2) v = gm_silu(v) * acc[NMAT - 1][t][i];
-            P.out[(int64_t)out_row[c] * P.M + row] = v;
-          }
-#pragma unroll
-          for (int m = 0; m < NMAT; ++m) acc[m][t][i] = 0.f;
+      for (int i = 0; i < 4; ++i) {
+        const int c = 4 * q + i;
+        if (c < n) {
+          float v = acc[0][i];
+          if constexpr (NMAT == 2) v = gm_silu(v) * acc[NMAT - 1][i];
+          P.out[(int64_t)out_row[c] * P.M + row] = v;
         }
+#pragma unroll
+        for (int m = 0; m < NMAT; ++m) acc[m][i] = 0.f;
+      }
     }
   }
 }
 
-template <int NMAT, int NT, int RTB>
+template <int NMAT, int RTB>
 int launch8(Gemm8 P, int nseg, hipStream_t s) {
-  constexpr size_t smem = 2 * (2 * 16 * NT * 256 + 4 * NMAT * 16 * 192 + 8 * 16 * NT * 4) + 2 * 16 * NT * 4;
-  static_assert((NT > 1 ? 1 : NMAT == 2 ? 2 : 3) * smem <= 160 * 1024, "LDS of a CU");
+  constexpr size_t smem = 2 * (2 * kPf8Seg * 256 + 4 * NMAT * 16 * 192 + 8 * kPf8Seg * 4) + 2 * kPf8Seg * 4;
+  static_assert((NMAT == 2 ? 2 : 3) * smem <= 160 * 1024, "LDS of a CU");
   P.nrt = P.M / (64 * RTB);
-  if (int rc = gm_set_smem(k_pf8_gemm<NMAT, NT, RTB>, smem)) return rc;
-  hipLaunchKernelGGL((k_pf8_gemm<NMAT, NT, RTB>), dim3((unsigned)((nseg + 7) / 8 * 8 * P.nrt)), dim3(256), smem, s, P);
+  if (int rc = gm_set_smem(k_pf8_gemm<NMAT, RTB>, smem)) return rc;
+  hipLaunchKernelGGL((k_pf8_gemm<NMAT, RTB>), dim3((unsigned)((nseg + 7) / 8 * 8 * P.nrt)), dim3(256), smem, s, P);
   GM_TRY(hipGetLastError());
   return GM_OK;
 }
@@ -298,7 +283,7 @@ int gm_pf8_split(const float* src, int rows, int K, const GmPf8Rows& a, hipStrea
 }
 
 int gm_pf8_gemm(const gm_moe_layer* L, bool down, const GmPf8Rows& a, const int32_t* segs, int nseg,
-                const int32_t* offsets, const int32_t* sorted, int T, int seg_tok, float* out, hipStream_t s) {
+                const int32_t* offsets, const int32_t* sorted, int T, float* out, hipStream_t s) {
   const int M = down ? L->D : L->FF, K = down ? L->FF : L->D;
   auto u8 = [](const void* p) { return static_cast<const uint8_t*>(p); };
   Gemm8 P{};
@@ -309,9 +294,5 @@ int gm_pf8_gemm(const gm_moe_layer* L, bool down, const GmPf8Rows& a, const int3
   P.hi = a.hi; P.lo = a.lo; P.meta = a.meta;
   P.out = out; P.segs = segs; P.offsets = offsets; P.sorted = down ? nullptr : sorted;
   P.T = T; P.k = L->k; P.E = L->E; P.M = M; P.K = K;
-  // M % 256 == 0: whole tiles
-  if (seg_tok == 16 && down) return launch8<1, 1, 4>(P, nseg, s);
-  if (seg_tok == 16) return launch8<2, 1, 1>(P, nseg, s);
-  if (down) return launch8<1, 2, 4>(P, nseg, s);
-  return launch8<2, 2, 1>(P, nseg, s);
+  return down ? launch8<1, 4>(P, nseg, s) : launch8<2, 1>(P, nseg, s);   // M % 256 == 0: whole tiles
 }
