@@ -380,9 +380,10 @@ int gm_rms_norm(const float* x, const float* w, int D, int n_rows, float eps, fl
  * library holds until the process ends.  No counterpart in the reference; it
  * is for callers that cannot allocate (code under stream / graph capture,
  * tight serving loops, harnesses that forbid hipMalloc).  Same kernels and
- * results as gm_moe_forward.  Returns GM_EWORKSPACE when
- * gm_moe_workspace_bytes(L, T) > GM_NOALLOC_SCRATCH_BYTES (config 5: T <= 8
- * needs 1.7 MiB, prefill fits up to T = 111).  stream must belong to the
+ * results as gm_moe_forward.  Returns GM_EWORKSPACE when the smallest workspace
+ * that gm_moe_forward takes for T tokens (gm_moe_workspace_bytes(L, T); with I8
+ * routed experts less, see gm_moe_prefill) is above GM_NOALLOC_SCRATCH_BYTES
+ * (config 5: T <= 8 needs 1.7 MiB, prefill fits up to T = 111).  stream must belong to the
  * current device.  The first call on each device resolves the array's address
  * (hipGetSymbolAddress, which may load the code object) and so must happen
  * outside stream capture; later calls may be captured.  All calls on one GPU share that GPU's array, which keeps

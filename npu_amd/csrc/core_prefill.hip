@@ -741,8 +741,9 @@ __global__ void __launch_bounds__(256) k_pf_gnorm(float* __restrict__ o, const f
 struct AttnWs { size_t h, qkv, out, part, total; int nblk, nsplit; };
 
 // Key parts: the blocks of a few tokens do not fill the chip, so their keys are
-// cut until there are about two blocks per CU, each part at least 128 keys (16
-// parts at most).  keys: cached positions with the prompt's own.
+// cut until there are about two blocks per CU: one part per 128 keys begun (129
+// keys: two of 80 and 49) and 16 parts at most.  keys: cached positions with the
+// prompt's own.
 AttnWs attn_layout(const gm_attn_layer* L, int T, int keys) {
   AttnWs w{};
   const size_t Dh = (size_t)L->head_dim, Hq = (size_t)L->n_head, Hkv = (size_t)L->n_head_kv, Tz = (size_t)T;

@@ -161,7 +161,9 @@ class GpuAttn:
     def prompt(self, x: torch.Tensor, cache: "KVCache", pos: int, cos: torch.Tensor, sin: torch.Tensor,
                residual: bool, out: torch.Tensor) -> None:
         """x [T, D], positions pos .. pos + T - 1, in one call (gm_attn_prefill).  The
-        workspace (61 KB a token, at most 1024 tokens' worth) is the call's own."""
+        workspace is the call's own: at the model's shape 60 KB a token and 16 KB for each part
+        that its keys are cut into (95 KB a token at 1024 tokens, 328 KB at 128 and below), at
+        most 1024 tokens' worth."""
         T = x.shape[0]
         n = L.lib().gm_attn_prefill_workspace_bytes(ctypes.byref(self.struct), T, cache.max_pos)
         if n == 0:
@@ -318,8 +320,8 @@ class GpuSsm:
         L.check(rc, "gm_ssm_decode_moe")
 
     def prompt(self, x: torch.Tensor, state, residual: bool, out: torch.Tensor) -> None:
-        """x [T, D] in one call (gm_ssm_prefill).  The workspace (108 KB a token, at most
-        1024 tokens' worth) is the call's own."""
+        """x [T, D] in one call (gm_ssm_prefill).  The workspace (105 KB a token at the
+        model's shape, at most 1024 tokens' worth) is the call's own."""
         conv, S = state
         T = x.shape[0]
         n = L.lib().gm_ssm_prefill_workspace_bytes(ctypes.byref(self.struct), T)
