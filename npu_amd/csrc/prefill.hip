@@ -280,6 +280,11 @@ __device__ __forceinline__ void pf_prep_token(int t, const float* __restrict__ x
 // w = w0 + w1 + w2 exactly (each piece holds the next 8 significant bits of
 // the 24; exact unless |w| < 2^-100, where bf16 subnormals cut the last
 // piece), and all nine piece products are accumulated.
+// FOLD (layers with I8 experts, whose logits came from the decode kernels' fp32 FMAs
+// before they had these GEMMs): a k-step is summed by itself, the lower pieces
+// first, every other one of -x (neg), which cancels the MFMA's rounding towards
+// -infinity; error of the logits against 64 bits at D = 2048 1.7e-7 -> 1.0e-7 (one
+// token at a time 1.1e-7).
 __device__ __forceinline__ void split3_bf16(const gm_u32x4 (&r)[2], gm_bf16x8 (&o)[3]) {
   gm_f32x8 v;
   v[0] = __uint_as_float(r[0].x); v[1] = __uint_as_float(r[0].y);
@@ -293,11 +298,12 @@ __device__ __forceinline__ void split3_bf16(const gm_u32x4 (&r)[2], gm_bf16x8 (&
   o[2] = __builtin_convertvector(r1, gm_bf16x8);
 }
 
-template <bool RF32>
-__device__ __forceinline__ void router_step(const gm_u32x4 (&a)[4][RF32 ? 2 : 1], const gm_u32x4 (&b)[3],
+template <bool RF32, bool FOLD>
+__device__ __forceinline__ void router_step(const gm_u32x4 (&a)[4][RF32 ? 2 : 1], const gm_u32x4 (&b)[3], bool neg,
                                             gm_f32x4 (&acc)[4]) {
 #pragma unroll
   for (int rt = 0; rt < 4; ++rt) {
+    gm_f32x4 d = FOLD ? gm_f32x4{0.f, 0.f, 0.f, 0.f} : acc[rt];
     if constexpr (RF32) {
       gm_bf16x8 ap[3];
       split3_bf16(a[rt], ap);
@@ -305,18 +311,19 @@ __device__ __forceinline__ void router_step(const gm_u32x4 (&a)[4][RF32 ? 2 : 1]
       for (int pa = 0; pa < 3; ++pa)
 #pragma unroll
         for (int p = 0; p < 3; ++p)
-          acc[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ap[pa], __builtin_bit_cast(gm_bf16x8, b[p]), acc[rt], 0,
-                                                            0, 0);
+          d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ap[FOLD ? 2 - pa : pa],
+                                                      __builtin_bit_cast(gm_bf16x8, b[FOLD ? 2 - p : p]), d, 0, 0, 0);
     } else {
 #pragma unroll
       for (int p = 0; p < 3; ++p)
-        acc[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gm_bf16x8, a[rt][0]),
-                                                          __builtin_bit_cast(gm_bf16x8, b[p]), acc[rt], 0, 0, 0);
+        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gm_bf16x8, a[rt][0]),
+                                                    __builtin_bit_cast(gm_bf16x8, b[FOLD ? 2 - p : p]), d, 0, 0, 0);
     }
+    acc[rt] = !FOLD ? d : neg ? acc[rt] - d : acc[rt] + d;
   }
 }
 
-template <int NK, bool RF32>
+template <int NK, bool RF32, bool FOLD>
 __device__ __forceinline__ void pf_router_block(int rb, int tb, int z, const void* __restrict__ w,
                                                 const void* __restrict__ wsh, const float* __restrict__ x,
                                                 const float* __restrict__ norm_w, int T, int D, int E, int ldp,
@@ -357,14 +364,15 @@ __device__ __forceinline__ void pf_router_block(int rb, int tb, int z, const voi
     gm_u32x4 xw[2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const gm_f32x4 v = norm_w ? xv[ks][h] * nv[ks][h] : xv[ks][h];
+      gm_f32x4 v = norm_w ? xv[ks][h] * nv[ks][h] : xv[ks][h];
+      if (FOLD && (ks & 1)) v = -v;
       xw[h] = __builtin_bit_cast(gm_u32x4, v);
     }
     gm_bf16x8 pl[3];
     split3_bf16(xw, pl);
     const gm_u32x4 b[3] = {__builtin_bit_cast(gm_u32x4, pl[0]), __builtin_bit_cast(gm_u32x4, pl[1]),
                            __builtin_bit_cast(gm_u32x4, pl[2])};
-    router_step<RF32>(a[ks], b, acc);
+    router_step<RF32, FOLD>(a[ks], b, ks & 1, acc);
   }
   if (wave > 0) {
 #pragma unroll
@@ -392,7 +400,7 @@ __device__ __forceinline__ void pf_router_block(int rb, int tb, int z, const voi
 // nrb, b / nrb % ntb, b / (nrb ntb)); blocks [n_rt, n_rt + T): the prep of
 // token b - n_rt.  The two roles share nothing: the launch replaces a prep
 // launch followed by a router launch.
-template <int NK, bool RF32>
+template <int NK, bool RF32, bool FOLD>
 __global__ void __launch_bounds__(256) k_pf_prep_router(const void* __restrict__ w, const void* __restrict__ wsh,
                                                         const float* __restrict__ x, const float* __restrict__ norm_w,
                                                         float eps, int T, int D, int E, int ldp,
@@ -406,7 +414,7 @@ __global__ void __launch_bounds__(256) k_pf_prep_router(const void* __restrict__
     pf_prep_token(b - n_rt, x, D, norm_w, eps, xh, xsc, xn32, rmsv, pred, predm);
     return;
   }
-  pf_router_block<NK, RF32>(b % nrb, (b / nrb) % ntb, b / (nrb * ntb), w, wsh, x, norm_w, T, D, E, ldp, part, red);
+  pf_router_block<NK, RF32, FOLD>(b % nrb, (b / nrb) % ntb, b / (nrb * ntb), w, wsh, x, norm_w, T, D, E, ldp, part, red);
 }
 
 // One wave per token: logits = the token's RMSNorm factor x the sum of the
@@ -1369,8 +1377,9 @@ __global__ void __launch_bounds__(256) k_pfs_down_i8(const uint8_t* __restrict__
 
 // Steps 1-3: prep and router (xn32: also the fp32 rows xn, or NULL), top-k and
 // dispatch into segs (shared_T: tokens of the shared expert's own segments, or 0).
+// fold: see router_step.
 int pf_route(const gm_moe_layer* L, const float* x, int T, uint8_t* ws, const GmMoeWs& lay, const PfWs& w,
-             float* xn32, int shared_T, int32_t* segs, int seg_tok, hipStream_t s) {
+             float* xn32, int shared_T, int32_t* segs, int seg_tok, bool fold, hipStream_t s) {
   const int D = L->D, E = L->E, k = L->k;
   float* logits = reinterpret_cast<float*>(ws + lay.logits);
   float* shg = reinterpret_cast<float*>(ws + lay.shg);
@@ -1383,13 +1392,19 @@ int pf_route(const gm_moe_layer* L, const float* x, int T, uint8_t* ws, const Gm
     const int nrb = (nrows + 63) / 64, ntb = (T + 15) / 16, n_rt = nrb * ntb * nsplit;
     const dim3 g((unsigned)(n_rt + T));
     const bool f32 = L->q_router == GM_QTYPE_F32;
-#define GM_PR(NK, F32)                                                                                       \
-  hipLaunchKernelGGL((k_pf_prep_router<NK, F32>), g, dim3(256), 0, s, L->router, L->sh_gate_inp, x, L->norm_w, \
+#define GM_PR(NK, F32, FOLD)                                                                                     \
+  hipLaunchKernelGGL((k_pf_prep_router<NK, F32, FOLD>), g, dim3(256), 0, s, L->router, L->sh_gate_inp, x, L->norm_w, \
                      L->norm_eps, T, D, E, ldp, w.part, nrb, ntb, n_rt, w.xh, w.xsc, xn32, w.rmsv)
-    if (router_krange(D) == 512 && f32) GM_PR(4, true);
-    else if (router_krange(D) == 512) GM_PR(4, false);
-    else if (f32) GM_PR(2, true);
-    else GM_PR(2, false);
+#define GM_PR2(NK, F32)              \
+  do {                               \
+    if (fold) GM_PR(NK, F32, true);  \
+    else GM_PR(NK, F32, false);      \
+  } while (0)
+    if (router_krange(D) == 512 && f32) GM_PR2(4, true);
+    else if (router_krange(D) == 512) GM_PR2(4, false);
+    else if (f32) GM_PR2(2, true);
+    else GM_PR2(2, false);
+#undef GM_PR2
 #undef GM_PR
   }
   GM_TRY(hipGetLastError());
@@ -1432,7 +1447,7 @@ int prefill_t(const gm_moe_layer* L, const float* x, float* y, int T, int flags,
   const bool sh_f32 = sh_apart && !sh_i8;
   const size_t P = (size_t)T * k;
   const int seg = pf_seg(L, T), nseg = max_segments(T, k, E, seg);
-  if (int rc = pf_route(L, x, T, ws, lay, w, sh_f32 ? w.xn : nullptr, sh_gemm ? T : 0, w.segs, seg, s)) return rc;
+  if (int rc = pf_route(L, x, T, ws, lay, w, sh_f32 ? w.xn : nullptr, sh_gemm ? T : 0, w.segs, seg, false, s)) return rc;
   if (sh_f32) {                                      // shared expert rows yp[P + t], fp32
     if (int rc = gm_launch_gateup(L->q_gate_sh, L->gate_sh, L->up_sh, FF, D, w.xn, T, w.hsh, s)) return rc;
     if (int rc = gm_launch_matvec(L->q_down_sh, L->down_sh, D, FF, w.hsh, T, w.yp + P * D, s)) return rc;
@@ -1524,7 +1539,7 @@ int gm_pf8_run(const gm_moe_layer* L, const float* x, float* y, int T, int flags
   const Pf8Ws v = pf8_layout(L, T, w, ws + lay.pre8, nullptr);
   const bool has_sh = L->gate_sh != nullptr;
   const int nseg = max_segments(T, k, L->E, kPf8Seg);
-  if (int rc = pf_route(L, x, T, ws, lay, w, v.xn, has_sh ? T : 0, v.segs, kPf8Seg, s)) return rc;
+  if (int rc = pf_route(L, x, T, ws, lay, w, v.xn, has_sh ? T : 0, v.segs, kPf8Seg, true, s)) return rc;
   if (int rc = gm_pf8_split(v.xn, T, D, v.xr, s)) return rc;
   if (int rc = gm_pf8_gemm(L, false, v.xr, v.segs, nseg, w.offsets, w.sorted, T, v.h, s)) return rc;
   if (int rc = gm_pf8_split(v.h, T * k + (has_sh ? T : 0), FF, v.hr, s)) return rc;

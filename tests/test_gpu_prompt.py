@@ -434,6 +434,29 @@ def test_moe_i8_prompt_no_less_exact_than_steps(gpu, q_gate, q_down):
     assert err(y) <= 1.05 * err(steps)
 
 
+@pytest.mark.parametrize("D,f32", [(2048, True), (2048, False), (4096, True)])
+def test_moe_i8_prompt_logits_no_less_exact_than_steps(gpu, D, f32):
+    """The router's logits against 64 bits, beside the decode kernels' on the same tokens: norms
+    over 6,400 rounding errors, which chance moves by about a hundredth; the bar leaves five."""
+    from npu_amd import synth
+    from npu_amd.moe import GpuMoeBlock
+    from oracle import moe as OM
+    T, E = 100, 64
+    print(f"i8 logits case D={D} {f32}", flush=True)
+    h = synth.host_moe_layer(390, D=D, FF=256, E=E, k=4, q_gate=QT.Q8_0, q_down=QT.Q8_0, shared=False, router_f32=f32)
+    blk = GpuMoeBlock.from_host(h, device=gpu)
+    x = torch.randn(T, D, generator=torch.Generator().manual_seed(391))
+    ref = OM.router_logits64(x, OM.OracleLayer(h))
+
+    def logits(xp):
+        blk(xp.to(gpu))
+        return blk.stages(len(xp))["ffn_moe_logits"].double().cpu()
+    err = lambda a: float((a - ref).norm() / ref.norm())
+    one, steps = err(logits(x)), err(torch.cat([logits(xp) for xp in x.split(4)]))
+    print(f"{one:.3e} against {steps:.3e}", flush=True)
+    assert one <= 1.05 * steps
+
+
 def test_moe_i8_prompt_in_a_small_workspace(gpu):
     """A workspace too small for the planes of the I8 GEMMs still runs the tokens (as decode
     chunks): the static scratch of gm_moe_forward_noalloc, at a T that fits an IQ layer."""
