@@ -351,8 +351,8 @@ def _i8_block(gpu, D, FF, E, k, q_gate, q_down, shared, seed):
     return GpuMoeBlock.from_host(h, device=gpu)
 
 
-# the first T past the decode kernels (mostly one token an expert), segments of exactly 32, of
-# 33 and of 1 token (few experts), one row tile, odd counts of 128-wide steps, no shared expert
+# the first T past the decode kernels (mostly one token an expert), experts with two whole
+# segments and one token, or about two segments (few experts), one row tile, odd counts of 128-wide steps, no shared expert
 @pytest.mark.parametrize("D,FF,E,k,T,q_gate,q_down,shared", [
     (512, 256, 64, 8, 9, QT.Q6_K, QT.Q5_K, True),
     (256, 256, 2, 2, 33, QT.Q8_0, QT.Q6_K, True),
